@@ -26,7 +26,7 @@ if _PKG not in sys.path:
     sys.path.insert(0, _PKG)
 
 from cv3amd import ops, quant, synth  # noqa: E402
-from cv3amd.device import DeviceArray, to_device  # noqa: E402
+from cv3amd.device import to_device  # noqa: E402
 from cv3amd.weights import WeightStore  # noqa: E402
 
 STEPS = 10      # Euler steps of a solve
