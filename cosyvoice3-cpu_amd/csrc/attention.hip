@@ -34,6 +34,8 @@ struct AttnParams {
   float scale;
   int mask_kind;  // 0 none, 1 causal(a = offset), 2 chunk(a = size, b = left)
   int64_t mask_a, mask_b;
+  uint2* op;      // k_flash64x: the output's bfloat16 planes in fragment order instead of o, or null
+  int64_t opl;    // 8-byte halves per plane
 };
 
 // Every mask spec leaves query qi an interval of visible keys [lo, hi):
@@ -527,6 +529,24 @@ __global__ __launch_bounds__(512) void k_flash64x(AttnParams p, int nq) {
   float l_tot = l_run + __shfl_xor(l_run, 16, 64);
   l_tot += __shfl_xor(l_tot, 32, 64);
   if (!qvalid) return;
+  if (p.op) {
+    // row b n + qi of [batch n, 64 h] rows as the fragments a plane linear reads: four neighbouring
+    // columns are half of a lane's 16 bytes
+    const int64_t row = b * p.n + qi;
+#pragma unroll
+    for (int db = 0; db < 4; ++db) {
+      const int64_t col = hq * 64 + db * 16 + 4 * g;
+      const int64_t at = (((row >> 5) * (4 * p.h) + (col >> 4)) * 64 + (row & 31) + 32 * ((col >> 3) & 1)) * 2 +
+                         ((col >> 2) & 1);
+      uint2 hi, mid, lo;
+      split_x3(oacc[db][0] / l_tot, oacc[db][1] / l_tot, hi.x, mid.x, lo.x);
+      split_x3(oacc[db][2] / l_tot, oacc[db][3] / l_tot, hi.y, mid.y, lo.y);
+      p.op[at] = hi;
+      p.op[at + p.opl] = mid;
+      p.op[at + 2 * p.opl] = lo;
+    }
+    return;
+  }
   float* orow = p.o + b * p.o_sb + hq * p.o_sh + qi * p.o_sn;
 #pragma unroll
   for (int db = 0; db < 4; ++db)
@@ -595,7 +615,7 @@ __global__ __launch_bounds__(256) void k_attn_generic(AttnParams p) {
 static int attention(bool x3, const float* q, const float* k, const float* v, float* out, int64_t batch, int h,
                      int hk, int64_t n, int64_t m, int d, const int64_t* q_strides, const int64_t* k_strides,
                      const int64_t* v_strides, const int64_t* o_strides, float scale, int mask_kind, int64_t mask_a,
-                     int64_t mask_b, cv3_stream_t s) {
+                     int64_t mask_b, cv3_stream_t s, uint16_t* out_planes = nullptr) {
   CV3_REQUIRE(h > 0 && hk > 0, CV3_EINVAL, "head counts must be positive");
   CV3_REQUIRE(h % hk == 0, CV3_EINVAL, "%d query heads is not a multiple of %d kv heads", h, hk);
   CV3_REQUIRE(d > 0 && d <= 256, CV3_EUNSUPPORTED, "head dim %d not supported (max 256)", d);
@@ -611,7 +631,9 @@ static int attention(bool x3, const float* q, const float* k, const float* v, fl
   p.q_sb = q_strides[0]; p.q_sh = q_strides[1]; p.q_sn = q_strides[2];
   p.k_sb = k_strides[0]; p.k_sh = k_strides[1]; p.k_sm = k_strides[2];
   p.v_sb = v_strides[0]; p.v_sh = v_strides[1]; p.v_sm = v_strides[2];
-  p.o_sb = o_strides[0]; p.o_sh = o_strides[1]; p.o_sn = o_strides[2];
+  if (o_strides) p.o_sb = o_strides[0], p.o_sh = o_strides[1], p.o_sn = o_strides[2];
+  p.op = reinterpret_cast<uint2*>(out_planes);
+  p.opl = ceil_div(batch * n, 32) * (4 * h) * 128;
   p.h = h;
   p.hk = hk;
   p.n = n;
@@ -626,6 +648,8 @@ static int attention(bool x3, const float* q, const float* k, const float* v, fl
                          (p.q_sb % 4 == 0) && (p.q_sh % 4 == 0) && (p.q_sn % 4 == 0) && (p.k_sb % 4 == 0) &&
                          (p.k_sh % 4 == 0) && (p.k_sm % 4 == 0) && (p.v_sb % 4 == 0) && (p.v_sh % 4 == 0) &&
                          (p.v_sm % 4 == 0);
+  CV3_REQUIRE(!out_planes || (d == 64 && aligned16 && (uintptr_t)out_planes % 16 == 0), CV3_EUNSUPPORTED,
+              "attention into planes needs head dim 64 and 16-byte aligned rows");
   if (d == 64 && aligned16) {
     CV3_REQUIRE(m < (1ll << 31) - 4 * 64, CV3_EUNSUPPORTED, "attention over 2^31 keys or more");
     const int64_t nq = ceil_div(n, QT);
@@ -661,4 +685,14 @@ extern "C" int cv3_attention_x3(const float* q, const float* k, const float* v, 
   CV3_ALIVE();
   return attention(true, q, k, v, out, batch, h, hk, n, m, d, q_strides, k_strides, v_strides, o_strides, scale,
                    mask_kind, mask_a, mask_b, s);
+}
+
+extern "C" int cv3_attention_x3_planes(const float* q, const float* k, const float* v, uint16_t* out_planes,
+                                       int64_t batch, int h, int hk, int64_t n, int64_t m, int d,
+                                       const int64_t* q_strides, const int64_t* k_strides, const int64_t* v_strides,
+                                       float scale, int mask_kind, int64_t mask_a, int64_t mask_b, cv3_stream_t s) {
+  CV3_ALIVE();
+  CV3_REQUIRE(out_planes, CV3_EINVAL, "attention into planes needs its output");
+  return attention(true, q, k, v, nullptr, batch, h, hk, n, m, d, q_strides, k_strides, v_strides, nullptr, scale,
+                   mask_kind, mask_a, mask_b, s, out_planes);
 }

@@ -10,9 +10,10 @@ namespace cv3 {
 __device__ __forceinline__ float act_silu(float x) { return x / (1.0f + expf(-x)); }
 __device__ __forceinline__ float act_sigmoid(float x) { return 1.0f / (1.0f + expf(-x)); }
 __device__ __forceinline__ float act_gelu_tanh(float x) {
-  // 0.5 x (1 + tanh(sqrt(2/pi) (x + 0.044715 x^3)))   (ops.py:41-43)
+  // 0.5 x (1 + tanh(u)), u = sqrt(2/pi) (x + 0.044715 x^3)   (ops.py:41-43), as x / (1 + e^-2u):
+  // the same function with one exponential, and no cancellation where tanh is near -1
   const float c = 0.7978845608028654f;
-  return 0.5f * x * (1.0f + tanhf(c * (x + 0.044715f * x * x * x)));
+  return x / (1.0f + expf(-2.0f * (c * (x + 0.044715f * x * x * x))));
 }
 __device__ __forceinline__ float act_gelu(float x) {
   // 0.5 x (1 + erf(x / sqrt 2)) with the Abramowitz-Stegun 7.1.26 erf (ops.py:46-60)

@@ -1,0 +1,861 @@
+// Linears with both operands as bfloat16 planes in the matrix cores' fragment order.
+//
+// The float32 linear as six bfloat16 plane products (bf16x3.hpp) and the q8 linear as three
+// (a code is exact in bfloat16), y = epi(x . W^T + bias), with the activation split into its
+// planes once, by the kernel that produces it (a norm, the attention, the activation epilogue of
+// the linear before), instead of by every tile that reads it.  A plane fragment is one contiguous
+// kilobyte: frag[p][b][t][l] is the 16 bytes lane l feeds to v_mfma_f32_32x32x16_bf16 for the
+// 16-k step t of the 32-row block b (row 32 b + l % 32, k = 16 t + 8 (l / 32) .. + 7), for weights
+// and activations alike, so loads need no address arithmetic, no swizzle and no split.
+//
+// The weight is the matrix core's A operand and the activation its B: a lane's accumulator
+// registers 4 g .. 4 g + 3 are four neighbouring outputs n of one row m = 32 b + l % 32, so the
+// epilogue reads and writes float4, holds a rotary pair in one lane, and writes its result's own
+// planes in whole 512-byte runs.
+//
+// Two kernels, chosen per shape by plane_variant():
+//  * k_pg_reg: the K range split over the WK waves of a workgroup, each wave the whole RM x RN
+//    block tile, fragments straight from L2 into registers, no barrier in the loop, the partial
+//    sums met in LDS.  A small grid has WK times the waves and 1 / WK of the serial K steps.
+//  * k_pg_lds: the tile split over the waves, fragments through a ring of LDS stages (two 16-k
+//    steps each) filled by global -> LDS DMA, each loaded once per workgroup.  Fewer bytes from
+//    L2 per product, which bounds the large grids.
+// In both, the compiler sinks every load to the end of the MFMA block it may move past and then
+// waits for all of them at once; sched_group_barrier pins one load between every one or two MFMAs
+// (K = 2048 x [3000] rows: 73 -> 63 us, one 128 x 128 tile per 16-k step 1390 -> 900 cycles, 768
+// of them MFMAs).
+#include <algorithm>
+
+#include "bf16x3.hpp"
+#include "common.hpp"
+#include "epilogue.hpp"
+
+using namespace cv3;
+
+namespace {
+
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+struct PlaneParams {
+  const uint4* w;   // weight fragments [planes][nbw][S][64]
+  int64_t wpl;      // fragments (16 bytes) per weight plane
+  const uint4* x;   // activation fragments [3][nbx][S][64]
+  int64_t xpl;
+  int nbw, nbx, S;  // 32-row blocks of each operand, 16-k steps
+  const float* scales;  // q8: [blocks][32 nbw]
+  int m, n;
+  const float* bias;
+  float* c;         // float32 rows, or null
+  int64_t ldc;
+  uint2* yp;        // result planes in fragment order, or null
+  int64_t ypl;      // 8-byte halves per result plane
+  cv3_epilogue epi;
+  int tiles_m, tiles_n, gm;
+};
+
+enum { W_F32 = 0, W_Q8 = 1, W_Q8_BLOCK = 2 };  // three planes; codes, one scale a row; codes, one scale per 64
+constexpr int planes_of(int kind) { return kind == W_F32 ? 3 : 1; }
+
+// Tile of workgroup L: XCD L % 8 takes a contiguous run of tiles, walked gm row tiles high.
+__device__ __forceinline__ void plane_tile(const PlaneParams& p, int& tm, int& tn) {
+  const int T = gridDim.x, L = blockIdx.x, x = L & 7, q = T >> 3, r = T & 7;
+  const int t = x * q + min(x, r) + (L >> 3);
+  const int per = p.gm * p.tiles_n, g = t / per, o = t - g * per;
+  const int first = g * p.gm, gh = min(p.gm, p.tiles_m - first);
+  tm = first + o % gh;
+  tn = o / gh;
+}
+
+__device__ __forceinline__ f32x16 mfma(const uint4& a, const uint4& b, const f32x16& c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c,
+                                                 0, 0, 0);
+}
+
+__device__ __forceinline__ void dma16(const uint4* g, uint4* l) { __builtin_amdgcn_global_load_lds(g, l, 16, 0, 0); }
+
+// R times: N1 instructions of class M1, then N2 of class M2 (0x8 MFMA, 0x20 VMEM read, 0x100 LDS read).
+template <int M, int N>
+__device__ __forceinline__ void sched_n() {
+  if constexpr (N > 0) __builtin_amdgcn_sched_group_barrier(M, N, 0);
+}
+template <int M1, int N1, int M2, int N2, int R>
+__device__ __forceinline__ void interleave() {
+  if constexpr (R > 0) {
+    sched_n<M1, N1>();
+    sched_n<M2, N2>();
+    interleave<M1, N1, M2, N2, R - 1>();
+  }
+}
+
+// The products of one 16-k step: hh (of q8: hq) into `big`, the small ones into `small`, each
+// kind over all blocks before the next so no MFMA waits for the one before it.  FIRST starts both
+// sums at zero.
+template <int KIND, int RM, int RN, bool FIRST>
+__device__ __forceinline__ void mma_step(f32x16 (&big)[RM][RN], f32x16 (&small)[RM][RN], const uint4 (&x)[RM][3],
+                                         const uint4 (&w)[RN][planes_of(KIND)]) {
+  const f32x16 zero = {0.f};
+#define CV3_PRODUCT(ACC, PW, PX, ZERO)                                                   \
+  _Pragma("unroll") for (int i = 0; i < RM; ++i) _Pragma("unroll") for (int j = 0; j < RN; ++j) \
+      ACC[i][j] = mfma(w[j][PW], x[i][PX], (ZERO) ? zero : ACC[i][j]);
+  CV3_PRODUCT(big, 0, 0, FIRST)
+  if constexpr (KIND == W_F32) {
+    CV3_PRODUCT(small, 1, 0, FIRST)
+    CV3_PRODUCT(small, 0, 1, false)
+    CV3_PRODUCT(small, 2, 0, false)
+    CV3_PRODUCT(small, 1, 1, false)
+    CV3_PRODUCT(small, 0, 2, false)
+  } else {
+    CV3_PRODUCT(small, 0, 1, FIRST)
+    CV3_PRODUCT(small, 0, 2, false)
+  }
+#undef CV3_PRODUCT
+}
+
+// The scales of one 64-k block for this lane's outputs: register 4 g + e of block j is output
+// 32 (tn RN + j) + 8 g + 4 (lane / 32) + e.
+template <int RN>
+struct BlockScales {
+  float4 v[RN][4];
+};
+
+template <int RN>
+__device__ __forceinline__ void load_scales(BlockScales<RN>& s, const float* base, int64_t ld, int blk, const int (&nb)[RN],
+                                            int h) {
+#pragma unroll
+  for (int j = 0; j < RN; ++j)
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      s.v[j][g] = *reinterpret_cast<const float4*>(base + blk * ld + nb[j] * 32 + 8 * g + 4 * h);
+}
+
+template <int RM, int RN>
+__device__ __forceinline__ void fold_scales(f32x16 (&acc)[RM][RN], const f32x16 (&big)[RM][RN],
+                                            const f32x16 (&small)[RM][RN], const BlockScales<RN>& s) {
+#pragma unroll
+  for (int i = 0; i < RM; ++i)
+#pragma unroll
+    for (int j = 0; j < RN; ++j)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const float sc[4] = {s.v[j][g].x, s.v[j][g].y, s.v[j][g].z, s.v[j][g].w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          acc[i][j][4 * g + e] = fmaf(sc[e], big[i][j][4 * g + e] + small[i][j][4 * g + e], acc[i][j][4 * g + e]);
+      }
+}
+
+template <int ACT>
+__device__ __forceinline__ float act_of(float v) {
+  if constexpr (ACT == CV3_ACT_GELU_TANH) return act_gelu_tanh(v);
+  if constexpr (ACT == CV3_ACT_SILU) return act_silu(v);
+  return v;
+}
+
+// Epilogue of G groups of four neighbouring outputs: group q of this lane is v[q], outputs
+// n[q] .. n[q] + 3 of row m[q].  Every operand is loaded before the first store (C may be the
+// residual itself), in k_pg_reg before the waves meet.  Order of operations as store_tile's
+// (gemm.hip): bias, rotary, activation, gate, residual.  GATED kernels take a gate and a residual;
+// the others spend no registers on them (which leaves the q8 64 x 128 tiles two workgroups per CU).
+template <int ACT, int KIND, bool GATED, int G>
+struct PlaneEpilogue {
+  int m[G], n[G];
+  float4 scale[G], bias[G], gate[G], res[G];
+
+  __device__ __forceinline__ void load(const PlaneParams& p) {
+    const cv3_epilogue& e = p.epi;
+#pragma unroll
+    for (int q = 0; q < G; ++q) {
+      const int mm = min(m[q], p.m - 1), nn = min(n[q], p.n - 4);
+      if constexpr (KIND == W_Q8) scale[q] = *reinterpret_cast<const float4*>(p.scales + nn);
+      if (p.bias) bias[q] = *reinterpret_cast<const float4*>(p.bias + nn);
+      if constexpr (GATED) {
+        if (e.gate)
+          gate[q] = *reinterpret_cast<const float4*>(
+              e.gate + (int64_t)(e.rows_per_gate > 1 ? mm / (int)e.rows_per_gate : mm) * e.gate_stride + nn);
+        if (e.residual) res[q] = *reinterpret_cast<const float4*>(e.residual + (int64_t)mm * e.ld_res + nn);
+      }
+    }
+  }
+
+  // The rotary of one block's groups q0 .. q0 + NQ - 1 (dit.py:40-54): a pair is two of a lane's four
+  // outputs.  Few waves hold a rotated column; the others skip the table loads (a wave-uniform vote).
+  template <int NQ>
+  __device__ __forceinline__ void rotate(const PlaneParams& p, float4 (&v)[G], int q0) const {
+    const cv3_epilogue& e = p.epi;
+    bool rot[NQ], any = false;
+    uint32_t cp[NQ];
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+      cp[q] = (uint32_t)n[q0 + q] % (uint32_t)e.rope_period;
+      rot[q] = n[q0 + q] < e.rope_limit && cp[q] < (uint32_t)e.rope_width;
+      any |= rot[q];
+    }
+    if (!__any(any)) return;
+    float4 cs[NQ], sn[NQ];
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+      const uint32_t row = (uint32_t)min(m[q0 + q], p.m - 1) % (uint32_t)e.rope_rows;
+      const uint32_t ti = row * (uint32_t)e.rope_width + (rot[q] ? cp[q] : 0u);
+      cs[q] = *reinterpret_cast<const float4*>(e.rope_cos + ti);
+      sn[q] = *reinterpret_cast<const float4*>(e.rope_sin + ti);
+    }
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+      const float4 u = v[q0 + q];
+      if (rot[q])
+        v[q0 + q] = make_float4(u.x * cs[q].x + (-u.y) * sn[q].x, u.y * cs[q].y + u.x * sn[q].y,
+                                u.z * cs[q].z + (-u.w) * sn[q].z, u.w * cs[q].w + u.z * sn[q].w);
+    }
+  }
+
+  __device__ __forceinline__ void store(const PlaneParams& p, float4 (&v)[G]) const {
+    const cv3_epilogue& e = p.epi;
+#pragma unroll
+    for (int q = 0; q < G; ++q) {
+      if constexpr (KIND == W_Q8)
+        v[q] = make_float4(v[q].x * scale[q].x, v[q].y * scale[q].y, v[q].z * scale[q].z, v[q].w * scale[q].w);
+      if (p.bias) v[q] = make_float4(v[q].x + bias[q].x, v[q].y + bias[q].y, v[q].z + bias[q].z, v[q].w + bias[q].w);
+    }
+    if (e.rope_cos) {
+      constexpr int NQ = G < 4 ? G : 4;
+#pragma unroll
+      for (int q0 = 0; q0 < G; q0 += NQ) rotate<NQ>(p, v, q0);
+    }
+#pragma unroll
+    for (int q = 0; q < G; ++q) {
+      float o[4] = {act_of<ACT>(v[q].x), act_of<ACT>(v[q].y), act_of<ACT>(v[q].z), act_of<ACT>(v[q].w)};
+      if constexpr (GATED) {
+        if (e.gate) {
+          o[0] = gate[q].x * o[0];
+          o[1] = gate[q].y * o[1];
+          o[2] = gate[q].z * o[2];
+          o[3] = gate[q].w * o[3];
+        }
+        if (e.residual) {
+          o[0] = res[q].x + o[0];
+          o[1] = res[q].y + o[1];
+          o[2] = res[q].z + o[2];
+          o[3] = res[q].w + o[3];
+        }
+      }
+      if (m[q] >= p.m || n[q] >= p.n) continue;
+      if (p.c) *reinterpret_cast<float4*>(p.c + (int64_t)m[q] * p.ldc + n[q]) = make_float4(o[0], o[1], o[2], o[3]);
+      if (p.yp) {
+        uint2 hi, mid, lo;
+        split_x3(o[0], o[1], hi.x, mid.x, lo.x);
+        split_x3(o[2], o[3], hi.y, mid.y, lo.y);
+        // fragment of block m / 32, step n / 16; lane (m % 32) + 32 (n / 8 % 2); half n / 4 % 2
+        const int64_t at =
+            (((int64_t)(m[q] >> 5) * (p.n >> 4) + (n[q] >> 4)) * 64 + (m[q] & 31) + 32 * ((n[q] >> 3) & 1)) * 2 +
+            ((n[q] >> 2) & 1);
+        p.yp[at] = hi;
+        p.yp[at + p.ypl] = mid;
+        p.yp[at + 2 * p.ypl] = lo;
+      }
+    }
+  }
+};
+
+// ---- fragments straight into registers, K split over the workgroup's waves ----
+// PF register stages (PF - 1 steps in flight); a block-scaled weight's ranges are whole 64-k blocks.
+template <int KIND, int ACT, bool GATED, int RM, int RN, int WK, int PF>
+__global__ __launch_bounds__(64 * WK) void k_pg_reg(PlaneParams p) {
+  constexpr int NPW = planes_of(KIND), UNIT = KIND == W_Q8_BLOCK ? 4 : 1, LOADS = RM * 3 + RN * NPW;
+  static_assert(UNIT == 1 || PF % 4 == 0, "a turn of the register ring is whole blocks");
+  
+  __shared__ float4 red[WK][RM * RN * 4 * 64];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  int tm, tn;
+  plane_tile(p, tm, tn);
+  const int units = p.S / UNIT;
+  const int s0 = units * wave / WK * UNIT, s1 = units * (wave + 1) / WK * UNIT;
+  // blocks past the last read it again; their outputs are dropped
+  const uint4 *xp[RM], *wp[RN];
+  int nb[RN];
+#pragma unroll
+  for (int i = 0; i < RM; ++i) xp[i] = p.x + (int64_t)min(tm * RM + i, p.nbx - 1) * p.S * 64 + lane;
+#pragma unroll
+  for (int j = 0; j < RN; ++j) {
+    nb[j] = min(tn * RN + j, p.nbw - 1);
+    wp[j] = p.w + (int64_t)nb[j] * p.S * 64 + lane;
+  }
+  f32x16 big[RM][RN], small[RM][RN], acc[RM][RN];
+#pragma unroll
+  for (int i = 0; i < RM; ++i)
+#pragma unroll
+    for (int j = 0; j < RN; ++j) big[i][j] = small[i][j] = acc[i][j] = f32x16{0.f};
+  uint4 bx[PF][RM][3], bw[PF][RN][NPW];
+  auto load = [&](int buf, int s) {
+#pragma unroll
+    for (int pl = 0; pl < 3; ++pl) {
+      if (pl < NPW) {
+#pragma unroll
+        for (int j = 0; j < RN; ++j) bw[buf][j][pl] = wp[j][pl * p.wpl + (int64_t)s * 64];
+      }
+#pragma unroll
+      for (int i = 0; i < RM; ++i) bx[buf][i][pl] = xp[i][pl * p.xpl + (int64_t)s * 64];
+    }
+  };
+#pragma unroll
+  for (int j = 0; j < PF - 1; ++j) load(j, max(min(s0 + j, s1 - 1), 0));  // (an empty range loads step 0)
+  __builtin_amdgcn_sched_barrier(0);
+  constexpr int MF = RM * RN * (KIND == W_F32 ? 6 : 3), PER = MF / LOADS > 0 ? MF / LOADS : 1;
+  const int h = lane >> 5;
+  const int64_t lds = (int64_t)p.nbw * 32;
+  BlockScales<RN> sc;
+  // one step: its MFMAs with the loads of the step PF - 1 ahead between them (a uniform branch: the
+  // wave's last turn of the ring may be short)
+#define CV3_STEP(J, FIRST)                                                          \
+  if (s + (J) < s1) {                                                               \
+    load(((J) + PF - 1) % PF, min(s + (J) + PF - 1, s1 - 1));                       \
+    mma_step<KIND, RM, RN, FIRST>(big, small, bx[J], bw[J]);                        \
+    interleave<0x20, 1, 0x8, PER, LOADS>();                                         \
+    __builtin_amdgcn_sched_barrier(0);                                              \
+  }
+  if constexpr (KIND == W_Q8_BLOCK) {
+    for (int s = s0; s < s1; s += PF) {
+#pragma unroll
+      for (int c = 0; c < PF; c += 4) {
+        if (s + c >= s1) break;
+        load_scales<RN>(sc, p.scales, lds, (s + c) >> 2, nb, h);
+        CV3_STEP(c, true)
+        CV3_STEP(c + 1, false)
+        CV3_STEP(c + 2, false)
+        CV3_STEP(c + 3, false)
+        fold_scales<RM, RN>(acc, big, small, sc);
+      }
+    }
+  } else {
+    for (int s = s0; s < s1; s += PF) {
+#pragma unroll
+      for (int j = 0; j < PF; ++j) CV3_STEP(j, false)
+    }
+#pragma unroll
+    for (int i = 0; i < RM; ++i)
+#pragma unroll
+      for (int j = 0; j < RN; ++j) acc[i][j] = big[i][j] + small[i][j];
+  }
+#undef CV3_STEP
+  // the waves' partial sums meet in LDS, in wave order; each wave finishes its share of the groups
+  constexpr int GROUPS = RM * RN * 4, G = GROUPS > WK ? GROUPS / WK : 1;
+  PlaneEpilogue<ACT, KIND, GATED, G> ep;
+#pragma unroll
+  for (int q = 0; q < G; ++q) {
+    const int id = min(wave * G + q, GROUPS - 1), blk = id >> 2, g = id & 3;
+    ep.m[q] = (tm * RM + blk / RN) * 32 + (lane & 31);
+    ep.n[q] = (tn * RN + blk % RN) * 32 + 8 * g + 4 * h;
+  }
+  ep.load(p);
+#pragma unroll
+  for (int i = 0; i < RM; ++i)
+#pragma unroll
+    for (int j = 0; j < RN; ++j)
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        red[wave][((i * RN + j) * 4 + g) * 64 + lane] =
+            make_float4(acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]);
+  __syncthreads();
+  if (wave * G >= GROUPS) return;  // more waves than groups: the first ones finish
+  float4 v[G];
+#pragma unroll
+  for (int q = 0; q < G; ++q) {
+    const int id = wave * G + q;
+    v[q] = red[0][id * 64 + lane];
+#pragma unroll
+    for (int u = 1; u < WK; ++u) {
+      const float4 t = red[u][id * 64 + lane];
+      v[q] = make_float4(v[q].x + t.x, v[q].y + t.y, v[q].z + t.z, v[q].w + t.w);
+    }
+  }
+  ep.store(p, v);
+}
+
+// ---- fragments through a ring of LDS stages ----
+#define CV3_VM(n) (((n) & 0xF) | (((n) >> 4) << 14) | (0x7 << 4) | (0xF << 8))
+
+// WM x WN waves of RM x RN blocks.  Stage s (16-k steps 2 s, 2 s + 1) sits in ring slot s % NST.  Per stage:
+//   read the step's second fragments while the first's MFMAs run; wait until the next stage has
+//   landed and every wave has read this one (vmcnt counts this wave's DMAs, which land in order);
+//   refill this slot NST stages ahead and read the next stage's first fragments under the second
+//   step's MFMAs.
+template <int KIND, int ACT, bool GATED, int WM, int WN, int RM, int RN, int NST>
+__global__ __launch_bounds__(64 * WM * WN) void k_pg_lds(PlaneParams p) {
+  constexpr int NPW = planes_of(KIND), NW = WM * WN, TM = WM * RM, TN = WN * RN;
+  constexpr int F = (TM * 3 + TN * NPW) * 2, FP = (F + NW - 1) / NW;  // fragments per stage, per wave
+  __shared__ uint4 sh0[F * 64];
+  __shared__ uint4 sh1[F * 64];
+  __shared__ uint4 sh2[F * 64];
+  __shared__ uint4 sh3[NST == 4 ? F * 64 : 1];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  int tm, tn;
+  plane_tile(p, tm, tn);
+  const int wm = wave / WN, wn = wave % WN, h = lane >> 5;
+  // fragment f of a stage: f / 2 = (block, plane) of the activation's 3 TM, then the weight's, f % 2 = step
+  const char* src[FP];
+#pragma unroll
+  for (int f = 0; f < FP; ++f) {
+    const int id = min(wave * FP + f, F - 1), ks = id & 1, r = id >> 1;
+    const uint4* base;
+    if (r < 3 * TM)
+      base = p.x + (r % 3) * p.xpl + (int64_t)min(tm * TM + r / 3, p.nbx - 1) * p.S * 64;
+    else
+      base = p.w + ((r - 3 * TM) % NPW) * p.wpl + (int64_t)min(tn * TN + (r - 3 * TM) / NPW, p.nbw - 1) * p.S * 64;
+    src[f] = reinterpret_cast<const char*>(base + ks * 64);
+  }
+  const uint32_t loff = lane * 16;
+  auto dma = [&](uint4* sh, int st) {
+#pragma unroll
+    for (int f = 0; f < FP; ++f)
+      dma16(reinterpret_cast<const uint4*>(src[f] + (uint64_t)(uint32_t)st * 2048 + loff),
+            sh + min(wave * FP + f, F - 1) * 64);
+  };
+  auto read = [&](const uint4* sh, int ks, uint4 (&x)[RM][3], uint4 (&w)[RN][NPW]) {
+#pragma unroll
+    for (int pl = 0; pl < 3; ++pl) {
+      if (pl < NPW) {
+#pragma unroll
+        for (int j = 0; j < RN; ++j) w[j][pl] = sh[((3 * TM + (wn * RN + j) * NPW + pl) * 2 + ks) * 64 + lane];
+      }
+#pragma unroll
+      for (int i = 0; i < RM; ++i) x[i][pl] = sh[(((wm * RM + i) * 3 + pl) * 2 + ks) * 64 + lane];
+    }
+  };
+  int nb[RN];
+#pragma unroll
+  for (int j = 0; j < RN; ++j) nb[j] = min(tn * TN + wn * RN + j, p.nbw - 1);
+  f32x16 big[RM][RN], small[RM][RN], acc[RM][RN];
+#pragma unroll
+  for (int i = 0; i < RM; ++i)
+#pragma unroll
+    for (int j = 0; j < RN; ++j) big[i][j] = small[i][j] = acc[i][j] = f32x16{0.f};
+  uint4 x0[RM][3], w0[RN][NPW], x1[RM][3], w1[RN][NPW];
+  constexpr int NRD = RM * 3 + RN * NPW, NMF = RM * RN * (KIND == W_F32 ? 6 : 3);
+  constexpr int RDP = (NRD + NMF / 2 - 1) / (NMF / 2);  // LDS reads per MFMA so that they fill its first half
+  const int NS = p.S / 2;
+  const int64_t lds = (int64_t)p.nbw * 32;
+  BlockScales<RN> sc;
+  dma(sh0, 0);
+  dma(sh1, min(1, NS - 1));
+  dma(sh2, min(2, NS - 1));
+  if constexpr (NST == 4) dma(sh3, min(3, NS - 1));
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_s_waitcnt(CV3_VM((NST - 1) * FP));
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_sched_barrier(0);
+  read(sh0, 0, x0, w0);
+#define CV3_STAGE(CUR, NXT, ST, FIRST)                                                              \
+  {                                                                                                 \
+    read(CUR, 1, x1, w1);                                                                           \
+    mma_step<KIND, RM, RN, FIRST>(big, small, x0, w0);                                              \
+    interleave<0x8, 1, 0x100, RDP, NRD / RDP>();                                                    \
+    __builtin_amdgcn_sched_barrier(0);                                                              \
+    __builtin_amdgcn_s_waitcnt(CV3_VM((NST - 2) * FP) & ~(0xF << 8));                               \
+    __builtin_amdgcn_s_barrier();                                                                   \
+    __builtin_amdgcn_sched_barrier(0);                                                              \
+    read(NXT, 0, x0, w0);                                                                           \
+    dma(CUR, min((ST) + NST, NS - 1));                                                              \
+    mma_step<KIND, RM, RN, false>(big, small, x1, w1);                                              \
+    interleave<0x8, 1, 0x100, RDP, NRD / RDP>();                                                    \
+    interleave<0x20, 1, 0x8, 1, FP>();                                                              \
+    __builtin_amdgcn_sched_barrier(0);                                                              \
+  }
+  int s = 0;
+  if constexpr (KIND == W_Q8_BLOCK) {
+    // a 64-k block is two stages (K % 64 == 0: NS even)
+#define CV3_BLOCK(A, B, C, ST)                               \
+  load_scales<RN>(sc, p.scales, lds, (ST) >> 1, nb, h);      \
+  CV3_STAGE(A, B, ST, true)                                  \
+  CV3_STAGE(B, C, (ST) + 1, false)                           \
+  fold_scales<RM, RN>(acc, big, small, sc);
+    for (; s + 4 <= NS; s += 4) {
+      CV3_BLOCK(sh0, sh1, sh2, s)
+      CV3_BLOCK(sh2, sh3, sh0, s + 2)
+    }
+    if (s < NS) {
+      CV3_BLOCK(sh0, sh1, sh2, s)
+    }
+#undef CV3_BLOCK
+  } else if constexpr (NST == 4) {
+    for (; s + 4 <= NS; s += 4) {
+      CV3_STAGE(sh0, sh1, s, false)
+      CV3_STAGE(sh1, sh2, s + 1, false)
+      CV3_STAGE(sh2, sh3, s + 2, false)
+      CV3_STAGE(sh3, sh0, s + 3, false)
+    }
+    if (s < NS) {
+      CV3_STAGE(sh0, sh1, s, false)
+      if (s + 1 < NS) {
+        CV3_STAGE(sh1, sh2, s + 1, false)
+        if (s + 2 < NS) CV3_STAGE(sh2, sh3, s + 2, false)
+      }
+    }
+  } else {
+    for (; s + 3 <= NS; s += 3) {
+      CV3_STAGE(sh0, sh1, s, false)
+      CV3_STAGE(sh1, sh2, s + 1, false)
+      CV3_STAGE(sh2, sh0, s + 2, false)
+    }
+    if (s < NS) {
+      CV3_STAGE(sh0, sh1, s, false)
+      if (s + 1 < NS) CV3_STAGE(sh1, sh2, s + 1, false)
+    }
+  }
+#undef CV3_STAGE
+  __builtin_amdgcn_s_waitcnt(CV3_VM(0));  // no DMA outlives the workgroup's LDS
+  constexpr int G = RM * RN * 4;
+  PlaneEpilogue<ACT, KIND, GATED, G> ep;
+  float4 v[G];
+#pragma unroll
+  for (int i = 0; i < RM; ++i)
+#pragma unroll
+    for (int j = 0; j < RN; ++j) {
+      if constexpr (KIND != W_Q8_BLOCK) acc[i][j] = big[i][j] + small[i][j];
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const int q = (i * RN + j) * 4 + g;
+        v[q] = make_float4(acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]);
+        ep.m[q] = (tm * TM + wm * RM + i) * 32 + (lane & 31);
+        ep.n[q] = (tn * TN + wn * RN + j) * 32 + 8 * g + 4 * h;
+      }
+    }
+  ep.load(p);
+  ep.store(p, v);
+}
+
+// frag[nb][t][l] = the codes q[32 nb + l % 32][16 t + 8 (l / 32) .. + 7] as bfloat16 (exact; rows past n
+// zero), and scales transposed to float32 [blocks][32 nbw].
+__global__ __launch_bounds__(256) void k_pack_q8_planes(const int8_t* q, int64_t n, int64_t k, int64_t ldq, uint4* frag,
+                                                        int64_t total) {
+  const int64_t T = k / 16;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (int64_t)gridDim.x * blockDim.x) {
+    const int l = (int)(i & 63);
+    const int64_t t = (i >> 6) % T, row = (i >> 6) / T * 32 + (l & 31), k0 = 16 * t + 8 * (l >> 5);
+    const uint2 w = row < n ? *reinterpret_cast<const uint2*>(q + row * ldq + k0) : make_uint2(0u, 0u);
+    uint4 r;
+    uint32_t* o = &r.x;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const uint32_t word = j < 2 ? w.x : w.y;
+      const int sh = (j & 1) * 16;
+      const f32x2_t v = {(float)((int32_t)(word << (24 - sh)) >> 24), (float)((int32_t)(word << (16 - sh)) >> 24)};
+      o[j] = __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2_t));
+    }
+    frag[i] = r;
+  }
+}
+
+__global__ __launch_bounds__(256) void k_scales_t(const void* scales, int sf16, int64_t n, int64_t npad, int64_t nb,
+                                                  int64_t use, float* out) {
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < use * npad; i += (int64_t)gridDim.x * blockDim.x) {
+    const int64_t b = i / npad, r = i - b * npad;
+    out[i] = r >= n ? 0.f
+             : sf16 ? __half2float(reinterpret_cast<const __half*>(scales)[r * nb + b])
+                    : reinterpret_cast<const float*>(scales)[r * nb + b];
+  }
+}
+
+// The kernel and tile for a shape: a few rows take small tiles with K split over the waves (a lone
+// wave's serial steps are the time), many rows the tiles that load the fewest bytes per product.  A
+// variant's time on `tiles` tiles over S 16-k steps is modelled as
+//   k_pg_lds: f0 + rounds (f1 + S max(a, b u)), rounds of 256 `occ` workgroups, u = tiles per CU and round
+//   k_pg_reg: f0 + f1 u + S max(a, b u), u = the tiles of the busiest CU
+// (a: one workgroup's step, b: a step with every CU busy; us).  The constants are least-squares fits to
+// every variant timed at [40 .. 3000] rows x (N, K) = (3072, 1024), (2048, 1024), (1024, 1024),
+// (1024, 2048), weights from HBM, within 4-9 %; the pick is the fastest variant or on average 0.9 % behind
+// it.  E.g. float32, us: [40, 1024] x 1024: 10.3 (1 x 1) against 17.3 (2 x 2) and 31 (128 x 128);
+// [1000, 3072] x 1024: 36.9 (128 x 96) against 43.5 (2 x 2) and 66.7 (1 x 1).
+struct Variant {
+  int tm, tn;  // blocks of 32
+  int occ;     // k_pg_lds: workgroups per CU; k_pg_reg: 0
+  float f0, f1, a, b;
+};
+enum { V_R11, V_R12, V_R22, V_L12, V_L22, V_L13, V_COUNT };
+constexpr Variant kVariants[3][V_COUNT] = {
+    // float32 weights
+    {{1, 1, 0, 3.89f, 1.06f, 0.087f, 0.065f}, {1, 2, 0, 3.05f, 2.05f, 0.117f, 0.095f},
+     {2, 2, 0, 1.12f, 4.72f, 0.156f, 0.146f}, {2, 4, 1, 3.98f, 6.19f, 0.248f, 0.297f},
+     {4, 4, 1, 0.86f, 8.31f, 0.397f, 0.650f}, {4, 3, 1, 0.97f, 11.73f, 0.321f, 0.362f}},
+    // q8 weights, one scale a row
+    {{1, 1, 0, 2.79f, 1.07f, 0.008f, 0.037f}, {1, 2, 0, 1.45f, 2.63f, 0.050f, 0.051f},
+     {2, 2, 0, 1.28f, 3.56f, 0.091f, 0.091f}, {2, 4, 2, 7.27f, 0.00f, 0.115f, 0.193f},
+     {4, 4, 1, 3.16f, 7.28f, 0.206f, 0.338f}, {4, 3, 1, 1.56f, 5.84f, 0.212f, 0.247f}},
+    // q8 weights, one scale per 64 codes
+    {{1, 1, 0, 2.15f, 1.70f, 0.040f, 0.043f}, {1, 2, 0, 1.58f, 2.65f, 0.058f, 0.062f},
+     {2, 2, 0, 1.89f, 2.63f, 0.103f, 0.135f}, {2, 4, 2, 10.54f, 0.00f, 0.216f, 0.241f},
+     {4, 4, 1, 5.85f, 0.00f, 0.503f, 0.571f}, {4, 3, 1, 5.93f, 0.00f, 0.424f, 0.445f}},
+};
+
+int plane_variant(int kind, int nbm, int nbn, int S) {
+  int best = V_R11;
+  float bt = 1e30f;
+  for (int i = 0; i < V_COUNT; ++i) {
+    const Variant& v = kVariants[kind][i];
+    const int64_t tiles = ceil_div(nbm, v.tm) * ceil_div(nbn, v.tn);
+    const int64_t rounds = v.occ ? ceil_div(tiles, 256 * v.occ) : 1;
+    const float u = v.occ ? (float)tiles / (256.f * (float)rounds) : (float)ceil_div(tiles, 256);
+    const float step = (float)S * std::max(v.a, v.b * u);
+    const float t = v.f0 + (v.occ ? (float)rounds * (v.f1 + step) : u * v.f1 + step);
+    if (t < bt) {
+      bt = t;
+      best = i;
+    }
+  }
+  return best;
+}
+
+template <int KIND, int ACT, bool GATED>
+void launch(int variant, const PlaneParams& p, hipStream_t st) {
+  const dim3 grid((unsigned)(p.tiles_m * p.tiles_n));
+  // the waves a tile's K is split over and the register ring, as measured per weight kind: float32
+  // steps hold three planes of both operands, so fewer fit
+  constexpr bool F = KIND == W_F32, B = KIND == W_Q8_BLOCK;
+  constexpr int NST = F ? 3 : 4;
+#define CV3_REG(RM, RN, WK, PF) \
+  hipLaunchKernelGGL((k_pg_reg<KIND, ACT, GATED, RM, RN, WK, PF>), grid, dim3(64 * (WK)), 0, st, p)
+#define CV3_LDS(WM, WN, RM, RN) \
+  hipLaunchKernelGGL((k_pg_lds<KIND, ACT, GATED, WM, WN, RM, RN, NST>), grid, dim3(64 * (WM) * (WN)), 0, st, p)
+  switch (variant) {
+    case V_R11: CV3_REG(1, 1, (F ? 4 : 8), 4); break;
+    case V_R12: CV3_REG(1, 2, (F ? 4 : 8), (F ? 3 : 4)); break;
+    case V_R22: CV3_REG(2, 2, (B ? 4 : 8), (F ? 2 : B ? 4 : 3)); break;
+    case V_L12: CV3_LDS(2, 2, 1, 2); break;
+    case V_L22: CV3_LDS((F ? 4 : 2), 2, (F ? 1 : 2), 2); break;
+    default: CV3_LDS(4, 1, 1, 3); break;
+  }
+#undef CV3_REG
+#undef CV3_LDS
+}
+
+template <int KIND>
+int launch_act(int variant, const PlaneParams& p, hipStream_t st) {
+  const bool gated = p.epi.gate || p.epi.residual;
+  switch (p.epi.act) {
+    case CV3_ACT_NONE:
+      gated ? launch<KIND, CV3_ACT_NONE, true>(variant, p, st) : launch<KIND, CV3_ACT_NONE, false>(variant, p, st);
+      return CV3_OK;
+    case CV3_ACT_GELU_TANH:
+      gated ? launch<KIND, CV3_ACT_GELU_TANH, true>(variant, p, st)
+            : launch<KIND, CV3_ACT_GELU_TANH, false>(variant, p, st);
+      return CV3_OK;
+    case CV3_ACT_SILU: launch<KIND, CV3_ACT_SILU, true>(variant, p, st); return CV3_OK;
+    default: return fail(CV3_EUNSUPPORTED, "plane linear: activation %d has no epilogue here", p.epi.act);
+  }
+}
+
+int plane_linear(int kind, const uint16_t* x, int64_t m, int64_t k, const uint16_t* w, const float* scales, int64_t n,
+                 const float* bias, float* y, int64_t ldy, uint16_t* y_planes, const cv3_epilogue* epi,
+                 int64_t plan_rows, hipStream_t st) {
+  CV3_REQUIRE(k % 64 == 0 && k >= (kind == W_Q8_BLOCK ? 256 : 128) && n % 4 == 0 && (!y_planes || n % 16 == 0),
+              CV3_EUNSUPPORTED, "plane linear needs K %% 64 == 0, K >= 128 (block scales: 256), N %% 4 == 0 (K = %lld, N = %lld)",
+              (long long)k, (long long)n);
+  auto a16 = [](const void* q) { return (uintptr_t)q % 16 == 0; };
+  PlaneParams p{};
+  p.epi = epi ? *epi : cv3_epilogue{};
+  const cv3_epilogue& e = p.epi;
+  CV3_REQUIRE(a16(x) && a16(w) && a16(scales) && a16(bias) && a16(y) && a16(y_planes) && ldy % 4 == 0 && a16(e.residual) &&
+                  e.ld_res % 4 == 0 && a16(e.gate) && e.gate_stride % 4 == 0 && a16(e.rope_cos) && a16(e.rope_sin),
+              CV3_EINVAL, "plane linear operands must be 16-byte aligned rows");
+  CV3_REQUIRE(!e.rope_cos || (e.rope_sin && e.rope_rows > 0 && e.rope_period > 0 && e.rope_period % 4 == 0 &&
+                              e.rope_width % 4 == 0 && e.rope_rows * e.rope_width < (1ll << 31)),
+              CV3_EINVAL, "plane linear: rotary widths must be multiples of four, the table within 32 bits");
+  CV3_REQUIRE(m < (1ll << 30) && plan_rows < (1ll << 30) && n < (1ll << 30) && k < (1ll << 30) && e.rows_per_gate < (1ll << 31), CV3_EINVAL,
+              "plane linear too large");
+  p.S = (int)(k / 16);
+  p.nbw = (int)ceil_div(n, 32);
+  p.nbx = (int)ceil_div(m, 32);
+  p.w = reinterpret_cast<const uint4*>(w);
+  p.wpl = (int64_t)p.nbw * p.S * 64;
+  p.x = reinterpret_cast<const uint4*>(x);
+  p.xpl = (int64_t)p.nbx * p.S * 64;
+  p.scales = scales;
+  p.m = (int)m;
+  p.n = (int)n;
+  p.bias = bias;
+  p.c = y;
+  p.ldc = ldy;
+  p.yp = reinterpret_cast<uint2*>(y_planes);
+  p.ypl = (int64_t)p.nbx * (n / 16) * 128;
+  const int v = plane_variant(kind, (int)ceil_div(plan_rows > 0 ? plan_rows : m, 32), p.nbw, p.S);
+  const Variant& t = kVariants[kind][v];
+  p.tiles_m = (int)ceil_div(p.nbx, t.tm);
+  p.tiles_n = (int)ceil_div(p.nbw, t.tn);
+  CV3_REQUIRE((int64_t)p.tiles_m * p.tiles_n < (1ll << 31), CV3_EINVAL, "plane linear too large");
+  // an XCD's run of tiles as near to the fewest bytes of both operands as whole rows of tiles allow
+  const double per = (double)p.tiles_m * p.tiles_n / 8, wb = (kind == W_F32 ? 3.0 : 1.0) * t.tn, xb = 3.0 * t.tm;
+  int gm = 1;
+  while (gm < p.tiles_m && (double)gm * gm * xb < per * wb) ++gm;
+  p.gm = gm;
+  const int rc = kind == W_F32  ? launch_act<W_F32>(v, p, st)
+                 : kind == W_Q8 ? launch_act<W_Q8>(v, p, st)
+                                : launch_act<W_Q8_BLOCK>(v, p, st);
+  if (rc) return rc;
+  CV3_LAUNCHED();
+  return CV3_OK;
+}
+
+// One wave per row of at most 1024 columns (a multiple of 16): lane l holds the 8-column chunks l and
+// l + 64, which are its fragments' 16 bytes.  RMS: y = (x * 1 / sqrt(mean x^2 + eps)) * w; else
+// LayerNorm with the AdaLN shift and scale rows (elementwise.hip has both as float32 kernels, with
+// the same operations in the same order).
+__device__ __forceinline__ float lane_sum(float v) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  return v;
+}
+
+template <bool RMS>
+__global__ __launch_bounds__(256) void k_norm_planes(const float* __restrict__ x, uint4* __restrict__ out, int64_t rows,
+                                                     int cols, float eps, const float* __restrict__ w,
+                                                     const float* __restrict__ shift, const float* __restrict__ scale,
+                                                     int64_t opl) {
+  const int lane = threadIdx.x & 63;
+  const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (row >= rows) return;
+  const int chunks = cols / 8;
+  const float* xr = x + row * cols;
+  float v[2][8], a[2][8], b[2][8];
+  auto load8 = [](const float* s, float (&d)[8]) {
+    const float4 lo = *reinterpret_cast<const float4*>(s), hi = *reinterpret_cast<const float4*>(s + 4);
+    d[0] = lo.x; d[1] = lo.y; d[2] = lo.z; d[3] = lo.w;
+    d[4] = hi.x; d[5] = hi.y; d[6] = hi.z; d[7] = hi.w;
+  };
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int c = min(lane + 64 * i, chunks - 1) * 8;
+    load8(xr + c, v[i]);
+    if constexpr (RMS) {
+      load8(w + c, a[i]);
+    } else {
+      load8(scale + c, a[i]);
+      load8(shift + c, b[i]);
+    }
+  }
+  float s = 0.f;
+  float mu = 0.f;
+  if constexpr (!RMS) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      if (lane + 64 * i < chunks) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) s += v[i][e];
+      }
+    mu = lane_sum(s) / (float)cols;
+  }
+  float q = 0.f;
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+    if (lane + 64 * i < chunks) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float d = v[i][e] - mu;
+        q = fmaf(d, d, q);
+      }
+    }
+  const float den = sqrtf(lane_sum(q) / (float)cols + eps);
+  const float inv = 1.0f / den;
+  const int S = cols / 16;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int c = lane + 64 * i;
+    if (c >= chunks) continue;
+    float o[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      o[e] = RMS ? (v[i][e] * inv) * a[i][e] : (v[i][e] - mu) / den * (1.0f + a[i][e]) + b[i][e];
+    uint4 hi, mid, lo;
+    split_x3(make_float4(o[0], o[1], o[2], o[3]), make_float4(o[4], o[5], o[6], o[7]), hi, mid, lo);
+    const int64_t at = ((row >> 5) * S + (c >> 1)) * 64 + (row & 31) + 32 * (c & 1);
+    out[at] = hi;
+    out[at + opl] = mid;
+    out[at + 2 * opl] = lo;
+  }
+}
+
+int norm_planes(bool rms, const float* x, uint16_t* planes, int64_t rows, int64_t cols, float eps, const float* w,
+                const float* shift, const float* scale, hipStream_t st) {
+  auto a16 = [](const void* q) { return (uintptr_t)q % 16 == 0; };
+  CV3_REQUIRE(cols % 16 == 0 && cols >= 16 && cols <= 1024, CV3_EUNSUPPORTED,
+              "a norm into planes takes 16 .. 1024 columns, a multiple of 16 (cols = %lld)", (long long)cols);
+  CV3_REQUIRE(a16(x) && a16(planes) && a16(w) && a16(shift) && a16(scale), CV3_EINVAL,
+              "a norm into planes needs 16-byte aligned operands");
+  if (rows <= 0) return CV3_OK;
+  const dim3 grid((unsigned)ceil_div(rows, 4));
+  const int64_t opl = ceil_div(rows, 32) * (cols / 16) * 64;
+  if (rms)
+    hipLaunchKernelGGL(k_norm_planes<true>, grid, dim3(256), 0, st, x, reinterpret_cast<uint4*>(planes), rows, (int)cols,
+                       eps, w, shift, scale, opl);
+  else
+    hipLaunchKernelGGL(k_norm_planes<false>, grid, dim3(256), 0, st, x, reinterpret_cast<uint4*>(planes), rows,
+                       (int)cols, eps, w, shift, scale, opl);
+  CV3_LAUNCHED();
+  return CV3_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
+int cv3_linear_x3_planes(const uint16_t* x, int64_t m, int64_t k, const uint16_t* frag, int64_t n, const float* bias,
+                         float* y, int64_t ldy, uint16_t* y_planes, const cv3_epilogue* epi, int64_t plan_rows,
+                         cv3_stream_t s) {
+  CV3_ALIVE();
+  CV3_REQUIRE(m >= 0 && k > 0 && n >= 0 && (!y || ldy >= n) && (y || y_planes), CV3_EINVAL,
+              "bad plane linear shape m=%lld k=%lld n=%lld", (long long)m, (long long)k, (long long)n);
+  if (!m || !n) return CV3_OK;
+  return plane_linear(W_F32, x, m, k, frag, nullptr, n, bias, y, ldy, y_planes, epi, plan_rows, stream_of(s));
+}
+
+int cv3_q8_planes_elems(int64_t n, int64_t k, int64_t block, int64_t* codes, int64_t* scales) {
+  CV3_REQUIRE(n >= 0 && k > 0 && block > 0 && codes && scales, CV3_EINVAL, "bad shape or null output");
+  const int64_t npad = ceil_div(n, 32) * 32;
+  *codes = npad * k;
+  *scales = npad * (block >= k ? 1 : ceil_div(k, block));
+  return CV3_OK;
+}
+
+int cv3_pack_q8_planes(const int8_t* q, int64_t n, int64_t k, int64_t ldq, const void* scales, int scale_dtype,
+                       int64_t kp, int64_t block, uint16_t* frag, float* scales_t, cv3_stream_t s) {
+  CV3_ALIVE();
+  CV3_REQUIRE(n >= 0 && k > 0 && k % 64 == 0 && ldq >= k && ldq % 8 == 0 && block > 0 && kp >= k && kp % block == 0,
+              CV3_EINVAL, "bad code pack shape n=%lld k=%lld block=%lld", (long long)n, (long long)k, (long long)block);
+  CV3_REQUIRE(block == 64 || block >= k, CV3_EUNSUPPORTED, "plane codes take 64-code blocks or one scale a row");
+  CV3_REQUIRE((uintptr_t)q % 8 == 0 && (uintptr_t)frag % 16 == 0 && (uintptr_t)scales_t % 16 == 0, CV3_EINVAL,
+              "plane codes need aligned rows");
+  const int64_t npad = ceil_div(n, 32) * 32, total = npad * k / 8, use = block >= k ? 1 : k / block;
+  if (!total) return CV3_OK;
+  hipStream_t st = stream_of(s);
+  hipLaunchKernelGGL(k_pack_q8_planes, dim3((unsigned)(ceil_div(total, 256) < 65536 ? ceil_div(total, 256) : 65536)),
+                     dim3(256), 0, st, q, n, k, ldq, reinterpret_cast<uint4*>(frag), total);
+  hipLaunchKernelGGL(k_scales_t, dim3((unsigned)ceil_div(use * npad, 256)), dim3(256), 0, st, scales,
+                     scale_dtype == CV3_F16 ? 1 : 0, n, npad, kp / block, use, scales_t);
+  CV3_LAUNCHED();
+  return CV3_OK;
+}
+
+int cv3_linear_q8_planes(const uint16_t* x, int64_t m, int64_t k, const uint16_t* frag, const float* scales_t,
+                         int64_t block, int64_t n, const float* bias, float* y, int64_t ldy, uint16_t* y_planes,
+                         const cv3_epilogue* epi, int64_t plan_rows, cv3_stream_t s) {
+  CV3_ALIVE();
+  CV3_REQUIRE(m >= 0 && k > 0 && n >= 0 && (!y || ldy >= n) && (y || y_planes) && scales_t, CV3_EINVAL,
+              "bad plane linear shape m=%lld k=%lld n=%lld", (long long)m, (long long)k, (long long)n);
+  CV3_REQUIRE(block == 64 || block >= k, CV3_EUNSUPPORTED, "plane codes take 64-code blocks or one scale a row");
+  if (!m || !n) return CV3_OK;
+  return plane_linear(block >= k ? W_Q8 : W_Q8_BLOCK, x, m, k, frag, scales_t, n, bias, y, ldy, y_planes, epi,
+                      plan_rows, stream_of(s));
+}
+
+int cv3_layer_norm_planes(const float* x, uint16_t* planes, int64_t rows, int64_t cols, float eps, const float* shift,
+                          const float* scale, cv3_stream_t s) {
+  CV3_ALIVE();
+  CV3_REQUIRE(shift && scale, CV3_EINVAL, "a layer norm into planes needs its shift and scale rows");
+  return norm_planes(false, x, planes, rows, cols, eps, nullptr, shift, scale, stream_of(s));
+}
+
+int cv3_rms_norm_planes(const float* x, const float* w, uint16_t* planes, int64_t rows, int64_t cols, float eps,
+                        cv3_stream_t s) {
+  CV3_ALIVE();
+  CV3_REQUIRE(w, CV3_EINVAL, "an RMS norm needs its weight");
+  return norm_planes(true, x, planes, rows, cols, eps, w, nullptr, nullptr, stream_of(s));
+}
+
+}  // extern "C"

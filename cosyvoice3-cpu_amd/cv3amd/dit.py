@@ -86,12 +86,18 @@ class DeviceLinear:
     K <= 2048) it runs on the int8 matrix cores instead, the activation's rows as four int8 digit
     planes (``cv3_linear_q8_digits``, exact products of the codes with each row rounded 30 bits
     below its largest element), given ``rexp``, an int32 workspace of at least m entries.
+
+    ``frag_x=True`` also readies the weight for activations that come as bfloat16 planes in fragment
+    order (``from_planes``, cv3_linear_x3_planes / cv3_linear_q8_planes), where ``takes_planes`` says
+    it can: float32 planes as they are, q8 codes (64-code blocks or one scale a row) widened to
+    bfloat16 beside the packed codes.
     """
 
     def __init__(self, weights: List[object], biases: List[Optional[np.ndarray]], planes: bool = False,
-                 digits: bool = False):
+                 digits: bool = False, frag_x: bool = False):
         ws = list(weights)
         self.planes = None
+        self.codes16: Optional[DeviceArray] = None
         self.rexp: Optional[DeviceArray] = None
         if all(_is_q(w) for w in ws):
             kinds = {w.kind for w in ws}
@@ -117,6 +123,13 @@ class DeviceLinear:
             # per-channel codes on the int8 matrix cores (cv3_pack_q8_frag32, cv3_linear_q8_digits)
             self.q8_digits = (self.q8_planes and digits and DIGITS and self.kp == self.block
                               and self.k <= 2048)
+            if frag_x and self.q8_planes and not self.q8_digits and (self.block == 64 or self.block >= self.k):
+                nc, ns = ctypes.c_int64(), ctypes.c_int64()
+                _lib.call("q8_planes_elems", self.n, self.k, self.block, ctypes.byref(nc), ctypes.byref(ns))
+                self.codes16, self.scales_t = DeviceArray((nc.value,), np.uint16), DeviceArray((ns.value,))
+                _lib.call("pack_q8_planes", self.q.ptr, self.n, self.k, self.kp, self.scales.ptr,
+                          _lib.F16 if self.sf16 else _lib.F32, self.kp, self.block, self.codes16.ptr,
+                          self.scales_t.ptr, None)
             if self.q8_digits:
                 npad = -(-self.n // 32) * 32
                 qf = DeviceArray((npad * (self.k + 4),), np.int8)
@@ -149,11 +162,30 @@ class DeviceLinear:
             self.bias = to_device(np.concatenate(parts))
         else:
             self.bias = None
+        # cv3_linear_*_planes: K a multiple of 64 from 128 (64-code blocks: 256), N of 4
+        held = self.planes is not None if not self.q8 else self.codes16 is not None
+        self.takes_planes = (bool(frag_x) and held and self.n % 4 == 0
+                             and self.k >= (256 if self.q8 and self.block < self.k else 128))
+
+    def from_planes(self, x: int, m: int, y=None, ldy: int = 0, y_planes=None, epi=None, st=None,
+                    plan_rows: int = 0):
+        """y[m, n] = epi(x . W^T + bias) with x [m, k] as bfloat16 planes in fragment order (a pointer);
+        the result goes to float32 rows ``y``, to its own planes ``y_planes``, or both.  ``plan_rows``:
+        the rows of the batch that this call is a part of (0: m)."""
+        b = self.bias.ptr if self.bias is not None else None
+        e = ctypes.byref(epi) if epi is not None else None
+        if self.q8:
+            _lib.call("linear_q8_planes", x, m, self.k, self.codes16.ptr, self.scales_t.ptr, self.block, self.n, b, y,
+                      ldy, y_planes, e, plan_rows, st)
+        else:
+            _lib.call("linear_x3_planes", x, m, self.k, self.planes.ptr, self.n, b, y, ldy, y_planes, e,
+                      plan_rows, st)
 
     @property
     def nbytes(self) -> int:
         if self.q8:
-            return self.q.nbytes + self.scales.nbytes
+            wide = self.codes16.nbytes + self.scales_t.nbytes if self.codes16 is not None else 0
+            return self.q.nbytes + self.scales.nbytes + wide
         return self.planes.nbytes if self.planes is not None else self.w.nbytes
 
     def __call__(self, x: int, m: int, ldx: int, y: int, ldy: int, epi=None, rexp_given: bool = False,
@@ -273,13 +305,24 @@ class DeviceDiT:
         for i in range(self.depth):
             b = f"transformer_blocks.{i}."
             self.qkv.append(DeviceLinear([g(b + f"attn.to_{p}.weight") for p in "qkv"],
-                                         [g(b + f"attn.to_{p}.bias") for p in "qkv"], planes, digits=True))
-            self.out.append(DeviceLinear([g(b + "attn.to_out.0.weight")], [g(b + "attn.to_out.0.bias")], planes))
+                                         [g(b + f"attn.to_{p}.bias") for p in "qkv"], planes, digits=True,
+                                         frag_x=planes))
+            self.out.append(DeviceLinear([g(b + "attn.to_out.0.weight")], [g(b + "attn.to_out.0.bias")], planes,
+                                         frag_x=planes))
             self.ff1.append(DeviceLinear([g(b + "ff.ff.0.0.weight")], [g(b + "ff.ff.0.0.bias")], planes,
-                                         digits=True))
-            self.ff2.append(DeviceLinear([g(b + "ff.ff.2.weight")], [g(b + "ff.ff.2.bias")], planes))
+                                         digits=True, frag_x=planes))
+            self.ff2.append(DeviceLinear([g(b + "ff.ff.2.weight")], [g(b + "ff.ff.2.bias")], planes, frag_x=planes))
         self.ff_dim = self.ff1[0].n if self.depth else 2 * D
-        self.proj_out = DeviceLinear([g("proj_out.weight")], [g("proj_out.bias")], planes)
+        self.proj_out = DeviceLinear([g("proj_out.weight")], [g("proj_out.bias")], planes, frag_x=planes)
+        # a norm or attention output is split into planes once, by its producer, when every linear that
+        # reads it takes planes (the digit-plane linears read float32 rows)
+        norms = D % 64 == 0 and D <= 1024
+        self.qkv_frag = norms and all(lin.takes_planes for lin in self.qkv)
+        self.ff1_frag = norms and all(lin.takes_planes for lin in self.ff1)
+        self.out_frag = (self.planes and self.dim_head == 64 and self.heads * self.dim_head == D
+                         and all(lin.takes_planes for lin in self.out))
+        self.ff2_frag = self.ff1_frag and self.ff_dim % 16 == 0 and all(lin.takes_planes for lin in self.ff2)
+        self.proj_out_frag = norms and self.proj_out.takes_planes
         self._T = None
         self._graph = None
         self.halves = False                  # set by prepare() from HALVES and T
@@ -308,6 +351,10 @@ class DeviceDiT:
             self.qkvb = DeviceArray((B * T, 3 * D))
             self.att = DeviceArray((B * T, D))
             self.ffb = DeviceArray((B * T, self.ff_dim))
+            # the same as planes in fragment order, for all rows and for one batch row of its own
+            # (fragments hold 32 rows, so a batch row cannot start inside one)
+            self.np, self.attp, self.ffp = ([self._planes(r, k) for r in (B * T, T)]
+                                            for k in (D, D, self.ff_dim))
             self.z1 = DeviceArray((B * T, D))
             self.outb = DeviceArray((B * T, mel))
             self.outT = DeviceArray((B, mel, T))
@@ -327,6 +374,12 @@ class DeviceDiT:
         self.stemb = DeviceArray((S, D))
         self.mods = DeviceArray((S, self.ld_mod))
         self._graph = None
+
+    @staticmethod
+    def _planes(rows: int, k: int) -> DeviceArray:
+        ne = ctypes.c_int64()
+        _lib.call("x3_frag_elems", rows, k, ctypes.byref(ne))
+        return DeviceArray((ne.value,), np.uint16)
 
     # -- one estimator evaluation + Euler update ---------------------------
     def _time_and_mod(self):
@@ -361,18 +414,41 @@ class DeviceDiT:
         scale = float(np.float32(1.0 / math.sqrt(dh)))
         base = mrow + i * 6 * D * f4
         sh_a, sc_a, g_a, sh_m, sc_m, g_m = (base + j * D * f4 for j in range(6))
-        self._norm(sh_a, sc_a, self.qkv[i].q8_digits, r0, rows, st)
+        slot = 1 if r0 else 0
+        plan = dict(st=st, plan_rows=2 * T)
+        np_, attp, ffp = self.np[slot].ptr, self.attp[slot].ptr, self.ffp[slot].ptr
         # partial rotary on q and k, channels 0..dh-1 (dit.py:119-120), in the GEMM epilogue
         rope_epi = _lib.epilogue(rope=(self.cos.ptr, self.sin.ptr, T, D, dh, 2 * D))
-        self.qkv[i](n, rows, D, qkvb, 3 * D, rope_epi, rexp_given=True, st=st, rexp_row0=r0)
-        _lib.call("attention_x3" if self.planes else "attention", qkvb, qkvb + D * f4, qkvb + 2 * D * f4, att,
-                  nb, H, H, T, T, dh, qs, qs, qs, os_, scale, 0, 0, 0, st)
-        self.out[i](att, rows, D, h, D,
-                    _lib.epilogue(residual=h, ld_res=D, gate=g_a, gate_stride=0, rows_per_gate=1), st=st)
-        self._norm(sh_m, sc_m, self.ff1[i].q8_digits, r0, rows, st)
-        self.ff1[i](n, rows, D, ffb, self.ff_dim, _lib.epilogue("gelu_tanh"), rexp_given=True, st=st, rexp_row0=r0)
-        self.ff2[i](ffb, rows, self.ff_dim, h, D,
-                    _lib.epilogue(residual=h, ld_res=D, gate=g_m, gate_stride=0, rows_per_gate=1), st=st)
+        if self.qkv_frag:
+            _lib.call("layer_norm_planes", h, np_, rows, D, 1e-6, sh_a, sc_a, st)
+            self.qkv[i].from_planes(np_, rows, qkvb, 3 * D, epi=rope_epi, **plan)
+        else:
+            self._norm(sh_a, sc_a, self.qkv[i].q8_digits, r0, rows, st)
+            self.qkv[i](n, rows, D, qkvb, 3 * D, rope_epi, rexp_given=True, st=st, rexp_row0=r0)
+        gate_a = _lib.epilogue(residual=h, ld_res=D, gate=g_a, gate_stride=0, rows_per_gate=1)
+        if self.out_frag:
+            _lib.call("attention_x3_planes", qkvb, qkvb + D * f4, qkvb + 2 * D * f4, attp, nb, H, H, T, T, dh, qs, qs,
+                      qs, scale, 0, 0, 0, st)
+            self.out[i].from_planes(attp, rows, h, D, epi=gate_a, **plan)
+        else:
+            _lib.call("attention_x3" if self.planes else "attention", qkvb, qkvb + D * f4, qkvb + 2 * D * f4, att,
+                      nb, H, H, T, T, dh, qs, qs, qs, os_, scale, 0, 0, 0, st)
+            self.out[i](att, rows, D, h, D, gate_a, st=st)
+        gelu = _lib.epilogue("gelu_tanh")
+        gate_m = _lib.epilogue(residual=h, ld_res=D, gate=g_m, gate_stride=0, rows_per_gate=1)
+        if self.ff1_frag:
+            _lib.call("layer_norm_planes", h, np_, rows, D, 1e-6, sh_m, sc_m, st)
+        else:
+            self._norm(sh_m, sc_m, self.ff1[i].q8_digits, r0, rows, st)
+        if self.ff2_frag:
+            self.ff1[i].from_planes(np_, rows, y_planes=ffp, epi=gelu, **plan)
+            self.ff2[i].from_planes(ffp, rows, h, D, epi=gate_m, **plan)
+            return
+        if self.ff1_frag:
+            self.ff1[i].from_planes(np_, rows, ffb, self.ff_dim, epi=gelu, **plan)
+        else:
+            self.ff1[i](n, rows, D, ffb, self.ff_dim, gelu, rexp_given=True, st=st, rexp_row0=r0)
+        self.ff2[i](ffb, rows, self.ff_dim, h, D, gate_m, st=st)
 
     def _step(self, s: int, dt: float, update: bool = True):
         T, D, B, mel, H, dh = self._T, self.dim, 2, self.mel, self.heads, self.dim_head
@@ -409,8 +485,12 @@ class DeviceDiT:
             for i in range(self.depth):
                 self._block(i, mrow, 0, B, None)
         base = mrow + self.depth * 6 * D * f4      # norm_out: (scale, shift) (dit.py:175-178)
-        _lib.call("layer_norm", self.h.ptr, self.n.ptr, BT, D, 1e-6, None, None, base + D * f4, base, 0, 0, None)
-        self.proj_out(self.n.ptr, BT, D, self.outb.ptr, mel)
+        if self.proj_out_frag:
+            _lib.call("layer_norm_planes", self.h.ptr, self.np[0].ptr, BT, D, 1e-6, base + D * f4, base, None)
+            self.proj_out.from_planes(self.np[0].ptr, BT, self.outb.ptr, mel)
+        else:
+            _lib.call("layer_norm", self.h.ptr, self.n.ptr, BT, D, 1e-6, None, None, base + D * f4, base, 0, 0, None)
+            self.proj_out(self.n.ptr, BT, D, self.outb.ptr, mel)
         # (B, T, 80) -> (B, 80, T), then x += dt ((1 + w) d0 - w d1)  (dit.py:180, flow.py:86-87)
         _lib.call("copy_strided", self.outb.ptr, self.outT.ptr, B, T, mel, S3(T * mel, mel, 1),
                   S3(mel * T, 1, T), None)

@@ -182,6 +182,30 @@ int cv3_linear_q8_digits(const float* x, int64_t m, int64_t k, int64_t ldx, cons
                          int scale_dtype, int64_t n, const float* bias, float* y, int64_t ldy, const cv3_epilogue* epi,
                          int32_t* row_exp, int row_exp_given,
                          cv3_stream_t s);
+/* The same linears with the activation, too, as bfloat16 planes in fragment order: x is what
+ * cv3_split_x3_frag writes for [m, k] rows (cv3_x3_frag_elems(m, k) uint16), made by the kernel before
+ * (cv3_layer_norm_planes, cv3_rms_norm_planes, cv3_attention_x3_planes, or y_planes of the linear before).
+ * The result goes to float32 rows (y), to its own planes (y_planes, cv3_x3_frag_elems(m, n); n % 16), or
+ * both.  q8 codes are held as bfloat16 (exact) in fragment order, the scales transposed to float32
+ * [blocks][ceil(n / 32) * 32]: 64-code blocks, or one scale a row (block >= k).  K % 64 == 0, K >= 128
+ * (64-code blocks: 256), n % 4 == 0, 16-byte aligned operands; activations none, GELU (tanh), SiLU.
+ * plan_rows (0: m): the rows that the tile, and with it the order of the sums, is chosen for; parts of one
+ * batch launched side by side pass the batch's, fill the machine as its tiles do and return its bits. */
+int cv3_linear_x3_planes(const uint16_t* x, int64_t m, int64_t k, const uint16_t* frag, int64_t n, const float* bias,
+                         float* y, int64_t ldy, uint16_t* y_planes, const cv3_epilogue* epi, int64_t plan_rows,
+                         cv3_stream_t s);
+int cv3_q8_planes_elems(int64_t n, int64_t k, int64_t block, int64_t* codes, int64_t* scales);
+int cv3_pack_q8_planes(const int8_t* q, int64_t n, int64_t k, int64_t ldq, const void* scales, int scale_dtype,
+                       int64_t kp, int64_t block, uint16_t* frag, float* scales_t, cv3_stream_t s);
+int cv3_linear_q8_planes(const uint16_t* x, int64_t m, int64_t k, const uint16_t* frag, const float* scales_t,
+                         int64_t block, int64_t n, const float* bias, float* y, int64_t ldy, uint16_t* y_planes,
+                         const cv3_epilogue* epi, int64_t plan_rows, cv3_stream_t s);
+/* AdaLN (dit.py:168-169) and RMSNorm (ops.py:101-104) whose result is [rows, cols] planes in fragment
+ * order; cols a multiple of 16, at most 1024, 16-byte aligned operands. */
+int cv3_layer_norm_planes(const float* x, uint16_t* planes, int64_t rows, int64_t cols, float eps, const float* shift,
+                          const float* scale, cv3_stream_t s);
+int cv3_rms_norm_planes(const float* x, const float* w, uint16_t* planes, int64_t rows, int64_t cols, float eps,
+                        cv3_stream_t s);
 /* Quantised weights (q8: q [n, kp] int8; q4: q [n, kp/2]); scales [n, kp/block] (f16 or f32). */
 int cv3_linear_q(int kind, const float* x, int64_t m, int64_t k, int64_t ldx, const void* q, const void* scales,
                  int scale_dtype, int64_t kp, int64_t block, int64_t n, const float* bias, float* y, int64_t ldy,
@@ -252,6 +276,12 @@ int cv3_attention_x3(const float* q, const float* k, const float* v, float* out,
                      int64_t n, int64_t m, int d, const int64_t* q_strides, const int64_t* k_strides,
                      const int64_t* v_strides, const int64_t* o_strides, float scale, int mask_kind,
                      int64_t mask_a, int64_t mask_b, cv3_stream_t s);
+/* cv3_attention_x3 with the output [batch * n, 64 h] as bfloat16 planes in fragment order, for the plane
+ * linear that reads it (d == 64, 16-byte aligned rows). */
+int cv3_attention_x3_planes(const float* q, const float* k, const float* v, uint16_t* out_planes, int64_t batch, int h,
+                            int hk, int64_t n, int64_t m, int d, const int64_t* q_strides, const int64_t* k_strides,
+                            const int64_t* v_strides, float scale, int mask_kind, int64_t mask_a, int64_t mask_b,
+                            cv3_stream_t s);
 
 /* ---------------- convolution (ops.conv1d ops.py:165-219, ops.depthwise_conv1d ops.py:222-237) ---------------- */
 /* x (cin, t_in) with strides (x_cs, x_ts), optionally nearest-upsampled by `up` before padding;

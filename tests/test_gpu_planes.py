@@ -1,0 +1,164 @@
+"""Linears, norms and attention on activations held as bfloat16 planes in fragment order.
+
+The planes of a float32 value are the rounding chain test_gpu_x3.py pins bit for bit, and reproduce it to
+2^-24; so every result is compared with float64 (or the oracle) at the bar of the other float32 kernels,
+max |error| / max |reference| <= 1e-5.  Shapes sit at the edges of the 32-row fragments, of each kernel's
+tile (32 x 32 up to 128 x 128) and of its K ranges, and reach every variant the shape rule picks.
+"""
+
+import ctypes
+
+import numpy as np
+import pytest
+
+from conftest import rel_err
+import oracle.ops as ref
+import oracle.quant as rquant
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-5
+
+
+@pytest.fixture(scope="module")
+def lib(gpu):
+    from cv3amd import _lib
+    from cv3amd.device import to_device, empty
+    return _lib, to_device, empty
+
+
+def elems(lib, m, k):
+    ne = ctypes.c_int64()
+    lib[0].call("x3_frag_elems", m, k, ctypes.byref(ne))
+    return ne.value
+
+
+def to_planes(lib, a):
+    _lib, to_device, empty = lib
+    m, k = a.shape
+    out = empty((elems(lib, m, k),), np.uint16)
+    d = to_device(np.ascontiguousarray(a, np.float32))
+    _lib.call("split_x3_frag", d.ptr, m, k, k, out.ptr, None)
+    return out
+
+
+def from_planes(p, m, k):
+    """The float32 rows of a plane buffer (hi + mid + lo, exact in float64)."""
+    mb = -(-m // 32)
+    with np.errstate(invalid="ignore"):    # rows past m are whatever the memory held
+        f = (p.numpy().astype(np.uint32) << 16).view(np.float32).astype(np.float64)
+    f = f.reshape(3, mb, k // 16, 2, 32, 8)                   # plane, block, step, lane half, row, k
+    return f.sum(0).transpose(0, 3, 1, 2, 4).reshape(mb * 32, k)[:m]
+
+
+def ptr(d):
+    return d.ptr if d is not None else None
+
+
+# (rows, K, N): one row, fragment and tile edges, few rows to many, every variant of the shape rule
+SHAPES = [(1, 128, 32), (31, 256, 68), (33, 1024, 96), (65, 320, 1024), (97, 1024, 3072), (302, 2048, 1024),
+          (500, 1024, 1024), (700, 1024, 3072), (1001, 1024, 2048), (1500, 1024, 1028), (2100, 1024, 3072)]
+KINDS = ["f32", "q8_rows", "q8_block"]
+
+
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("m,k,n", SHAPES)
+def test_linear_from_planes(lib, m, k, n, kind):
+    _lib, to_device, empty = lib
+    if kind == "q8_block" and k < 256:
+        pytest.skip("64-code blocks need K >= 256")
+    rng = np.random.default_rng([m, k, n])
+    x = rng.normal(size=(m, k)).astype(np.float32)
+    w = (0.02 * rng.normal(size=(n, k))).astype(np.float32)
+    b = rng.normal(size=n).astype(np.float32)
+    xp, bd = to_planes(lib, x), to_device(b)
+    if kind == "f32":
+        wd, w64 = to_planes(lib, w), w.astype(np.float64)
+        run = lambda *a: _lib.call("linear_x3_planes", xp.ptr, m, k, wd.ptr, n, *a)  # noqa: E731
+    else:
+        block = 64 if kind == "q8_block" else k
+        sdt = np.float16 if kind == "q8_block" else np.float32
+        q, s, kp = rquant.quantize_q8(w, block, sdt)
+        w64 = (q.astype(np.float64).reshape(n, -1, block) * s.astype(np.float64)[:, :, None]).reshape(n, -1)[:, :k]
+        qd, sd = to_device(np.ascontiguousarray(q)), to_device(np.ascontiguousarray(s))
+        nc, ns = ctypes.c_int64(), ctypes.c_int64()
+        _lib.call("q8_planes_elems", n, k, block, ctypes.byref(nc), ctypes.byref(ns))
+        wd, st = empty((nc.value,), np.uint16), empty((ns.value,))
+        _lib.call("pack_q8_planes", qd.ptr, n, k, kp, sd.ptr, _lib.F16 if sdt == np.float16 else _lib.F32, kp, block,
+                  wd.ptr, st.ptr, None)
+        run = lambda *a: _lib.call("linear_q8_planes", xp.ptr, m, k, wd.ptr, st.ptr, block, n, *a)  # noqa: E731
+    want = x.astype(np.float64) @ w64.T + b
+    y = empty((m, n))
+    run(bd.ptr, y.ptr, n, None, None, 0, None)
+    assert rel_err(y.numpy(), want) < TOL
+    if n % 16:
+        return
+    # the gated residual, in place, and an activation straight into planes
+    h, gate = rng.normal(size=(m, n)).astype(np.float32), rng.normal(size=n).astype(np.float32)
+    hd, gd = to_device(h), to_device(gate)
+    epi = _lib.epilogue(residual=hd.ptr, ld_res=n, gate=gd.ptr, gate_stride=0, rows_per_gate=1)
+    run(bd.ptr, hd.ptr, n, None, ctypes.byref(epi), 0, None)
+    assert rel_err(hd.numpy(), h + gate * want) < TOL
+    yp = empty((elems(lib, m, n),), np.uint16)
+    run(bd.ptr, None, 0, yp.ptr, ctypes.byref(_lib.epilogue("gelu_tanh")), 0, None)
+    assert rel_err(from_planes(yp, m, n), ref.gelu_tanh(want)) < TOL
+
+
+@pytest.mark.parametrize("rows_per_batch,m", [(151, 302), (29, 58), (400, 400)])
+def test_rotary_from_planes(lib, rows_per_batch, m):
+    """The DiT's partial rotary on q and k (columns 0..63 of each 256 here), as the plane linear without it
+    followed by the rotary kernel."""
+    _lib, to_device, empty = lib
+    from cv3amd.dit import dit_rope_tables
+    rng = np.random.default_rng(m)
+    k = D = 256
+    xp, wd = (to_planes(lib, rng.normal(size=(r, k)).astype(np.float32)) for r in (m, 3 * D))
+    c, s = (to_device(a) for a in dit_rope_tables(rows_per_batch, 64))
+    y, z = empty((m, 3 * D)), empty((m, 3 * D))
+    epi = _lib.epilogue(rope=(c.ptr, s.ptr, rows_per_batch, D, 64, 2 * D))
+    _lib.call("linear_x3_planes", xp.ptr, m, k, wd.ptr, 3 * D, None, y.ptr, 3 * D, None, ctypes.byref(epi), 0, None)
+    _lib.call("linear_x3_planes", xp.ptr, m, k, wd.ptr, 3 * D, None, z.ptr, 3 * D, None, None, 0, None)
+    for col in (0, D):
+        _lib.call("rope_pairs", z.ptr + 4 * col, 3 * D, m, rows_per_batch, 64, c.ptr, s.ptr, None)
+    assert rel_err(y.numpy(), z.numpy()) < 1e-6   # the same products; two roundings and a fused multiply-add apart
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 16), (33, 896), (5, 1008), (100, 1024), (64, 528)])
+def test_norms_into_planes(lib, rows, cols):
+    _lib, to_device, empty = lib
+    rng = np.random.default_rng(cols)
+    x = (3 + 5 * rng.normal(size=(rows, cols))).astype(np.float32)
+    sh, sc = (rng.normal(size=cols).astype(np.float32) for _ in range(2))
+    xd, shd, scd = to_device(x), to_device(sh), to_device(sc)
+    p = empty((elems(lib, rows, cols),), np.uint16)
+    _lib.call("layer_norm_planes", xd.ptr, p.ptr, rows, cols, 1e-6, shd.ptr, scd.ptr, None)
+    assert rel_err(from_planes(p, rows, cols), ref.layer_norm(x, None, None, 1e-6) * (1 + sc) + sh) < TOL
+    _lib.call("rms_norm_planes", xd.ptr, scd.ptr, p.ptr, rows, cols, 1e-6, None)
+    assert rel_err(from_planes(p, rows, cols), ref.rms_norm(x, sc, 1e-6)) < TOL
+
+
+@pytest.mark.parametrize("batch,n", [(2, 37), (1, 64), (2, 151)])
+def test_attention_into_planes(lib, batch, n):
+    """Bit for bit the planes of what cv3_attention_x3 writes as float32."""
+    _lib, to_device, empty = lib
+    h, d = 3, 64
+    rng = np.random.default_rng(n)
+    qkv = to_device(rng.normal(size=(batch * n, 3 * h * d)).astype(np.float32))
+    S3 = ctypes.c_int64 * 3
+    st, os_ = S3(n * 3 * h * d, d, 3 * h * d), S3(n * h * d, d, h * d)
+    args = (qkv.ptr, qkv.ptr + 4 * h * d, qkv.ptr + 8 * h * d)
+    y, p = empty((batch * n, h * d)), empty((elems(lib, batch * n, h * d),), np.uint16)
+    _lib.call("attention_x3", *args, y.ptr, batch, h, h, n, n, d, st, st, st, os_, 0.125, 0, 0, 0, None)
+    _lib.call("attention_x3_planes", *args, p.ptr, batch, h, h, n, n, d, st, st, st, 0.125, 0, 0, 0, None)
+    got, want = from_planes(p, batch * n, h * d), y.numpy().astype(np.float64)
+    assert np.all(np.abs(got - want) <= 2.0 ** -24 * np.abs(want))
+
+
+def test_plane_linear_refuses_what_it_cannot_read(lib):
+    _lib, to_device, empty = lib
+    a = empty((4096,))
+    for m, k, n in ((4, 96, 32), (4, 64, 32), (4, 128, 30)):
+        with pytest.raises(NotImplementedError):
+            _lib.call("linear_x3_planes", a.ptr, m, k, a.ptr, n, None, a.ptr, n, None, None, 0, None)
+    with pytest.raises(ValueError):
+        _lib.call("linear_x3_planes", a.ptr + 4, 4, 128, a.ptr, 32, None, a.ptr, 32, None, None, 0, None)
