@@ -50,11 +50,23 @@ struct PlaneParams {
   uint2* yp;        // result planes in fragment order, or null
   int64_t ypl;      // 8-byte halves per result plane
   cv3_epilogue epi;
+  // A_QKV: c holds q rows; the caches are at this layer's row pos0 of head 0
+  float *kc, *vc;
+  int heads, kv_heads, cap, pos0;
+  const float *cos, *sin;  // [cap][64]
   int tiles_m, tiles_n, gm;
 };
 
-enum { W_F32 = 0, W_Q8 = 1, W_Q8_BLOCK = 2 };  // three planes; codes, one scale a row; codes, one scale per 64
+// weights as three planes; as codes with one scale a row, per 64 codes, per 32 codes
+enum { W_F32 = 0, W_ROW = 1, W_B64 = 2, W_B32 = 3 };
 constexpr int planes_of(int kind) { return kind == W_F32 ? 3 : 1; }
+constexpr int fold_steps(int kind) { return kind == W_B64 ? 4 : kind == W_B32 ? 2 : 0; }  // 16-k steps per scale
+
+// Epilogues beyond the activations of cv3_epilogue, for the LM's prompt:
+//  A_SWIGLU  outputs 2 j, 2 j + 1 are gate j and up j (the weight's rows interleaved): silu(g) u, N / 2 wide
+//  A_QKV     bias, half-split rotary on q and k (each head's rows interleaved so that dims j and j + 32 are
+//            outputs 2 j, 2 j + 1 of the head), q to rows, k and v to their cache rows
+enum { A_SWIGLU = 100, A_QKV = 101 };
 
 // Tile of workgroup L: XCD L % 8 takes a contiguous run of tiles, walked gm row tiles high.
 __device__ __forceinline__ void plane_tile(const PlaneParams& p, int& tm, int& tn) {
@@ -147,7 +159,6 @@ __device__ __forceinline__ void fold_scales(f32x16 (&acc)[RM][RN], const f32x16 
 template <int ACT>
 __device__ __forceinline__ float act_of(float v) {
   if constexpr (ACT == CV3_ACT_GELU_TANH) return act_gelu_tanh(v);
-  if constexpr (ACT == CV3_ACT_SILU) return act_silu(v);
   return v;
 }
 
@@ -166,7 +177,7 @@ struct PlaneEpilogue {
 #pragma unroll
     for (int q = 0; q < G; ++q) {
       const int mm = min(m[q], p.m - 1), nn = min(n[q], p.n - 4);
-      if constexpr (KIND == W_Q8) scale[q] = *reinterpret_cast<const float4*>(p.scales + nn);
+      if constexpr (KIND == W_ROW) scale[q] = *reinterpret_cast<const float4*>(p.scales + nn);
       if (p.bias) bias[q] = *reinterpret_cast<const float4*>(p.bias + nn);
       if constexpr (GATED) {
         if (e.gate)
@@ -208,14 +219,56 @@ struct PlaneEpilogue {
     }
   }
 
+  __device__ __forceinline__ void store_swiglu(const PlaneParams& p, const float4 (&v)[G]) const {
+    uint32_t* y = reinterpret_cast<uint32_t*>(p.yp);
+#pragma unroll
+    for (int q = 0; q < G; ++q) {
+      if (m[q] >= p.m || n[q] >= p.n) continue;
+      uint32_t hi, mid, lo;
+      split_x3(v[q].y * act_silu(v[q].x), v[q].w * act_silu(v[q].z), hi, mid, lo);
+      const int c = n[q] >> 1;  // outputs c, c + 1: a quarter of a lane's 16 bytes
+      const int64_t at =
+          (((int64_t)(m[q] >> 5) * (p.n >> 5) + (c >> 4)) * 64 + (m[q] & 31) + 32 * ((c >> 3) & 1)) * 4 + ((c >> 1) & 3);
+      y[at] = hi;
+      y[at + 2 * p.ypl] = mid;
+      y[at + 4 * p.ypl] = lo;
+    }
+  }
+
+  // qwen2.py:64-71,155-168
+  __device__ __forceinline__ void store_qkv(const PlaneParams& p, const float4 (&v)[G]) const {
+    float2 cs[G], sn[G];
+#pragma unroll
+    for (int q = 0; q < G; ++q) {
+      const int64_t t = (int64_t)(p.pos0 + min(m[q], p.m - 1)) * 64 + ((n[q] & 63) >> 1);
+      cs[q] = *reinterpret_cast<const float2*>(p.cos + t);
+      sn[q] = *reinterpret_cast<const float2*>(p.sin + t);
+    }
+#pragma unroll
+    for (int q = 0; q < G; ++q) {
+      if (m[q] >= p.m || n[q] >= p.n) continue;
+      const int head = n[q] >> 6, r = n[q] & 63, kv = head - p.heads;
+      if (kv >= p.kv_heads) {
+        *reinterpret_cast<float4*>(p.vc + ((int64_t)(kv - p.kv_heads) * p.cap + m[q]) * 64 + r) = v[q];
+        continue;
+      }
+      float* row = kv < 0 ? p.c + (int64_t)m[q] * p.ldc + head * 64 : p.kc + ((int64_t)kv * p.cap + m[q]) * 64;
+      const float4 u = v[q];
+      *reinterpret_cast<float2*>(row + (r >> 1)) = make_float2(u.x * cs[q].x + (-u.y) * sn[q].x, u.z * cs[q].y + (-u.w) * sn[q].y);
+      *reinterpret_cast<float2*>(row + (r >> 1) + 32) = make_float2(u.y * cs[q].x + u.x * sn[q].x, u.w * cs[q].y + u.z * sn[q].y);
+    }
+  }
+
   __device__ __forceinline__ void store(const PlaneParams& p, float4 (&v)[G]) const {
     const cv3_epilogue& e = p.epi;
 #pragma unroll
     for (int q = 0; q < G; ++q) {
-      if constexpr (KIND == W_Q8)
+      if constexpr (KIND == W_ROW)
         v[q] = make_float4(v[q].x * scale[q].x, v[q].y * scale[q].y, v[q].z * scale[q].z, v[q].w * scale[q].w);
       if (p.bias) v[q] = make_float4(v[q].x + bias[q].x, v[q].y + bias[q].y, v[q].z + bias[q].z, v[q].w + bias[q].w);
     }
+    if constexpr (ACT == A_QKV) return store_qkv(p, v);
+    if constexpr (ACT == A_SWIGLU) return store_swiglu(p, v);
     if (e.rope_cos) {
       constexpr int NQ = G < 4 ? G : 4;
 #pragma unroll
@@ -260,7 +313,7 @@ struct PlaneEpilogue {
 // PF register stages (PF - 1 steps in flight); a block-scaled weight's ranges are whole 64-k blocks.
 template <int KIND, int ACT, bool GATED, int RM, int RN, int WK, int PF>
 __global__ __launch_bounds__(64 * WK) void k_pg_reg(PlaneParams p) {
-  constexpr int NPW = planes_of(KIND), UNIT = KIND == W_Q8_BLOCK ? 4 : 1, LOADS = RM * 3 + RN * NPW;
+  constexpr int NPW = planes_of(KIND), FOLD = fold_steps(KIND), UNIT = FOLD ? FOLD : 1, LOADS = RM * 3 + RN * NPW;
   static_assert(UNIT == 1 || PF % 4 == 0, "a turn of the register ring is whole blocks");
   
   __shared__ float4 red[WK][RM * RN * 4 * 64];
@@ -312,16 +365,18 @@ __global__ __launch_bounds__(64 * WK) void k_pg_reg(PlaneParams p) {
     interleave<0x20, 1, 0x8, PER, LOADS>();                                         \
     __builtin_amdgcn_sched_barrier(0);                                              \
   }
-  if constexpr (KIND == W_Q8_BLOCK) {
+  if constexpr (FOLD > 0) {
     for (int s = s0; s < s1; s += PF) {
 #pragma unroll
-      for (int c = 0; c < PF; c += 4) {
+      for (int c = 0; c < PF; c += FOLD) {
         if (s + c >= s1) break;
-        load_scales<RN>(sc, p.scales, lds, (s + c) >> 2, nb, h);
+        load_scales<RN>(sc, p.scales, lds, (s + c) / FOLD, nb, h);
         CV3_STEP(c, true)
         CV3_STEP(c + 1, false)
-        CV3_STEP(c + 2, false)
-        CV3_STEP(c + 3, false)
+        if constexpr (FOLD == 4) {
+          CV3_STEP(c + 2, false)
+          CV3_STEP(c + 3, false)
+        }
         fold_scales<RM, RN>(acc, big, small, sc);
       }
     }
@@ -460,7 +515,7 @@ __global__ __launch_bounds__(64 * WM * WN) void k_pg_lds(PlaneParams p) {
     __builtin_amdgcn_sched_barrier(0);                                                              \
   }
   int s = 0;
-  if constexpr (KIND == W_Q8_BLOCK) {
+  if constexpr (KIND == W_B64) {
     // a 64-k block is two stages (K % 64 == 0: NS even)
 #define CV3_BLOCK(A, B, C, ST)                               \
   load_scales<RN>(sc, p.scales, lds, (ST) >> 1, nb, h);      \
@@ -473,6 +528,23 @@ __global__ __launch_bounds__(64 * WM * WN) void k_pg_lds(PlaneParams p) {
     }
     if (s < NS) {
       CV3_BLOCK(sh0, sh1, sh2, s)
+    }
+#undef CV3_BLOCK
+  } else if constexpr (KIND == W_B32) {
+    // a 32-k block is one stage
+#define CV3_BLOCK(A, B, ST)                          \
+  load_scales<RN>(sc, p.scales, lds, ST, nb, h);     \
+  CV3_STAGE(A, B, ST, true)                          \
+  fold_scales<RM, RN>(acc, big, small, sc);
+    for (; s + 4 <= NS; s += 4) {
+      CV3_BLOCK(sh0, sh1, s)
+      CV3_BLOCK(sh1, sh2, s + 1)
+      CV3_BLOCK(sh2, sh3, s + 2)
+      CV3_BLOCK(sh3, sh0, s + 3)
+    }
+    if (s < NS) {  // NS is even
+      CV3_BLOCK(sh0, sh1, s)
+      CV3_BLOCK(sh1, sh2, s + 1)
     }
 #undef CV3_BLOCK
   } else if constexpr (NST == 4) {
@@ -509,7 +581,7 @@ __global__ __launch_bounds__(64 * WM * WN) void k_pg_lds(PlaneParams p) {
   for (int i = 0; i < RM; ++i)
 #pragma unroll
     for (int j = 0; j < RN; ++j) {
-      if constexpr (KIND != W_Q8_BLOCK) acc[i][j] = big[i][j] + small[i][j];
+      if constexpr (fold_steps(KIND) == 0) acc[i][j] = big[i][j] + small[i][j];
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
         const int q = (i * RN + j) * 4 + g;
@@ -522,35 +594,56 @@ __global__ __launch_bounds__(64 * WM * WN) void k_pg_lds(PlaneParams p) {
   ep.store(p, v);
 }
 
+// Packed row r is source row r, but within the first `limit` rows each run of `span` rows is its two
+// halves interleaved (span 0: none).
+__device__ __forceinline__ int64_t source_row(int64_t r, int64_t span, int64_t limit) {
+  return r < limit ? r / span * span + (r & 1) * (span / 2) + (r % span) / 2 : r;
+}
+
 // frag[nb][t][l] = the codes q[32 nb + l % 32][16 t + 8 (l / 32) .. + 7] as bfloat16 (exact; rows past n
-// zero), and scales transposed to float32 [blocks][32 nbw].
-__global__ __launch_bounds__(256) void k_pack_q8_planes(const int8_t* q, int64_t n, int64_t k, int64_t ldq, uint4* frag,
-                                                        int64_t total) {
+// zero), and scales transposed to float32 [blocks][32 nbw].  q4: byte j of a 32-code block's 16 holds codes
+// j (low nibble) and j + 16 (high), each + 8.
+__global__ __launch_bounds__(256) void k_pack_codes(const uint8_t* q, bool q4, int64_t n, int64_t k, int64_t row_bytes,
+                                                    int64_t span, int64_t limit, uint4* frag, int64_t total) {
   const int64_t T = k / 16;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (int64_t)gridDim.x * blockDim.x) {
     const int l = (int)(i & 63);
     const int64_t t = (i >> 6) % T, row = (i >> 6) / T * 32 + (l & 31), k0 = 16 * t + 8 * (l >> 5);
-    const uint2 w = row < n ? *reinterpret_cast<const uint2*>(q + row * ldq + k0) : make_uint2(0u, 0u);
+    float v[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = 0.f;
+    if (row < n) {
+      const uint8_t* src = q + source_row(row, span, limit) * row_bytes;
+      if (q4) {
+        const uint2 w = *reinterpret_cast<const uint2*>(src + k0 / 32 * 16 + (k0 & 8));
+        const int sh = (k0 & 16) ? 4 : 0;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = (float)((int)(((j < 4 ? w.x : w.y) >> (8 * (j & 3) + sh)) & 15u) - 8);
+      } else {
+        const uint2 w = *reinterpret_cast<const uint2*>(src + k0);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = (float)((int32_t)((j < 4 ? w.x : w.y) << (24 - 8 * (j & 3))) >> 24);
+      }
+    }
     uint4 r;
     uint32_t* o = &r.x;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const uint32_t word = j < 2 ? w.x : w.y;
-      const int sh = (j & 1) * 16;
-      const f32x2_t v = {(float)((int32_t)(word << (24 - sh)) >> 24), (float)((int32_t)(word << (16 - sh)) >> 24)};
-      o[j] = __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2_t));
+      const f32x2_t p2 = {v[2 * j], v[2 * j + 1]};
+      o[j] = __builtin_bit_cast(uint32_t, __builtin_convertvector(p2, bf16x2_t));
     }
     frag[i] = r;
   }
 }
 
 __global__ __launch_bounds__(256) void k_scales_t(const void* scales, int sf16, int64_t n, int64_t npad, int64_t nb,
-                                                  int64_t use, float* out) {
+                                                  int64_t use, int64_t span, int64_t limit, float* out) {
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < use * npad; i += (int64_t)gridDim.x * blockDim.x) {
     const int64_t b = i / npad, r = i - b * npad;
+    const int64_t src = r < n ? source_row(r, span, limit) * nb + b : 0;
     out[i] = r >= n ? 0.f
-             : sf16 ? __half2float(reinterpret_cast<const __half*>(scales)[r * nb + b])
-                    : reinterpret_cast<const float*>(scales)[r * nb + b];
+             : sf16 ? __half2float(reinterpret_cast<const __half*>(scales)[src])
+                    : reinterpret_cast<const float*>(scales)[src];
   }
 }
 
@@ -586,6 +679,7 @@ constexpr Variant kVariants[3][V_COUNT] = {
 };
 
 int plane_variant(int kind, int nbm, int nbn, int S) {
+  kind = std::min(kind, (int)W_B64);
   int best = V_R11;
   float bt = 1e30f;
   for (int i = 0; i < V_COUNT; ++i) {
@@ -608,7 +702,7 @@ void launch(int variant, const PlaneParams& p, hipStream_t st) {
   const dim3 grid((unsigned)(p.tiles_m * p.tiles_n));
   // the waves a tile's K is split over and the register ring, as measured per weight kind: float32
   // steps hold three planes of both operands, so fewer fit
-  constexpr bool F = KIND == W_F32, B = KIND == W_Q8_BLOCK;
+  constexpr bool F = KIND == W_F32, B = fold_steps(KIND) > 0;
   constexpr int NST = F ? 3 : 4;
 #define CV3_REG(RM, RN, WK, PF) \
   hipLaunchKernelGGL((k_pg_reg<KIND, ACT, GATED, RM, RN, WK, PF>), grid, dim3(64 * (WK)), 0, st, p)
@@ -627,38 +721,46 @@ void launch(int variant, const PlaneParams& p, hipStream_t st) {
 }
 
 template <int KIND>
-int launch_act(int variant, const PlaneParams& p, hipStream_t st) {
+int launch_act(int act, int variant, const PlaneParams& p, hipStream_t st) {
   const bool gated = p.epi.gate || p.epi.residual;
-  switch (p.epi.act) {
-    case CV3_ACT_NONE:
-      gated ? launch<KIND, CV3_ACT_NONE, true>(variant, p, st) : launch<KIND, CV3_ACT_NONE, false>(variant, p, st);
-      return CV3_OK;
-    case CV3_ACT_GELU_TANH:
-      gated ? launch<KIND, CV3_ACT_GELU_TANH, true>(variant, p, st)
-            : launch<KIND, CV3_ACT_GELU_TANH, false>(variant, p, st);
-      return CV3_OK;
-    case CV3_ACT_SILU: launch<KIND, CV3_ACT_SILU, true>(variant, p, st); return CV3_OK;
-    default: return fail(CV3_EUNSUPPORTED, "plane linear: activation %d has no epilogue here", p.epi.act);
+  CV3_REQUIRE(!gated || act == CV3_ACT_NONE, CV3_EUNSUPPORTED,
+              "plane linear: a gate or residual comes without an activation here");
+  if (act == CV3_ACT_NONE) {
+    if (gated)
+      launch<KIND, CV3_ACT_NONE, true>(variant, p, st);
+    else
+      launch<KIND, CV3_ACT_NONE, false>(variant, p, st);
+    return CV3_OK;
   }
+  if constexpr (KIND != W_B32) {
+    if (act == CV3_ACT_GELU_TANH) {
+      launch<KIND, CV3_ACT_GELU_TANH, false>(variant, p, st);
+      return CV3_OK;
+    }
+  }
+  if constexpr (KIND != W_F32) {
+    if (act == A_SWIGLU) {
+      launch<KIND, A_SWIGLU, false>(variant, p, st);
+      return CV3_OK;
+    }
+    if (act == A_QKV) {
+      launch<KIND, A_QKV, false>(variant, p, st);
+      return CV3_OK;
+    }
+  }
+  return fail(CV3_EUNSUPPORTED, "plane linear: activation %d has no epilogue here", act);
 }
 
-int plane_linear(int kind, const uint16_t* x, int64_t m, int64_t k, const uint16_t* w, const float* scales, int64_t n,
-                 const float* bias, float* y, int64_t ldy, uint16_t* y_planes, const cv3_epilogue* epi,
-                 int64_t plan_rows, hipStream_t st) {
-  CV3_REQUIRE(k % 64 == 0 && k >= (kind == W_Q8_BLOCK ? 256 : 128) && n % 4 == 0 && (!y_planes || n % 16 == 0),
-              CV3_EUNSUPPORTED, "plane linear needs K %% 64 == 0, K >= 128 (block scales: 256), N %% 4 == 0 (K = %lld, N = %lld)",
-              (long long)k, (long long)n);
+// Fills the shape, tile and operands of p (its epilogue set) and launches it.
+int plane_launch(int kind, int act, PlaneParams& p, const uint16_t* x, int64_t m, int64_t k, const uint16_t* w,
+                 const float* scales, int64_t n, const float* bias, int64_t plan_rows, hipStream_t st) {
   auto a16 = [](const void* q) { return (uintptr_t)q % 16 == 0; };
-  PlaneParams p{};
-  p.epi = epi ? *epi : cv3_epilogue{};
-  const cv3_epilogue& e = p.epi;
-  CV3_REQUIRE(a16(x) && a16(w) && a16(scales) && a16(bias) && a16(y) && a16(y_planes) && ldy % 4 == 0 && a16(e.residual) &&
-                  e.ld_res % 4 == 0 && a16(e.gate) && e.gate_stride % 4 == 0 && a16(e.rope_cos) && a16(e.rope_sin),
-              CV3_EINVAL, "plane linear operands must be 16-byte aligned rows");
-  CV3_REQUIRE(!e.rope_cos || (e.rope_sin && e.rope_rows > 0 && e.rope_period > 0 && e.rope_period % 4 == 0 &&
-                              e.rope_width % 4 == 0 && e.rope_rows * e.rope_width < (1ll << 31)),
-              CV3_EINVAL, "plane linear: rotary widths must be multiples of four, the table within 32 bits");
-  CV3_REQUIRE(m < (1ll << 30) && plan_rows < (1ll << 30) && n < (1ll << 30) && k < (1ll << 30) && e.rows_per_gate < (1ll << 31), CV3_EINVAL,
+  CV3_REQUIRE(k % 64 == 0 && k >= (fold_steps(kind) ? 256 : 128) && n % 4 == 0, CV3_EUNSUPPORTED,
+              "plane linear needs K %% 64 == 0, K >= 128 (block scales: 256), N %% 4 == 0 (K = %lld, N = %lld)",
+              (long long)k, (long long)n);
+  CV3_REQUIRE(a16(x) && a16(w) && a16(scales) && a16(bias) && a16(p.c) && a16(p.yp) && p.ldc % 4 == 0, CV3_EINVAL,
+              "plane linear operands must be 16-byte aligned rows");
+  CV3_REQUIRE(m < (1ll << 30) && plan_rows < (1ll << 30) && n < (1ll << 30) && k < (1ll << 30), CV3_EINVAL,
               "plane linear too large");
   p.S = (int)(k / 16);
   p.nbw = (int)ceil_div(n, 32);
@@ -671,12 +773,8 @@ int plane_linear(int kind, const uint16_t* x, int64_t m, int64_t k, const uint16
   p.m = (int)m;
   p.n = (int)n;
   p.bias = bias;
-  p.c = y;
-  p.ldc = ldy;
-  p.yp = reinterpret_cast<uint2*>(y_planes);
-  p.ypl = (int64_t)p.nbx * (n / 16) * 128;
   const int v = plane_variant(kind, (int)ceil_div(plan_rows > 0 ? plan_rows : m, 32), p.nbw, p.S);
-  const Variant& t = kVariants[kind][v];
+  const Variant& t = kVariants[std::min(kind, (int)W_B64)][v];
   p.tiles_m = (int)ceil_div(p.nbx, t.tm);
   p.tiles_n = (int)ceil_div(p.nbw, t.tn);
   CV3_REQUIRE((int64_t)p.tiles_m * p.tiles_n < (1ll << 31), CV3_EINVAL, "plane linear too large");
@@ -685,12 +783,34 @@ int plane_linear(int kind, const uint16_t* x, int64_t m, int64_t k, const uint16
   int gm = 1;
   while (gm < p.tiles_m && (double)gm * gm * xb < per * wb) ++gm;
   p.gm = gm;
-  const int rc = kind == W_F32  ? launch_act<W_F32>(v, p, st)
-                 : kind == W_Q8 ? launch_act<W_Q8>(v, p, st)
-                                : launch_act<W_Q8_BLOCK>(v, p, st);
+  const int rc = kind == W_F32   ? launch_act<W_F32>(act, v, p, st)
+                 : kind == W_ROW ? launch_act<W_ROW>(act, v, p, st)
+                 : kind == W_B64 ? launch_act<W_B64>(act, v, p, st)
+                                 : launch_act<W_B32>(act, v, p, st);
   if (rc) return rc;
   CV3_LAUNCHED();
   return CV3_OK;
+}
+
+int plane_linear(int kind, const uint16_t* x, int64_t m, int64_t k, const uint16_t* w, const float* scales, int64_t n,
+                 const float* bias, float* y, int64_t ldy, uint16_t* y_planes, const cv3_epilogue* epi,
+                 int64_t plan_rows, hipStream_t st) {
+  CV3_REQUIRE(!y_planes || n % 16 == 0, CV3_EUNSUPPORTED, "a result in planes needs N %% 16 == 0 (N = %lld)", (long long)n);
+  auto a16 = [](const void* q) { return (uintptr_t)q % 16 == 0; };
+  PlaneParams p{};
+  p.epi = epi ? *epi : cv3_epilogue{};
+  const cv3_epilogue& e = p.epi;
+  CV3_REQUIRE(a16(e.residual) && e.ld_res % 4 == 0 && a16(e.gate) && e.gate_stride % 4 == 0 && a16(e.rope_cos) &&
+                  a16(e.rope_sin) && e.rows_per_gate < (1ll << 31),
+              CV3_EINVAL, "plane linear operands must be 16-byte aligned rows");
+  CV3_REQUIRE(!e.rope_cos || (e.rope_sin && e.rope_rows > 0 && e.rope_period > 0 && e.rope_period % 4 == 0 &&
+                              e.rope_width % 4 == 0 && e.rope_rows * e.rope_width < (1ll << 31)),
+              CV3_EINVAL, "plane linear: rotary widths must be multiples of four, the table within 32 bits");
+  p.c = y;
+  p.ldc = ldy;
+  p.yp = reinterpret_cast<uint2*>(y_planes);
+  p.ypl = ceil_div(m, 32) * (n / 16) * 128;
+  return plane_launch(kind, e.act, p, x, m, k, w, scales, n, bias, plan_rows, st);
 }
 
 // One wave per row of at most 1024 columns (a multiple of 16): lane l holds the 8-column chunks l and
@@ -805,7 +925,7 @@ int cv3_linear_x3_planes(const uint16_t* x, int64_t m, int64_t k, const uint16_t
   return plane_linear(W_F32, x, m, k, frag, nullptr, n, bias, y, ldy, y_planes, epi, plan_rows, stream_of(s));
 }
 
-int cv3_q8_planes_elems(int64_t n, int64_t k, int64_t block, int64_t* codes, int64_t* scales) {
+int cv3_code_planes_elems(int64_t n, int64_t k, int64_t block, int64_t* codes, int64_t* scales) {
   CV3_REQUIRE(n >= 0 && k > 0 && block > 0 && codes && scales, CV3_EINVAL, "bad shape or null output");
   const int64_t npad = ceil_div(n, 32) * 32;
   *codes = npad * k;
@@ -813,34 +933,43 @@ int cv3_q8_planes_elems(int64_t n, int64_t k, int64_t block, int64_t* codes, int
   return CV3_OK;
 }
 
-int cv3_pack_q8_planes(const int8_t* q, int64_t n, int64_t k, int64_t ldq, const void* scales, int scale_dtype,
-                       int64_t kp, int64_t block, uint16_t* frag, float* scales_t, cv3_stream_t s) {
+int cv3_pack_code_planes(int kind, const void* q, int64_t n, int64_t k, const void* scales, int scale_dtype, int64_t kp,
+                         int64_t block, int64_t span, int64_t limit, uint16_t* frag, float* scales_t, cv3_stream_t s) {
   CV3_ALIVE();
-  CV3_REQUIRE(n >= 0 && k > 0 && k % 64 == 0 && ldq >= k && ldq % 8 == 0 && block > 0 && kp >= k && kp % block == 0,
-              CV3_EINVAL, "bad code pack shape n=%lld k=%lld block=%lld", (long long)n, (long long)k, (long long)block);
-  CV3_REQUIRE(block == 64 || block >= k, CV3_EUNSUPPORTED, "plane codes take 64-code blocks or one scale a row");
+  CV3_REQUIRE(kind == CV3_KIND_Q8 || kind == CV3_KIND_Q4, CV3_EINVAL, "unknown quant kind %d", kind);
+  CV3_REQUIRE(n >= 0 && k > 0 && k % 64 == 0 && block > 0 && kp >= k && kp % block == 0 && kp % 16 == 0, CV3_EINVAL,
+              "bad code pack shape n=%lld k=%lld block=%lld", (long long)n, (long long)k, (long long)block);
+  CV3_REQUIRE(span >= 0 && span % 2 == 0 && (span ? limit >= 0 && limit <= n && limit % span == 0 : limit == 0),
+              CV3_EINVAL, "bad row interleave span=%lld limit=%lld", (long long)span, (long long)limit);
+  CV3_REQUIRE(block == 64 || block == 32 || block >= k, CV3_EUNSUPPORTED,
+              "plane codes take 32- or 64-code blocks or one scale a row");
+  CV3_REQUIRE(kind == CV3_KIND_Q8 || (block == 32 && scale_dtype == CV3_F16), CV3_EUNSUPPORTED,
+              "q4 codes come in 32-code blocks with float16 scales");
   CV3_REQUIRE((uintptr_t)q % 8 == 0 && (uintptr_t)frag % 16 == 0 && (uintptr_t)scales_t % 16 == 0, CV3_EINVAL,
               "plane codes need aligned rows");
   const int64_t npad = ceil_div(n, 32) * 32, total = npad * k / 8, use = block >= k ? 1 : k / block;
   if (!total) return CV3_OK;
   hipStream_t st = stream_of(s);
-  hipLaunchKernelGGL(k_pack_q8_planes, dim3((unsigned)(ceil_div(total, 256) < 65536 ? ceil_div(total, 256) : 65536)),
-                     dim3(256), 0, st, q, n, k, ldq, reinterpret_cast<uint4*>(frag), total);
+  const bool q4 = kind == CV3_KIND_Q4;
+  hipLaunchKernelGGL(k_pack_codes, dim3((unsigned)(ceil_div(total, 256) < 65536 ? ceil_div(total, 256) : 65536)),
+                     dim3(256), 0, st, reinterpret_cast<const uint8_t*>(q), q4, n, k, q4 ? kp / 2 : kp, span, limit,
+                     reinterpret_cast<uint4*>(frag), total);
   hipLaunchKernelGGL(k_scales_t, dim3((unsigned)ceil_div(use * npad, 256)), dim3(256), 0, st, scales,
-                     scale_dtype == CV3_F16 ? 1 : 0, n, npad, kp / block, use, scales_t);
+                     scale_dtype == CV3_F16 ? 1 : 0, n, npad, kp / block, use, span, limit, scales_t);
   CV3_LAUNCHED();
   return CV3_OK;
 }
 
-int cv3_linear_q8_planes(const uint16_t* x, int64_t m, int64_t k, const uint16_t* frag, const float* scales_t,
+int cv3_linear_code_planes(const uint16_t* x, int64_t m, int64_t k, const uint16_t* frag, const float* scales_t,
                          int64_t block, int64_t n, const float* bias, float* y, int64_t ldy, uint16_t* y_planes,
                          const cv3_epilogue* epi, int64_t plan_rows, cv3_stream_t s) {
   CV3_ALIVE();
   CV3_REQUIRE(m >= 0 && k > 0 && n >= 0 && (!y || ldy >= n) && (y || y_planes) && scales_t, CV3_EINVAL,
               "bad plane linear shape m=%lld k=%lld n=%lld", (long long)m, (long long)k, (long long)n);
-  CV3_REQUIRE(block == 64 || block >= k, CV3_EUNSUPPORTED, "plane codes take 64-code blocks or one scale a row");
+  CV3_REQUIRE(block == 64 || block == 32 || block >= k, CV3_EUNSUPPORTED,
+              "plane codes take 32- or 64-code blocks or one scale a row");
   if (!m || !n) return CV3_OK;
-  return plane_linear(block >= k ? W_Q8 : W_Q8_BLOCK, x, m, k, frag, scales_t, n, bias, y, ldy, y_planes, epi,
+  return plane_linear(block >= k ? W_ROW : block == 64 ? W_B64 : W_B32, x, m, k, frag, scales_t, n, bias, y, ldy, y_planes, epi,
                       plan_rows, stream_of(s));
 }
 
@@ -856,6 +985,82 @@ int cv3_rms_norm_planes(const float* x, const float* w, uint16_t* planes, int64_
   CV3_ALIVE();
   CV3_REQUIRE(w, CV3_EINVAL, "an RMS norm needs its weight");
   return norm_planes(true, x, planes, rows, cols, eps, w, nullptr, nullptr, stream_of(s));
+}
+
+// Qwen2Model.forward over t prompt rows at positions pos0 .. (qwen2.py:139-179), then the last position's
+// head logits: seven launches a layer.
+namespace {
+__global__ void k_set_pos(int64_t* pos, int64_t v) { *pos = v; }
+}  // namespace
+
+int cv3_qwen2_prefill(const cv3_qwen2_model* m, const cv3_qwen2_state* st, const cv3_qwen2_planes* w, const float* x,
+                      int64_t t, int64_t pos0, float* h, float* q, uint16_t* planes, uint16_t* inter_planes,
+                      cv3_stream_t s) {
+  CV3_ALIVE();
+  CV3_REQUIRE(m && st && w && x && h && q && planes && inter_planes, CV3_EINVAL, "null prefill operand");
+  const int64_t D = m->hidden, I = m->inter, H = m->heads, Hk = m->kv_heads, L = m->layers, cap = st->cap;
+  const int64_t R = (H + 2 * Hk) * 64;
+  CV3_REQUIRE(m->head_dim == 64 && H > 0 && Hk > 0 && H % Hk == 0 && H * 64 == D && D % 64 == 0 && D <= 1024 && D >= 256 &&
+                  I % 64 == 0 && I >= 256,
+              CV3_EUNSUPPORTED, "prompt planes take head dim 64, hidden 256 .. 1024 and multiples of 64");
+  CV3_REQUIRE(t > 0 && pos0 >= 0 && pos0 + t <= cap && cap < (1ll << 30), CV3_EINVAL, "the prompt does not fit the KV cache");
+  hipStream_t stream = stream_of(s);
+  auto kind_of = [](int64_t block, int64_t k) { return block >= k ? W_ROW : block == 64 ? W_B64 : W_B32; };
+  // a projection's fragments and scales per layer
+  auto at = [&](const cv3_code_planes& c, int64_t l, int64_t rows, int64_t k, const uint16_t*& f, const float*& sc) {
+    f = c.frag + l * rows * k;
+    sc = c.scales + l * rows * (c.block >= k ? 1 : k / c.block);
+  };
+  const uint16_t* f;
+  const float* sc;
+  int rc;
+  for (int64_t l = 0; l < L; ++l) {
+    const float* in = l ? h : x;
+    if ((rc = norm_planes(true, in, planes, t, D, m->eps, m->ln1 + l * D, nullptr, nullptr, stream))) return rc;
+    at(w->qkv, l, R, D, f, sc);
+    PlaneParams p{};
+    p.c = q;
+    p.ldc = H * 64;
+    p.kc = st->k_cache + (l * Hk * cap + pos0) * 64;
+    p.vc = st->v_cache + (l * Hk * cap + pos0) * 64;
+    p.heads = (int)H;
+    p.kv_heads = (int)Hk;
+    p.cap = (int)cap;
+    p.pos0 = (int)pos0;
+    p.cos = m->rope_cos;
+    p.sin = m->rope_sin;
+    if ((rc = plane_launch(kind_of(w->qkv.block, D), A_QKV, p, planes, t, D, f, sc, R, w->qkv_bias + l * R, 0, stream)))
+      return rc;
+    const int64_t qs[3] = {0, 64, H * 64}, ks[3] = {0, cap * 64, 64};
+    if ((rc = cv3_attention_x3_planes(q, st->k_cache + l * Hk * cap * 64, st->v_cache + l * Hk * cap * 64, planes, 1, (int)H,
+                                      (int)Hk, t, pos0 + t, 64, qs, ks, ks, 0.125f, t > 1 ? 1 : 0, pos0, 0, s)))
+      return rc;
+    at(w->o, l, D, D, f, sc);
+    cv3_epilogue e{};
+    e.residual = in;
+    e.ld_res = D;
+    if ((rc = plane_linear(kind_of(w->o.block, D), planes, t, D, f, sc, D, nullptr, h, D, nullptr, &e, 0, stream))) return rc;
+    if ((rc = norm_planes(true, h, planes, t, D, m->eps, m->ln2 + l * D, nullptr, nullptr, stream))) return rc;
+    at(w->gate_up, l, 2 * I, D, f, sc);
+    PlaneParams g{};
+    g.yp = reinterpret_cast<uint2*>(inter_planes);
+    g.ypl = ceil_div(t, 32) * (I / 16) * 128;
+    if ((rc = plane_launch(kind_of(w->gate_up.block, D), A_SWIGLU, g, planes, t, D, f, sc, 2 * I, nullptr, 0, stream)))
+      return rc;
+    at(w->down, l, D, I, f, sc);
+    e.residual = h;
+    if ((rc = plane_linear(kind_of(w->down.block, I), inter_planes, t, I, f, sc, D, nullptr, h, D, nullptr, &e, 0, stream)))
+      return rc;
+  }
+  // the last position: final norm, head, and its position for the decode
+  if ((rc = cv3_rms_norm(h + (t - 1) * D, m->norm, q, 1, D, m->eps, s))) return rc;
+  const cv3_qweight& hd = m->head;
+  if ((rc = cv3_linear_q(hd.kind, q, 1, D, D, hd.q, hd.scales, hd.scale_dtype, hd.kp, hd.block, hd.rows, m->head_bias,
+                         st->logits, hd.rows, nullptr, s)))
+    return rc;
+  hipLaunchKernelGGL(k_set_pos, dim3(1), dim3(1), 0, stream, st->pos, pos0 + t - 1);
+  CV3_LAUNCHED();
+  return CV3_OK;
 }
 
 }  // extern "C"

@@ -88,7 +88,7 @@ class DeviceLinear:
     below its largest element), given ``rexp``, an int32 workspace of at least m entries.
 
     ``frag_x=True`` also readies the weight for activations that come as bfloat16 planes in fragment
-    order (``from_planes``, cv3_linear_x3_planes / cv3_linear_q8_planes), where ``takes_planes`` says
+    order (``from_planes``, cv3_linear_x3_planes / cv3_linear_code_planes), where ``takes_planes`` says
     it can: float32 planes as they are, q8 codes (64-code blocks or one scale a row) widened to
     bfloat16 beside the packed codes.
     """
@@ -125,10 +125,10 @@ class DeviceLinear:
                               and self.k <= 2048)
             if frag_x and self.q8_planes and not self.q8_digits and (self.block == 64 or self.block >= self.k):
                 nc, ns = ctypes.c_int64(), ctypes.c_int64()
-                _lib.call("q8_planes_elems", self.n, self.k, self.block, ctypes.byref(nc), ctypes.byref(ns))
+                _lib.call("code_planes_elems", self.n, self.k, self.block, ctypes.byref(nc), ctypes.byref(ns))
                 self.codes16, self.scales_t = DeviceArray((nc.value,), np.uint16), DeviceArray((ns.value,))
-                _lib.call("pack_q8_planes", self.q.ptr, self.n, self.k, self.kp, self.scales.ptr,
-                          _lib.F16 if self.sf16 else _lib.F32, self.kp, self.block, self.codes16.ptr,
+                _lib.call("pack_code_planes", _lib.KIND_Q8, self.q.ptr, self.n, self.k, self.scales.ptr,
+                          _lib.F16 if self.sf16 else _lib.F32, self.kp, self.block, 0, 0, self.codes16.ptr,
                           self.scales_t.ptr, None)
             if self.q8_digits:
                 npad = -(-self.n // 32) * 32
@@ -175,7 +175,7 @@ class DeviceLinear:
         b = self.bias.ptr if self.bias is not None else None
         e = ctypes.byref(epi) if epi is not None else None
         if self.q8:
-            _lib.call("linear_q8_planes", x, m, self.k, self.codes16.ptr, self.scales_t.ptr, self.block, self.n, b, y,
+            _lib.call("linear_code_planes", x, m, self.k, self.codes16.ptr, self.scales_t.ptr, self.block, self.n, b, y,
                       ldy, y_planes, e, plan_rows, st)
         else:
             _lib.call("linear_x3_planes", x, m, self.k, self.planes.ptr, self.n, b, y, ldy, y_planes, e,

@@ -49,6 +49,15 @@ class Persist(ctypes.Structure):
                 ("workgroups", ctypes.c_int), ("cooperative", ctypes.c_int)]
 
 
+class CodePlanes(ctypes.Structure):
+    _fields_ = [("frag", c_vp), ("scales", c_vp), ("block", c_i64)]
+
+
+class Planes(ctypes.Structure):
+    _fields_ = [("qkv", CodePlanes), ("o", CodePlanes), ("gate_up", CodePlanes), ("down", CodePlanes),
+                ("qkv_bias", c_vp)]
+
+
 class Sampler(ctypes.Structure):
     _fields_ = [("top_p", ctypes.c_double), ("rep_threshold", ctypes.c_double), ("top_k", c_i64),
                 ("win_size", c_i64), ("speech_token_size", c_i64), ("min_len", c_i64),
@@ -144,6 +153,19 @@ class _Stacked:
         return QWeight(self.q.ptr, self.scales.ptr, self.rows, self.k, self.kp, self.block,
                        _lib.F16 if self.sf16 else _lib.F32, _lib.KIND_Q4 if self.kind == "q4" else _lib.KIND_Q8)
 
+    def planes(self, span: int = 0, limit: int = 0):
+        """(fragments, scales) of every layer's rows for cv3_linear_code_planes, each layer packed on its
+        own; ``span`` / ``limit`` interleave rows as cv3_pack_code_planes does."""
+        layers = self.q.shape[0] // self.rows
+        nc, ns = ctypes.c_int64(), ctypes.c_int64()
+        _lib.call("code_planes_elems", self.rows, self.k, self.block, ctypes.byref(nc), ctypes.byref(ns))
+        frag, scales = DeviceArray((layers, nc.value), np.uint16), DeviceArray((layers, ns.value))
+        for l in range(layers):
+            kind, q, sc, sdt, kp, block, n = self.layer(l)
+            _lib.call("pack_code_planes", kind, q, n, self.k, sc, sdt, kp, block, span, limit,
+                      frag.ptr + 2 * l * nc.value, scales.ptr + 4 * l * ns.value, None)
+        return frag, scales
+
     @property
     def nbytes(self):
         """Bytes held in HBM (a widened q4 body: int8 codes)."""
@@ -208,6 +230,7 @@ class DeviceQwen2:
         p0 = self.ints.ptr
         self.state = State(self.k_cache.ptr, self.v_cache.ptr, self.cap, p0, p0 + 8, p0 + 16, self.x.ptr,
                            self.logits.ptr, self.workspace.ptr, nws)
+        self._prompt = self._prompt_planes()
         self._graph: Optional[Graph] = None
         self._pos_host = 0
         # sampler control block: [start, stop step + 1, PCG64 state hi, lo, inc hi, lo]
@@ -217,6 +240,31 @@ class DeviceQwen2:
         # the one-launch step's launch: ordinary (the device runs nothing else meanwhile) or
         # hipLaunchCooperativeKernel, which guarantees co-residency at ~20 us more per token
         self.cooperative = False
+
+    def _prompt_planes(self) -> Optional[Planes]:
+        """The body's projections as code planes for ``prefill`` (cv3_qwen2_prefill), beside the decode's
+        rows: q and k heads with their halves interleaved, so that a rotary pair is two neighbouring
+        outputs, and gate beside up.  None for geometries it does not take."""
+        D, I, dh = self.hidden, self.inter, self.head_dim
+        ok = (dh == 64 and self.heads * dh == D and D % 64 == 0 and 256 <= D <= 1024 and I % 64 == 0 and I >= 256
+              and self.heads % self.kv_heads == 0)
+        for w in (self.qkv, self.o, self.gate_up, self.down):
+            ok = ok and w.rows % 32 == 0 and (w.block in (32, 64) or w.block >= w.k) and w.kp % 16 == 0
+        if not ok:
+            return None
+        turned = (self.heads + self.kv_heads) * dh
+        p, self._prompt_arrays = Planes(), []
+        for name, w, span, limit in (("qkv", self.qkv, dh, turned), ("o", self.o, 0, 0),
+                                     ("gate_up", self.gate_up, 2 * I, 2 * I), ("down", self.down, 0, 0)):
+            frag, scales = w.planes(span, limit)
+            self._prompt_arrays += [frag, scales]
+            setattr(p, name, CodePlanes(frag.ptr, scales.ptr, w.block))
+        b = self.qkv_bias.numpy().reshape(self.layers, -1)
+        qk = b[:, :turned].reshape(self.layers, -1, 2, dh // 2).transpose(0, 1, 3, 2).reshape(self.layers, -1)
+        bias = to_device(np.concatenate([qk, b[:, turned:]], axis=1))
+        self._prompt_arrays.append(bias)
+        p.qkv_bias = bias.ptr
+        return p
 
     # -- weights streamed per token (the HBM roofline numerator) -----------
     def bytes_per_token(self, length: int) -> dict:
@@ -280,6 +328,8 @@ class DeviceQwen2:
         (qwen2.py:139-179) on the device: RMSNorm, [q; k; v] projection with bias, half-split
         rotary, k and v appended to the cache, causal attention over the cache (mask
         ("causal", pos0) when T > 1), o_proj + residual, RMSNorm, SwiGLU, down + residual.
+        On the bfloat16 matrix cores with the activations as planes (cv3_qwen2_prefill) where the
+        geometry allows it, else layer by layer on the float32 ones.
         Leaves the head logits of the last position in ``logits`` and ``pos`` at that
         position, so ``select`` / ``generate_*_after_prefill`` draw the next token."""
         xd = x if isinstance(x, DeviceArray) else to_device(np.ascontiguousarray(x, np.float32))
@@ -289,6 +339,18 @@ class DeviceQwen2:
         if pos0 < 0 or pos0 + t >= self.cap:
             raise ValueError("the prompt does not fit the KV cache")
         D, H, Hk, dh, I, cap = self.hidden, self.heads, self.kv_heads, self.head_dim, self.inter, self.cap
+        if self._prompt is not None:
+            if xd.ptr % 16:
+                xd = xd.copy()
+            work = [DeviceArray((t, D)), DeviceArray((t, D))]
+            for k in (D, I):
+                ne = ctypes.c_int64()
+                _lib.call("x3_frag_elems", t, k, ctypes.byref(ne))
+                work.append(DeviceArray((ne.value,), np.uint16))
+            _lib.call("qwen2_prefill", ctypes.byref(self.model), ctypes.byref(self.state), ctypes.byref(self._prompt),
+                      xd.ptr, t, pos0, *(w.ptr for w in work), None)
+            self._pos_host = pos0 + t - 1
+            return
         R = self.qkv.rows
         h = DeviceArray((t, D))
         _lib.call("copy_d2d", h.ptr, xd.ptr, t * D * 4, None)

@@ -186,20 +186,22 @@ int cv3_linear_q8_digits(const float* x, int64_t m, int64_t k, int64_t ldx, cons
  * cv3_split_x3_frag writes for [m, k] rows (cv3_x3_frag_elems(m, k) uint16), made by the kernel before
  * (cv3_layer_norm_planes, cv3_rms_norm_planes, cv3_attention_x3_planes, or y_planes of the linear before).
  * The result goes to float32 rows (y), to its own planes (y_planes, cv3_x3_frag_elems(m, n); n % 16), or
- * both.  q8 codes are held as bfloat16 (exact) in fragment order, the scales transposed to float32
- * [blocks][ceil(n / 32) * 32]: 64-code blocks, or one scale a row (block >= k).  K % 64 == 0, K >= 128
- * (64-code blocks: 256), n % 4 == 0, 16-byte aligned operands; activations none, GELU (tanh), SiLU.
- * plan_rows (0: m): the rows that the tile, and with it the order of the sums, is chosen for; parts of one
- * batch launched side by side pass the batch's, fill the machine as its tiles do and return its bits. */
+ * both.  Quantised codes are held as bfloat16 (exact) in fragment order, the scales transposed to float32
+ * [blocks][ceil(n / 32) * 32]: 32- or 64-code blocks, or one scale a row (block >= k); span interleaves the two
+ * halves of every `span` rows among the first `limit` (0, 0: rows in order).  K % 64 == 0, K >= 128 (blocks:
+ * 256), n % 4 == 0, 16-byte aligned operands; a bias and rotary, then GELU (tanh), a gate and residual, or
+ * neither (GELU not with 32-code blocks).  plan_rows (0: m): the rows that the tile, and with it the order of
+ * the sums, is chosen for; parts of one batch launched side by side pass the batch's, fill the machine as its
+ * tiles do and return its bits. */
 int cv3_linear_x3_planes(const uint16_t* x, int64_t m, int64_t k, const uint16_t* frag, int64_t n, const float* bias,
                          float* y, int64_t ldy, uint16_t* y_planes, const cv3_epilogue* epi, int64_t plan_rows,
                          cv3_stream_t s);
-int cv3_q8_planes_elems(int64_t n, int64_t k, int64_t block, int64_t* codes, int64_t* scales);
-int cv3_pack_q8_planes(const int8_t* q, int64_t n, int64_t k, int64_t ldq, const void* scales, int scale_dtype,
-                       int64_t kp, int64_t block, uint16_t* frag, float* scales_t, cv3_stream_t s);
-int cv3_linear_q8_planes(const uint16_t* x, int64_t m, int64_t k, const uint16_t* frag, const float* scales_t,
-                         int64_t block, int64_t n, const float* bias, float* y, int64_t ldy, uint16_t* y_planes,
-                         const cv3_epilogue* epi, int64_t plan_rows, cv3_stream_t s);
+int cv3_code_planes_elems(int64_t n, int64_t k, int64_t block, int64_t* codes, int64_t* scales);
+int cv3_pack_code_planes(int kind, const void* q, int64_t n, int64_t k, const void* scales, int scale_dtype, int64_t kp,
+                         int64_t block, int64_t span, int64_t limit, uint16_t* frag, float* scales_t, cv3_stream_t s);
+int cv3_linear_code_planes(const uint16_t* x, int64_t m, int64_t k, const uint16_t* frag, const float* scales_t,
+                           int64_t block, int64_t n, const float* bias, float* y, int64_t ldy, uint16_t* y_planes,
+                           const cv3_epilogue* epi, int64_t plan_rows, cv3_stream_t s);
 /* AdaLN (dit.py:168-169) and RMSNorm (ops.py:101-104) whose result is [rows, cols] planes in fragment
  * order; cols a multiple of 16, at most 1024, 16-byte aligned operands. */
 int cv3_layer_norm_planes(const float* x, uint16_t* planes, int64_t rows, int64_t cols, float eps, const float* shift,
@@ -496,6 +498,25 @@ int cv3_qwen2_select(const cv3_qwen2_model* m, const cv3_qwen2_state* s, const c
 /* n doubles of Generator.random() from the PCG64 state pcg[0..3] (device, layout as in cv3_sampler.ctl[2..5]),
  * which is advanced: the draw primitive of the sampler, exposed so its stream can be checked against NumPy. */
 int cv3_pcg64_random(int64_t* pcg, int64_t n, double* out, cv3_stream_t stream);
+/* The body's projections for prompts, packed by cv3_pack_code_planes layer after layer: qkv with each q and k
+ * head's halves interleaved (span head_dim), gate_up with the gate and up rows interleaved (span 2 inter);
+ * qkv_bias [layers, qkv rows] in qkv's row order. */
+typedef struct {
+  const uint16_t* frag;
+  const float* scales;
+  int64_t block;
+} cv3_code_planes;
+typedef struct {
+  cv3_code_planes qkv, o, gate_up, down;
+  const float* qkv_bias;
+} cv3_qwen2_planes;
+/* Qwen2Model.forward over t prompt embeddings x [t, hidden] at positions pos0 .. pos0 + t - 1 (qwen2.py:139-179):
+ * k and v into the cache rows, causal attention over the cache, and the head logits of the last position, whose
+ * index *pos then holds.  Workspace: h and q [t, hidden] floats, planes and inter_planes cv3_x3_frag_elems(t, hidden)
+ * and (t, inter) uint16.  head_dim 64, hidden 256 .. 1024, multiples of 64. */
+int cv3_qwen2_prefill(const cv3_qwen2_model* m, const cv3_qwen2_state* s, const cv3_qwen2_planes* w, const float* x,
+                      int64_t t, int64_t pos0, float* h, float* q, uint16_t* planes, uint16_t* inter_planes,
+                      cv3_stream_t stream);
 /* x = speech_embedding[*token] (ops.py:126-144): the first input of a decode. */
 int cv3_qwen2_embed_token(const cv3_qwen2_model* m, const cv3_qwen2_state* s, cv3_stream_t stream);
 

@@ -82,11 +82,11 @@ def test_linear_from_planes(lib, m, k, n, kind):
         w64 = (q.astype(np.float64).reshape(n, -1, block) * s.astype(np.float64)[:, :, None]).reshape(n, -1)[:, :k]
         qd, sd = to_device(np.ascontiguousarray(q)), to_device(np.ascontiguousarray(s))
         nc, ns = ctypes.c_int64(), ctypes.c_int64()
-        _lib.call("q8_planes_elems", n, k, block, ctypes.byref(nc), ctypes.byref(ns))
+        _lib.call("code_planes_elems", n, k, block, ctypes.byref(nc), ctypes.byref(ns))
         wd, st = empty((nc.value,), np.uint16), empty((ns.value,))
-        _lib.call("pack_q8_planes", qd.ptr, n, k, kp, sd.ptr, _lib.F16 if sdt == np.float16 else _lib.F32, kp, block,
-                  wd.ptr, st.ptr, None)
-        run = lambda *a: _lib.call("linear_q8_planes", xp.ptr, m, k, wd.ptr, st.ptr, block, n, *a)  # noqa: E731
+        _lib.call("pack_code_planes", _lib.KIND_Q8, qd.ptr, n, k, sd.ptr, _lib.F16 if sdt == np.float16 else _lib.F32,
+                  kp, block, 0, 0, wd.ptr, st.ptr, None)
+        run = lambda *a: _lib.call("linear_code_planes", xp.ptr, m, k, wd.ptr, st.ptr, block, n, *a)  # noqa: E731
     want = x.astype(np.float64) @ w64.T + b
     y = empty((m, n))
     run(bd.ptr, y.ptr, n, None, None, 0, None)
@@ -162,3 +162,34 @@ def test_plane_linear_refuses_what_it_cannot_read(lib):
             _lib.call("linear_x3_planes", a.ptr, m, k, a.ptr, n, None, a.ptr, n, None, None, 0, None)
     with pytest.raises(ValueError):
         _lib.call("linear_x3_planes", a.ptr + 4, 4, 128, a.ptr, 32, None, a.ptr, 32, None, None, 0, None)
+
+
+@pytest.mark.parametrize("profile,t,pos0", [("per_channel", 1, 0), ("per_channel", 33, 7), ("balanced", 130, 0),
+                                            ("tiny", 65, 1), ("tiny", 1, 40), ("per_channel", 321, 0),
+                                            ("balanced", 500, 20), ("tiny", 300, 0)])
+def test_prompt_on_code_planes(gpu, profile, t, pos0):
+    """DeviceQwen2.prefill on code planes against the same method's float32 route (its former only one, pinned
+    to the oracle by test_gpu_decode.py): logits, the appended cache rows and the position, at fragment and
+    tile edges, one row, and on top of cached rows, for every storage profile."""
+    import cv3amd.quant as quant
+    from cv3amd import synth
+    from cv3amd.qwen2 import DeviceQwen2
+    from cv3amd.weights import WeightStore
+    tensors = synth.quantize_store(synth.qwen2_tensors(layers=2), profile, quant.quantize_q8, quant.quantize_q4)
+    rng = np.random.default_rng(t)
+    x = rng.normal(size=(t, 896)).astype(np.float32)
+    k, v = (rng.normal(size=(2, 2, pos0, 64)).astype(np.float32) for _ in range(2))
+    got = []
+    for planes in (True, False):
+        d = DeviceQwen2(WeightStore(dict(tensors), synth.qwen2_meta(layers=2), quant.QTensor), cap=576)
+        assert d._prompt is not None
+        if not planes:
+            d._prompt = None
+        if pos0:
+            d.fill_cache(k, v)
+        d.prefill(x, pos0)
+        got.append([d.logits.numpy(), d.k_cache.numpy(), d.v_cache.numpy()])
+        assert int(d.ints.numpy()[0]) == pos0 + t - 1
+    for a, b in zip(*got):
+        assert rel_err(a, b) < TOL
+    assert not got[0][1][:, :, pos0 + t:].any() and not got[0][2][:, :, pos0 + t:].any()
