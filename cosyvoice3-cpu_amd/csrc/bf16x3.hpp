@@ -37,4 +37,32 @@ __device__ __forceinline__ void split_x3(const float4& a, const float4& b, uint4
   split_x3(b.z, b.w, hi.w, mid.w, lo.w);
 }
 
+// Scheduling groups: R times, N1 instructions of class M1, then N2 of class M2 (0x8 MFMA, 0x20 VMEM read,
+// 0x100 LDS read).
+template <int M, int N>
+__device__ __forceinline__ void sched_n() {
+  if constexpr (N > 0) __builtin_amdgcn_sched_group_barrier(M, N, 0);
+}
+template <int M1, int N1, int M2, int N2, int R>
+__device__ __forceinline__ void interleave() {
+  if constexpr (R > 0) {
+    sched_n<M1, N1>();
+    sched_n<M2, N2>();
+    interleave<M1, N1, M2, N2, R - 1>();
+  }
+}
+
+// 16 bytes per lane, global -> LDS.  (A function of its own: called inside a kernel template's lambda the
+// builtin makes clang drop the kernel's host stub.)
+__device__ __forceinline__ void dma16(const uint4* g, uint4* l) { __builtin_amdgcn_global_load_lds(g, l, 16, 0, 0); }
+
+typedef float f32x16_t __attribute__((ext_vector_type(16)));
+__device__ __forceinline__ f32x16_t mfma_bf16(const uint4& a, const uint4& b, const f32x16_t& c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c,
+                                                 0, 0, 0);
+}
+
 }  // namespace cv3
+
+// s_waitcnt for at most n vector-memory operations in flight (loads complete in order), others untouched.
+#define CV3_VM(n) (((n) & 0xF) | (((n) >> 4) << 14) | (0x7 << 4) | (0xF << 8))

@@ -30,11 +30,15 @@
 #include "common.hpp"
 #include "epilogue.hpp"
 
+namespace cv3 {
+int split_x3_frag(const float* w, int64_t n, int64_t k, int64_t ldw, uint16_t* frag, hipStream_t st);
+}  // namespace cv3
+
 using namespace cv3;
 
 namespace {
 
-typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef f32x16_t f32x16;
 
 struct PlaneParams {
   const uint4* w;   // weight fragments [planes][nbw][S][64]
@@ -54,6 +58,11 @@ struct PlaneParams {
   float *kc, *vc;
   int heads, kv_heads, cap, pos0;
   const float *cos, *sin;  // [cap][64]
+  // the float32 rows x was split from, or null: an infinity and the largest floats have no planes (inf - inf),
+  // and code products may pass the range before their scale: outputs that come out not finite are formed
+  // again from these
+  const float* fx;
+  int64_t ldfx;
   int tiles_m, tiles_n, gm;
 };
 
@@ -78,27 +87,6 @@ __device__ __forceinline__ void plane_tile(const PlaneParams& p, int& tm, int& t
   tn = o / gh;
 }
 
-__device__ __forceinline__ f32x16 mfma(const uint4& a, const uint4& b, const f32x16& c) {
-  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c,
-                                                 0, 0, 0);
-}
-
-__device__ __forceinline__ void dma16(const uint4* g, uint4* l) { __builtin_amdgcn_global_load_lds(g, l, 16, 0, 0); }
-
-// R times: N1 instructions of class M1, then N2 of class M2 (0x8 MFMA, 0x20 VMEM read, 0x100 LDS read).
-template <int M, int N>
-__device__ __forceinline__ void sched_n() {
-  if constexpr (N > 0) __builtin_amdgcn_sched_group_barrier(M, N, 0);
-}
-template <int M1, int N1, int M2, int N2, int R>
-__device__ __forceinline__ void interleave() {
-  if constexpr (R > 0) {
-    sched_n<M1, N1>();
-    sched_n<M2, N2>();
-    interleave<M1, N1, M2, N2, R - 1>();
-  }
-}
-
 // The products of one 16-k step: hh (of q8: hq) into `big`, the small ones into `small`, each
 // kind over all blocks before the next so no MFMA waits for the one before it.  FIRST starts both
 // sums at zero.
@@ -108,7 +96,7 @@ __device__ __forceinline__ void mma_step(f32x16 (&big)[RM][RN], f32x16 (&small)[
   const f32x16 zero = {0.f};
 #define CV3_PRODUCT(ACC, PW, PX, ZERO)                                                   \
   _Pragma("unroll") for (int i = 0; i < RM; ++i) _Pragma("unroll") for (int j = 0; j < RN; ++j) \
-      ACC[i][j] = mfma(w[j][PW], x[i][PX], (ZERO) ? zero : ACC[i][j]);
+      ACC[i][j] = mfma_bf16(w[j][PW], x[i][PX], (ZERO) ? zero : ACC[i][j]);
   CV3_PRODUCT(big, 0, 0, FIRST)
   if constexpr (KIND == W_F32) {
     CV3_PRODUCT(small, 1, 0, FIRST)
@@ -219,6 +207,29 @@ struct PlaneEpilogue {
     }
   }
 
+  // row m of fx times the weight's outputs n .. n + 3, in float32 (rarely run)
+  __device__ __forceinline__ float4 again(const PlaneParams& p, int mm, int nn, float4 row) const {
+    constexpr int NPW = planes_of(KIND), FOLD = fold_steps(KIND);
+    const uint16_t* w = reinterpret_cast<const uint16_t*>(p.w);
+    float a[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (int k = 0; k < p.S * 16; ++k) {
+      const float x = p.fx[(int64_t)mm * p.ldfx + k];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int r = nn + e;
+        const int64_t at = (((int64_t)(r >> 5) * p.S + (k >> 4)) * 64 + (r & 31) + 32 * ((k >> 3) & 1)) * 8 + (k & 7);
+        float v = 0.f;
+#pragma unroll
+        for (int pl = 0; pl < NPW; ++pl) v += __uint_as_float((uint32_t)w[at + pl * p.wpl * 8] << 16);
+        if constexpr (KIND == W_ROW) v *= e == 0 ? row.x : e == 1 ? row.y : e == 2 ? row.z : row.w;
+        if constexpr (FOLD > 0) v *= p.scales[(int64_t)(k / (16 * FOLD)) * p.nbw * 32 + r];
+        a[e] = fmaf(x, v, a[e]);
+      }
+    }
+    return make_float4(a[0], a[1], a[2], a[3]);
+  }
+
   __device__ __forceinline__ void store_swiglu(const PlaneParams& p, const float4 (&v)[G]) const {
     uint32_t* y = reinterpret_cast<uint32_t*>(p.yp);
 #pragma unroll
@@ -265,6 +276,11 @@ struct PlaneEpilogue {
     for (int q = 0; q < G; ++q) {
       if constexpr (KIND == W_ROW)
         v[q] = make_float4(v[q].x * scale[q].x, v[q].y * scale[q].y, v[q].z * scale[q].z, v[q].w * scale[q].w);
+      if (p.fx) {
+        const float top = 3.4028235e38f;
+        const bool fine = fabsf(v[q].x) <= top && fabsf(v[q].y) <= top && fabsf(v[q].z) <= top && fabsf(v[q].w) <= top;
+        if (!fine && m[q] < p.m && n[q] < p.n) v[q] = again(p, m[q], n[q], scale[q]);
+      }
       if (p.bias) v[q] = make_float4(v[q].x + bias[q].x, v[q].y + bias[q].y, v[q].z + bias[q].z, v[q].w + bias[q].w);
     }
     if constexpr (ACT == A_QKV) return store_qkv(p, v);
@@ -426,8 +442,6 @@ __global__ __launch_bounds__(64 * WK) void k_pg_reg(PlaneParams p) {
 }
 
 // ---- fragments through a ring of LDS stages ----
-#define CV3_VM(n) (((n) & 0xF) | (((n) >> 4) << 14) | (0x7 << 4) | (0xF << 8))
-
 // WM x WN waves of RM x RN blocks.  Stage s (16-k steps 2 s, 2 s + 1) sits in ring slot s % NST.  Per stage:
 //   read the step's second fragments while the first's MFMAs run; wait until the next stage has
 //   landed and every wave has read this one (vmcnt counts this wave's DMAs, which land in order);
@@ -794,7 +808,7 @@ int plane_launch(int kind, int act, PlaneParams& p, const uint16_t* x, int64_t m
 
 int plane_linear(int kind, const uint16_t* x, int64_t m, int64_t k, const uint16_t* w, const float* scales, int64_t n,
                  const float* bias, float* y, int64_t ldy, uint16_t* y_planes, const cv3_epilogue* epi,
-                 int64_t plan_rows, hipStream_t st) {
+                 int64_t plan_rows, hipStream_t st, const float* fx = nullptr, int64_t ldfx = 0) {
   CV3_REQUIRE(!y_planes || n % 16 == 0, CV3_EUNSUPPORTED, "a result in planes needs N %% 16 == 0 (N = %lld)", (long long)n);
   auto a16 = [](const void* q) { return (uintptr_t)q % 16 == 0; };
   PlaneParams p{};
@@ -810,6 +824,8 @@ int plane_linear(int kind, const uint16_t* x, int64_t m, int64_t k, const uint16
   p.ldc = ldy;
   p.yp = reinterpret_cast<uint2*>(y_planes);
   p.ypl = ceil_div(m, 32) * (n / 16) * 128;
+  p.fx = fx;
+  p.ldfx = ldfx;
   return plane_launch(kind, e.act, p, x, m, k, w, scales, n, bias, plan_rows, st);
 }
 
@@ -971,6 +987,35 @@ int cv3_linear_code_planes(const uint16_t* x, int64_t m, int64_t k, const uint16
   if (!m || !n) return CV3_OK;
   return plane_linear(block >= k ? W_ROW : block == 64 ? W_B64 : W_B32, x, m, k, frag, scales_t, n, bias, y, ldy, y_planes, epi,
                       plan_rows, stream_of(s));
+}
+
+// ops.linear on float32 rows: x split into planes in a workspace of the library's allocator, then the plane
+// linear.
+int cv3_linear_rows_planes(int kind, const float* x, int64_t m, int64_t k, int64_t ldx, const uint16_t* frag,
+                           const float* scales_t, int64_t block, int64_t n, const float* bias, float* y, int64_t ldy,
+                           const cv3_epilogue* epi, cv3_stream_t s) {
+  CV3_ALIVE();
+  CV3_REQUIRE(kind == CV3_KIND_F32 || kind == CV3_KIND_Q8 || kind == CV3_KIND_Q4, CV3_EINVAL, "unknown weight kind %d", kind);
+  CV3_REQUIRE(m >= 0 && k > 0 && n >= 0 && ldx >= k && ldy >= n && y && (kind == CV3_KIND_F32 || (scales_t && block > 0)),
+              CV3_EINVAL, "bad linear shape m=%lld k=%lld n=%lld", (long long)m, (long long)k, (long long)n);
+  CV3_REQUIRE(kind == CV3_KIND_F32 || block == 64 || block == 32 || block >= k, CV3_EUNSUPPORTED,
+              "plane codes take 32- or 64-code blocks or one scale a row");
+  CV3_REQUIRE(k % 64 == 0 && (uintptr_t)x % 16 == 0 && ldx % 4 == 0, CV3_EUNSUPPORTED,
+              "rows split into planes need K %% 64 == 0 and 16-byte alignment");
+  if (!m || !n) return CV3_OK;
+  hipStream_t st = stream_of(s);
+  void* ws = nullptr;
+  int rc = cv3_malloc(&ws, (size_t)(6 * ceil_div(m, 32) * 32 * k));
+  if (rc) return rc;
+  if (s) rc = cv3_record_stream(ws, s);
+  uint16_t* planes = reinterpret_cast<uint16_t*>(ws);
+  if (!rc) rc = split_x3_frag(x, m, k, ldx, planes, st);
+  if (!rc) {
+    const int wk = kind == CV3_KIND_F32 ? W_F32 : block >= k ? W_ROW : block == 64 ? W_B64 : W_B32;
+    rc = plane_linear(wk, planes, m, k, frag, scales_t, n, bias, y, ldy, nullptr, epi, 0, st, x, ldx);
+  }
+  const int rf = cv3_free(ws);
+  return rc ? rc : rf;
 }
 
 int cv3_layer_norm_planes(const float* x, uint16_t* planes, int64_t rows, int64_t cols, float eps, const float* shift,

@@ -403,6 +403,14 @@ int cv3_event_elapsed_ms(void* ev0, void* ev1, float* ms) {
   return CV3_OK;
 }
 
+int cv3_stream_capturing(cv3_stream_t s, int* yes) {
+  CV3_REQUIRE(yes, CV3_EINVAL, "null output pointer");
+  hipStream_t st = stream_of(s);
+  CV3_REQUIRE(st, CV3_EHIP, "no stream");
+  *yes = capturing(st);
+  return CV3_OK;
+}
+
 int cv3_graph_begin(cv3_stream_t s) {
   CV3_ALIVE();
   CV3_REQUIRE(g_tls_deferred.empty(), CV3_EINVAL, "a capture is already in progress on this thread");

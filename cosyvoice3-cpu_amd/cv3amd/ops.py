@@ -24,6 +24,7 @@ from .quant import QTensor
 
 Weight = Union[np.ndarray, QTensor]
 TILE_BYTES = 8 << 20  # ops.py:23 (accepted, unused)
+GEMV_ROWS = 4         # cv3_linear_f32 / cv3_linear_q run a GEMV up to here
 
 
 def _dev(x) -> Tuple[DeviceArray, bool]:
@@ -166,6 +167,8 @@ def linear(x, weight: Weight, bias=None):
         if dq.k != k:
             raise ValueError(f"linear: x has {k} features but the weight expects {dq.k}")
         y = DeviceArray(xd.shape[:-1] + (n,), np.float32)
+        if m > GEMV_ROWS and _linear_planes(xd, m, k, weight, dq, n, bd, y):
+            return _ret(y, res)
         _lib.call("linear_q", dq.kind_code, xd.ptr, m, k, k, dq.q.ptr, dq.scales.ptr, dq.scale_code,
                   dq.kp, dq.block, n, bd.ptr if bd is not None else None, y.ptr, n, None, None)
     else:
@@ -174,9 +177,26 @@ def linear(x, weight: Weight, bias=None):
         if wd.size // max(n, 1) != k:
             raise ValueError(f"linear: x has {k} features but the weight is {wd.shape}")
         y = DeviceArray(xd.shape[:-1] + (n,), np.float32)
+        if m > GEMV_ROWS and _linear_planes(xd, m, k, weight, wd, n, bd, y):
+            return _ret(y, res)
         _lib.call("linear_f32", xd.ptr, m, k, k, wd.ptr, k, n, bd.ptr if bd is not None else None,
                   y.ptr, n, None, None)
     return _ret(y, res)
+
+
+def _linear_planes(xd, m, k, weight, dev, n, bd, y) -> bool:
+    """y = x . W^T + bias on the bfloat16 matrix cores, x split into planes on the way, for a cached weight
+    whose planes the device keeps beside it.  More than four rows: up to four are the GEMV's.  The float32
+    kernels walk K serially and run at half the rate: [3000, 1024] x [3072, 1024] q8 196 us, here 94;
+    [40, 4864] x [896, 4864] 120, here 23; [331, 1024] x [2048, 1024] float32 26, here 24 (host)."""
+    if xd.ptr % 16 or (bd is not None and bd.ptr % 16):
+        return False
+    w = _w.device_planes(weight, dev)
+    if w is None:
+        return False
+    _lib.call("linear_rows_planes", w.kind_code, xd.ptr, m, k, k, w.frag.ptr, w.scales_ptr, w.block, n,
+              bd.ptr if bd is not None else None, y.ptr, n, None, None)
+    return True
 
 
 def embedding(table: Weight, ids):

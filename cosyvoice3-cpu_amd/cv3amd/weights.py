@@ -16,6 +16,7 @@ writeable array is re-uploaded on every call because it may change.
 
 from __future__ import annotations
 
+import ctypes
 import threading
 import weakref
 from dataclasses import dataclass
@@ -83,6 +84,67 @@ def device_f32(arr) -> DeviceArray:
             hit = _CACHE.get(id(arr))
             return hit if hit is not None else _remember(arr, to_device(arr, np.float32))
     return to_device(np.asarray(arr), np.float32)
+
+
+@dataclass
+class DevicePlanes:
+    """A linear weight laid out for ``cv3_linear_rows_planes``."""
+    kind_code: int
+    frag: DeviceArray
+    scales_ptr: Optional[int]
+    block: int
+    scales: Optional[DeviceArray] = None
+
+
+def device_planes(weight, dev) -> Optional[DevicePlanes]:
+    """The matrix cores' layout of a weight whose device copy is ``dev`` (a DeviceArray or DeviceQ), made
+    beside that copy on first use and kept and released with it.  None for what the plane linear does not
+    take, for K up to 512 (two launches: 10.7 us against 8.6 of the one float32 kernel at K = 256, within 15 %
+    of each other either way at 512, 13.5 against 21.5 at 1024, whatever m; q8 more), for a first use inside
+    a capture (packing waits for the device), and for weights that are not cached: a writeable array, or one
+    that lives on the device (its owner may write to it between calls)."""
+    quantised = isinstance(dev, DeviceQ)
+    if quantised:
+        cached = not isinstance(weight.q, DeviceArray) and not isinstance(weight.scales, DeviceArray)
+        n, k, block = dev.n, dev.k, dev.block
+        cached = cached and (block in (32, 64) or block >= k) and dev.kp % 16 == 0
+    else:
+        cached = isinstance(weight, np.ndarray) and not weight.flags.writeable and weight.ndim == 2
+        n, k = (dev.shape if cached else (0, 1))
+        block = k
+    if not cached or k % 64 or n % 4 or not n or k <= 512:
+        return None
+    key = ("planes", id(weight))
+    hit = _CACHE.get(key)
+    if hit is not None:
+        return hit
+    with _UPLOAD:
+        hit = _CACHE.get(key)
+        if hit is None:
+            capturing = ctypes.c_int()
+            _lib.call("stream_capturing", None, ctypes.addressof(capturing))
+            if capturing.value:
+                return None
+            hit = _CACHE[key] = _pack_planes(dev, n, k, block)
+            weakref.finalize(weight, _CACHE.pop, key, None)
+    return hit
+
+
+def _pack_planes(dev, n: int, k: int, block: int) -> DevicePlanes:
+    ne, ns = ctypes.c_int64(), ctypes.c_int64()
+    if isinstance(dev, DeviceQ):
+        _lib.call("code_planes_elems", n, k, block, ctypes.addressof(ne), ctypes.addressof(ns))
+        frag, scales = DeviceArray((ne.value,), np.uint16), DeviceArray((ns.value,))
+        _lib.call("pack_code_planes", dev.kind_code, dev.q.ptr, n, k, dev.scales.ptr, dev.scale_code, dev.kp, block, 0,
+                  0, frag.ptr, scales.ptr, None)
+        out = DevicePlanes(dev.kind_code, frag, scales.ptr, block, scales)
+    else:
+        _lib.call("x3_frag_elems", n, k, ctypes.addressof(ne))
+        frag = DeviceArray((ne.value,), np.uint16)
+        _lib.call("split_x3_frag", dev.ptr, n, k, k, frag.ptr, None)
+        out = DevicePlanes(_lib.KIND_F32, frag, None, k)
+    _lib.call("stream_sync", None)   # another thread's stream may read it next
+    return out
 
 
 class WeightStore:

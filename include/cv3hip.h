@@ -93,6 +93,7 @@ int cv3_event_record(void* ev, cv3_stream_t s);
  * orders work across streams, e.g. vocoder windows run side by side). */
 int cv3_stream_wait_event(cv3_stream_t s, void* ev);
 int cv3_event_elapsed_ms(void* ev0, void* ev1, float* ms);
+int cv3_stream_capturing(cv3_stream_t s, int* yes);   /* 1 between cv3_graph_begin and cv3_graph_end */
 int cv3_graph_begin(cv3_stream_t s);
 int cv3_graph_end(cv3_stream_t s, void** exec);
 int cv3_graph_launch(void* exec, cv3_stream_t s);
@@ -202,6 +203,12 @@ int cv3_pack_code_planes(int kind, const void* q, int64_t n, int64_t k, const vo
 int cv3_linear_code_planes(const uint16_t* x, int64_t m, int64_t k, const uint16_t* frag, const float* scales_t,
                            int64_t block, int64_t n, const float* bias, float* y, int64_t ldy, uint16_t* y_planes,
                            const cv3_epilogue* epi, int64_t plan_rows, cv3_stream_t s);
+/* ops.linear (ops.py:121-123, quant.py:156-204) on float32 rows with such a weight: x is split into planes in a
+ * workspace of the caching allocator, then multiplied as above.  kind: the weight's (float32 planes of
+ * cv3_split_x3_frag, or codes).  Rows with infinities give what float32 products of them give. */
+int cv3_linear_rows_planes(int kind, const float* x, int64_t m, int64_t k, int64_t ldx, const uint16_t* frag,
+                           const float* scales_t, int64_t block, int64_t n, const float* bias, float* y, int64_t ldy,
+                           const cv3_epilogue* epi, cv3_stream_t s);
 /* AdaLN (dit.py:168-169) and RMSNorm (ops.py:101-104) whose result is [rows, cols] planes in fragment
  * order; cols a multiple of 16, at most 1024, 16-byte aligned operands. */
 int cv3_layer_norm_planes(const float* x, uint16_t* planes, int64_t rows, int64_t cols, float eps, const float* shift,

@@ -193,3 +193,68 @@ def test_prompt_on_code_planes(gpu, profile, t, pos0):
     for a, b in zip(*got):
         assert rel_err(a, b) < TOL
     assert not got[0][1][:, :, pos0 + t:].any() and not got[0][2][:, :, pos0 + t:].any()
+
+
+@pytest.mark.parametrize("kind", ["f32", "q8_rows", "q8_block", "q4"])
+@pytest.mark.parametrize("m,k,n", [(5, 576, 64), (33, 896, 1152), (130, 1024, 68), (331, 1024, 2048), (40, 4864, 896)])
+def test_drop_in_linear_on_planes(lib, m, k, n, kind):
+    """ops.linear with a cached weight against float64, and rows with an infinity, a NaN and the largest
+    float against the float32 kernels (a weight that lives on the device keeps those)."""
+    import cv3amd.ops as ops
+    import cv3amd.quant as quant
+    _lib, to_device, empty = lib
+    rng = np.random.default_rng([m, k, n])
+    x, w = rng.normal(size=(m, k)).astype(np.float32), (0.02 * rng.normal(size=(n, k))).astype(np.float32)
+    b = rng.normal(size=n).astype(np.float32)
+    w[w == 0] = 0.01
+    if kind == "f32":
+        w.flags.writeable = False
+        wc, wd, w64 = w, to_device(w), w.astype(np.float64)
+    else:
+        if kind == "q4":
+            q, s, _ = quant.quantize_q4(w)
+            block = 32
+        else:
+            block = 64 if kind == "q8_block" else k
+            q, s, _ = quant.quantize_q8(w, block, np.float16 if kind == "q8_block" else np.float32)
+        name = "q4" if kind == "q4" else "q8"
+        wc = quant.QTensor(name, q, s, (n, k), block)
+        wd = quant.QTensor(name, to_device(q), to_device(s), (n, k), block)
+        w64 = wc.dequant().astype(np.float64)
+    assert rel_err(ops.linear(x, wc, b), x.astype(np.float64) @ w64.T + b) < TOL
+    x[1, 3], x[2, 5], x[3, 7], x[4, k - 1] = np.inf, -np.inf, np.nan, np.finfo(np.float32).max
+    got, want = ops.linear(to_device(x), wc, b).numpy(), ops.linear(to_device(x), wd, b).numpy()
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
+    np.testing.assert_array_equal(np.isinf(got), np.isinf(want))
+    ok = np.isfinite(want)
+    assert np.array_equal(got[np.isinf(want)], want[np.isinf(want)])
+    for r in range(m):
+        if ok[r].any():
+            assert np.abs(got[r] - want[r])[ok[r]].max() <= TOL * np.abs(want[r][ok[r]]).max()
+
+
+def test_drop_in_linear_first_used_in_a_capture(lib):
+    """A weight that a capture meets first keeps the float32 kernel there; its planes come with the next
+    eager call, and both give the same layer."""
+    import cv3amd.ops as ops
+    from cv3amd.device import Graph
+    _lib, to_device, empty = lib
+    rng = np.random.default_rng(4)
+    w = (0.02 * rng.normal(size=(96, 640))).astype(np.float32)
+    w.flags.writeable = False
+    x = to_device(rng.normal(size=(40, 640)).astype(np.float32))
+    ops.linear(x.rows(0, 2), w)   # the weight is on the device, its planes are not
+    out = []
+    with Graph() as g:
+        out.append(ops.linear(x, w))
+    g.launch()
+    assert rel_err(out[0].numpy(), x.numpy().astype(np.float64) @ w.T.astype(np.float64)) < TOL
+    eager = ops.linear(x, w)
+    assert rel_err(eager.numpy(), x.numpy().astype(np.float64) @ w.T.astype(np.float64)) < TOL
+    with Graph() as h:
+        out.append(ops.linear(x, w))
+    for r in range(3):
+        x.copy_from(rng.normal(size=(40, 640)).astype(np.float32))
+        want = ops.linear(x, w).numpy()
+        h.launch()
+        np.testing.assert_array_equal(out[1].numpy(), want)
