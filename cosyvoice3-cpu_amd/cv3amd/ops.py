@@ -327,10 +327,7 @@ def sdpa(q, k, v, mask_spec=None, scale: Optional[float] = None, tile_bytes: int
     if scale is None:
         scale = 1.0 / math.sqrt(d)
     out = DeviceArray((h, n, d), np.float32)
-    S = ctypes.c_int64 * 3
-    _lib.call("attention", qd.ptr, kd.ptr, vd.ptr, out.ptr, 1, h, hk, n, m, d,
-              S(0, n * d, d), S(0, m * d, d), S(0, m * d, d), S(0, n * d, d),
-              float(np.float32(scale)), mk, ma, mb, None)
+    _lib.call("sdpa", qd.ptr, kd.ptr, vd.ptr, out.ptr, h, hk, n, m, d, float(np.float32(scale)), mk, ma, mb, None)
     return _ret(out, res)
 
 

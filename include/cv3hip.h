@@ -285,6 +285,11 @@ int cv3_attention_x3(const float* q, const float* k, const float* v, float* out,
                      int64_t n, int64_t m, int d, const int64_t* q_strides, const int64_t* k_strides,
                      const int64_t* v_strides, const int64_t* o_strides, float scale, int mask_kind,
                      int64_t mask_a, int64_t mask_b, cv3_stream_t s);
+/* ops.sdpa itself: contiguous (h, n, d) and (hk, m, d), as cv3_attention_x3.  Outputs that come out not finite
+ * are formed again in float32, so infinities give what float32 products of them give; keys that no query of a
+ * tile sees are not read. */
+int cv3_sdpa(const float* q, const float* k, const float* v, float* out, int h, int hk, int64_t n, int64_t m, int d,
+             float scale, int mask_kind, int64_t mask_a, int64_t mask_b, cv3_stream_t s);
 /* cv3_attention_x3 with the output [batch * n, 64 h] as bfloat16 planes in fragment order, for the plane
  * linear that reads it (d == 64, 16-byte aligned rows). */
 int cv3_attention_x3_planes(const float* q, const float* k, const float* v, uint16_t* out_planes, int64_t batch, int h,

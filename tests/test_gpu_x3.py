@@ -627,3 +627,47 @@ def test_dit_digits_switch(lib, monkeypatch):
         print(f"[dit-digits] digits={digits} T={T}", flush=True)
         outs.append(d.solve(x0).numpy().copy())
     assert rel_err(outs[1], outs[0]) < 1e-5
+
+
+SDPA_MASKS = [None, ("causal", 0), ("causal", 70), ("causal", -3), ("chunk", 25, 1), ("chunk", 40, -1), ("chunk", 50, 0)]
+
+
+@pytest.mark.parametrize("mask", SDPA_MASKS, ids=str)
+@pytest.mark.parametrize("h,hk,n,m", [(2, 1, 1, 1), (14, 2, 33, 37), (16, 16, 129, 129), (14, 2, 333, 403), (14, 2, 700, 700)])
+def test_sdpa_tiles_and_masks(lib, h, hk, n, m, mask):
+    """Both query tiles (32 and 64) and the skipped stages of every mask against the oracle, with an
+    infinity, a NaN or a float near the largest in a query, a key or a value, over the queries that see it."""
+    import cv3amd.ops as ops
+    _lib, to_device, _ = lib
+    rng = np.random.default_rng([h, n, m])
+    q, k, v = (rng.normal(size=s).astype(np.float32) for s in ((h, n, 64), (hk, m, 64), (hk, m, 64)))
+
+    def f32(q, k, v):
+        with np.errstate(all="ignore"):
+            return ref.sdpa(q, k, v, mask)
+
+    def seen(j):
+        i = np.arange(n)
+        if mask is None:
+            return i >= 0
+        if mask[0] == "causal":
+            return j <= i + mask[1]
+        c = i // mask[1]
+        return (j < (c + 1) * mask[1]) & ((mask[2] < 0) | (j >= (c - mask[2]) * mask[1]))
+
+    got, want = ops.sdpa(q, k, v, mask), f32(q, k, v)
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
+    ok = ~np.isnan(want)
+    if ok.any():
+        assert np.abs(got - want)[ok].max() <= 2e-6 * max(1.0, np.abs(want[ok]).max())
+    for where, value in ((0, np.inf), (1, -np.inf), (2, np.inf), (2, np.nan), (1, 3.4e38)):
+        a = [q.copy(), k.copy(), v.copy()]
+        j = (n if where == 0 else m) // 2
+        a[where][0, j, 5] = value
+        got, want = ops.sdpa(*a, mask), f32(*a)
+        rows = np.ones(n, bool) if where == 0 else seen(j)
+        g, w = got[:, rows], want[:, rows]
+        np.testing.assert_array_equal(np.isnan(g), np.isnan(w))
+        np.testing.assert_array_equal(g[np.isinf(w)], w[np.isinf(w)])
+        ok = np.isfinite(w)
+        assert not ok.any() or np.abs(g - w)[ok].max() <= 2e-6 * max(1.0, np.abs(w[ok]).max())
