@@ -82,6 +82,11 @@ static bool capturing(hipStream_t st) {
 // allocation from a different stream waits for all of them, so a block is never
 // handed out while a kernel on any of its streams may still touch it.
 //
+// A block freed on its home stream and used on no other records nothing (an event is a
+// packet of its own between two kernels: a linear call of 1 row 10.1 us with, 8.3 without,
+// of 331 float32 rows 24.3 and 15.9, sdpa over 333 rows 15.0 and 12.0): its home takes it again in stream order, any other
+// stream only once the home has nothing left to do.
+//
 // Graph capture: a block freed while the freeing thread's stream is capturing is
 // still referenced by the graph being built.  It stays allocated and belongs to
 // that graph from cv3_graph_end on; cv3_graph_destroy returns it to the cache
@@ -96,6 +101,7 @@ struct Block {
   std::vector<hipStream_t> users;                          // streams besides home
   std::vector<hipEvent_t> events;                          // event pool, grows to #streams
   std::vector<std::pair<hipStream_t, hipEvent_t>> pending;  // recorded at the last free
+  bool quiet = false;  // last freed on its home stream, used on no other: no event was recorded
 };
 
 static std::multimap<size_t, void*> g_free;            // size class -> ptr
@@ -150,6 +156,15 @@ static int release_locked(void* ptr, Block& b, const std::vector<hipStream_t>& s
   return CV3_OK;
 }
 
+// Whether a thread's stream has nothing left to do.  Never asks a stream under capture (cv3_graph_begin holds
+// g_mu, as the callers do).
+static bool idle(hipStream_t s) {
+  if (capturing(s)) return false;
+  const bool yes = hipStreamQuery(s) == hipSuccess;
+  if (!yes) (void)hipGetLastError();
+  return yes;
+}
+
 static void add_stream(std::vector<hipStream_t>& v, hipStream_t s) {
   for (hipStream_t x : v)
     if (x == s) return;
@@ -201,7 +216,7 @@ int cv3_malloc(void** ptr, size_t bytes) {
     for (auto it = range.first; it != range.second; ++it) {
       void* p = it->second;
       Block& b = g_blocks[p];
-      bool ok = true;
+      bool ok = !b.quiet || b.home == cur || (!cap && idle(b.home));
       if (cap)
         for (auto& pe : b.pending) ok = ok && pe.first == cur;
       if (!ok) continue;
@@ -209,6 +224,7 @@ int cv3_malloc(void** ptr, size_t bytes) {
         if (pe.first != cur) CV3_HIP(hipStreamWaitEvent(cur, pe.second, 0));
       g_free.erase(it);
       b.pending.clear();
+      b.quiet = false;
       b.home = cur;
       b.users.clear();
       g_cached -= sz;
@@ -227,7 +243,7 @@ int cv3_malloc(void** ptr, size_t bytes) {
   }
   if (e != hipSuccess) return fail(CV3_EHIP, "hipMalloc(%zu) failed: %s", sz, hipGetErrorString(e));
   std::lock_guard<std::mutex> lk(g_mu);
-  g_blocks[p] = Block{sz, cur, {}, {}, {}};
+  g_blocks[p] = Block{sz, cur, {}, {}, {}, false};
   g_in_use += sz;
   *ptr = p;
   return CV3_OK;
@@ -257,6 +273,14 @@ int cv3_free(void* ptr) {
   auto it = g_blocks.find(ptr);
   CV3_REQUIRE(it != g_blocks.end(), CV3_EINVAL, "cv3_free of a pointer not from cv3_malloc");
   Block& b = it->second;
+  if (cur == b.home && b.users.empty()) {
+    b.pending.clear();
+    b.quiet = true;
+    g_free.emplace(b.size, ptr);
+    g_in_use -= b.size;
+    g_cached += b.size;
+    return CV3_OK;
+  }
   std::vector<hipStream_t> streams{b.home};
   for (hipStream_t u : b.users) add_stream(streams, u);
   add_stream(streams, cur);
@@ -414,7 +438,9 @@ int cv3_stream_capturing(cv3_stream_t s, int* yes) {
 int cv3_graph_begin(cv3_stream_t s) {
   CV3_ALIVE();
   CV3_REQUIRE(g_tls_deferred.empty(), CV3_EINVAL, "a capture is already in progress on this thread");
-  CV3_HIP(hipStreamBeginCapture(stream_of(s), hipStreamCaptureModeThreadLocal));
+  hipStream_t st = stream_of(s);
+  std::lock_guard<std::mutex> lk(g_mu);   // against idle()
+  CV3_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
   return CV3_OK;
 }
 

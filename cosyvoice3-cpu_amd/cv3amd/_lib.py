@@ -71,6 +71,7 @@ def parse_header(path: str = HEADER):
 # re-entrant: init() holds it while its call() loads the library through lib()
 _lock = threading.RLock()
 _lib = None
+_entries = {}   # entry points by short name, looked up once
 _inited = False
 _shut = False
 
@@ -116,7 +117,9 @@ def call(name: str, *args):
     must not enqueue work)."""
     if _shut:
         raise RuntimeError(f"cv3_{name}: the library has been shut down")
-    fn = getattr(lib(), "cv3_" + name)
+    fn = _entries.get(name)
+    if fn is None:
+        fn = _entries[name] = getattr(lib(), "cv3_" + name)
     rc = fn(*args)
     if rc:
         _raise(rc, "cv3_" + name)

@@ -9,6 +9,7 @@ stream, so work on one thread is ordered without explicit synchronisation.
 from __future__ import annotations
 
 import ctypes
+import math
 from typing import Optional, Sequence
 
 import numpy as np
@@ -25,16 +26,18 @@ class _Block:
     __slots__ = ("ptr", "nbytes")
 
     def __init__(self, nbytes: int):
-        _lib.init()
+        if not _lib._inited:
+            _lib.init()
         p = ctypes.c_void_p()
-        _lib.call("malloc", ctypes.addressof(p), max(1, int(nbytes)))
+        nbytes = int(nbytes)
+        _lib.call("malloc", ctypes.addressof(p), nbytes or 1)
         self.ptr = p.value
-        self.nbytes = int(nbytes)
+        self.nbytes = nbytes
 
     def __del__(self):
         try:
             if self.ptr and _lib._lib is not None:
-                _lib.lib().cv3_free(ctypes.c_void_p(self.ptr))
+                _lib._lib.cv3_free(self.ptr)
         except Exception:
             pass
         self.ptr = None
@@ -47,17 +50,18 @@ class DeviceArray:
 
     def __init__(self, shape: Sequence[int], dtype=np.float32, block: Optional[_Block] = None,
                  offset: int = 0):
-        self.shape = tuple(int(s) for s in shape)
-        self.dtype = np.dtype(dtype)
-        if self.dtype not in _DTYPES:
-            raise TypeError(f"unsupported device dtype {self.dtype}")
-        self._block = block if block is not None else _Block(self.nbytes)
+        # on every call's path: plain integers rather than NumPy's scalars and reductions (2 us a call)
+        self.shape = shape = tuple(map(int, shape))
+        self.dtype = dtype = np.dtype(dtype)
+        if dtype not in _DTYPES:
+            raise TypeError(f"unsupported device dtype {dtype}")
+        self._block = block if block is not None else _Block(math.prod(shape) * dtype.itemsize)
         self.offset = int(offset)
 
     # -- basic properties ------------------------------------------------
     @property
     def size(self) -> int:
-        return int(np.prod(self.shape)) if self.shape else 1
+        return math.prod(self.shape)
 
     @property
     def nbytes(self) -> int:
@@ -84,9 +88,9 @@ class DeviceArray:
         shape = list(shape)
         if -1 in shape:
             i = shape.index(-1)
-            rest = int(np.prod([s for j, s in enumerate(shape) if j != i])) or 1
+            rest = int(math.prod([s for j, s in enumerate(shape) if j != i])) or 1
             shape[i] = self.size // rest
-        if int(np.prod(shape)) != self.size:
+        if int(math.prod(shape)) != self.size:
             raise ValueError(f"cannot reshape {self.shape} to {tuple(shape)}")
         return DeviceArray(shape, self.dtype, self._block, self.offset)
 
@@ -100,7 +104,7 @@ class DeviceArray:
         """Sub-view starting ``elem_offset`` elements in (no bounds growth allowed)."""
         dt = np.dtype(dtype) if dtype is not None else self.dtype
         off = self.offset + elem_offset * self.dtype.itemsize
-        n = int(np.prod(shape)) * dt.itemsize
+        n = int(math.prod(shape)) * dt.itemsize
         if off < 0 or off + n > self._block.nbytes:
             raise ValueError("view exceeds the allocation")
         return DeviceArray(shape, dt, self._block, off)

@@ -188,7 +188,7 @@ def _linear_planes(xd, m, k, weight, dev, n, bd, y) -> bool:
     """y = x . W^T + bias on the bfloat16 matrix cores, x split into planes on the way, for a cached weight
     whose planes the device keeps beside it.  More than four rows: up to four are the GEMV's.  The float32
     kernels walk K serially and run at half the rate: [3000, 1024] x [3072, 1024] q8 196 us, here 94;
-    [40, 4864] x [896, 4864] 120, here 23; [331, 1024] x [2048, 1024] float32 26, here 24 (host)."""
+    [40, 4864] x [896, 4864] 120, here 23; [331, 1024] x [2048, 1024] float32 25, here 16."""
     if xd.ptr % 16 or (bd is not None and bd.ptr % 16):
         return False
     w = _w.device_planes(weight, dev)

@@ -104,3 +104,38 @@ def test_record_stream_orders_reuse(gpu):
         synchronize()
         assert float(dst.numpy().min()) == 7.0
         del over, dst
+
+
+def test_block_freed_at_home_waits_for_its_stream(gpu):
+    """A block freed on the one stream that used it goes back to that stream at once, and to another
+    thread's stream only when the first has run dry."""
+    import cv3amd.ops as ops
+    from cv3amd.device import DeviceArray, synchronize, to_device
+    nbytes = 37 << 20   # a size class of its own
+    rng = np.random.default_rng(2)
+    x = to_device(rng.normal(size=(3000, 1024)).astype(np.float32))
+    w = rng.normal(size=(4096, 1024)).astype(np.float32)
+    w.flags.writeable = False
+    ops.linear(x, w)
+    synchronize()
+
+    def fresh():
+        a = DeviceArray((nbytes,), np.uint8)
+        return a, a.ptr
+
+    with ThreadPoolExecutor(1) as other:
+        other.submit(lambda: DeviceArray((16,))).result()   # the other thread's stream exists
+        a, ptr = fresh()
+        for _ in range(200):     # some 20 ms of work
+            y = ops.linear(x, w)
+        a.zero_()
+        del a
+        a, again = fresh()
+        assert again == ptr
+        del a
+        b, elsewhere = other.submit(fresh).result()
+        assert elsewhere != ptr
+        synchronize()
+        c, late = other.submit(fresh).result()
+        assert late == ptr
+        del b, c, y
