@@ -927,6 +927,251 @@ int norm_planes(bool rms, const float* x, uint16_t* planes, int64_t rows, int64_
   return CV3_OK;
 }
 
+// ---- the vocoder's causal convolutions on planes ----
+// y[t] = bias + sum_tap W_tap x[t - (taps - 1 - tap) dil] over channels-last rows: a plane linear of
+// K = taps C whose activation fragment of a step is the channel step's, read some rows up.  The producer
+// has already applied Snake and split, once per element instead of once per tap and column tile.  Then,
+// in the order of the reference: bias, residual, the float rows, and Snake of them as the next conv's
+// planes.
+// K is split over eight waves as in k_pg_reg.  The tile's rows and their halo go to LDS once (by passes over
+// the channels where they exceed it) and every tap reads them there, so only the weight's fragments stream
+// from L2: 3 KB against 6 RM products a step.  Few registers (two workgroups to a CU) beat a deep ring:
+// 32-row tiles with four stages 9.6 us, with twelve 11.0.  What bounds it at a second of mel is latency: 5 to
+// 6 us of a launch of 7 (k = 3) to 13 us (k = 11) go to the first fetch, the sum over waves and the launch.
+// A resblock step of the 256-channel stage over 440 rows, k = 7: 41 us in five launches before, 21 in two.
+struct ConvPlaneParams {
+  const uint4 *x, *w;
+  int64_t xpl, wpl;   // 16-byte fragments per plane
+  uint32_t xbytes;
+  int S, SC, SP, taps, dil;  // 16-k steps in all, per tap, and per tap and pass (SC / SP passes over channels)
+  int m, n, nbx, nbw;
+  const float *bias, *res, *alpha;
+  float eps;
+  float* y;
+  uint2* yp;
+  int64_t ypl;
+  int tiles_m, tiles_n, cx, rows_x, cols_x;  // XCD x: cols_x columns from x % cx, rows_x rows from x / cx
+};
+
+__device__ __forceinline__ float snake(float v, float a, float eps) {
+  const float s = sinf(a * v);
+  return v + (1.0f / (a + eps)) * (s * s);
+}
+
+// 16 bytes per lane, global -> LDS, zeros past the descriptor's bound
+__device__ __forceinline__ void buffer_dma16(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint4* l) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, l, 16, (int)voff, 0, 0, 0);
+}
+
+template <int RM, int PF, int XB>
+__global__ __launch_bounds__(512, 4) void k_conv_planes(ConvPlaneParams p) {
+  constexpr int WK = 8, RN = 1;
+  static_assert(PF % XB == 0, "the x registers alternate within a turn of the weight ring");
+  // x of the tile and pass, [plane][channel step][half][row], 16 bytes each; then the waves' partial sums
+  extern __shared__ uint4 xs[];
+  float4(*red)[RM * RN * 4 * 64] = reinterpret_cast<float4(*)[RM * RN * 4 * 64]>(xs);
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), h = lane >> 5;
+  const int xcd = blockIdx.x & 7, at_x = blockIdx.x >> 3;
+  const int tm = xcd / p.cx * p.rows_x + at_x / p.cols_x, tn = xcd % p.cx * p.cols_x + at_x % p.cols_x;
+  if (tm >= p.tiles_m || tn >= p.tiles_n) return;
+  const int steps = p.taps * p.SP, s0 = steps * wave / WK, s1 = steps * (wave + 1) / WK;  // of each pass
+  const int start = max(min(s0, s1 - 1), 0), tap0 = start / p.SP, cs0 = start - tap0 * p.SP;
+  const uint4* wp = p.w + (int64_t)tn * p.S * 64 + lane;
+  f32x16 big[RM][RN], small[RM][RN];
+#pragma unroll
+  for (int i = 0; i < RM; ++i) big[i][0] = small[i][0] = f32x16{0.f};
+  uint4 bx[XB][RM][3], bw[PF][RN][3];
+  // rows first .. first + R - 1 of x; those before 0 and past the tensor's blocks are zeros by the bound
+  const int halo = (p.taps - 1) * p.dil, R = 32 * RM + halo, first = tm * RM * 32 - halo;
+  const __amdgpu_buffer_rsrc_t xr =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<uint4*>(p.x), (short)0, (int)p.xbytes, 0x00027000);
+  const int cols = 2 * p.SP, total = 3 * cols * R, dcol = 512 / R, drow = 512 - dcol * R;
+  for (int c0 = 0; c0 < p.SC; c0 += p.SP) {
+    // the weight's next step: past the wave's last it stays there (an empty range: at one before it)
+    int sn = start, wtap = tap0, wcs = cs0;
+    auto load = [&](int buf) {
+      const int64_t at = (int64_t)(wtap * p.SC + c0 + wcs) * 64;
+#pragma unroll
+      for (int pl = 0; pl < 3; ++pl) bw[buf][0][pl] = wp[pl * p.wpl + at];
+      if (sn + 1 < s1) {
+        ++sn;
+        if (++wcs == p.SP) {
+          wcs = 0;
+          ++wtap;
+        }
+      }
+    };
+#pragma unroll
+    for (int j = 0; j < PF - 1; ++j) load(j);
+    if (c0) __syncthreads();  // every wave has read the pass before
+    int col = threadIdx.x / R, r = threadIdx.x - col * R;
+    for (int i = threadIdx.x; i < total; i += 512) {
+      const int g = first + r, pl = col / cols, ch = col - pl * cols;
+      const uint32_t at = (uint32_t)(pl * p.xpl + (int64_t)((g >> 5) * p.SC + c0 + (ch >> 1)) * 64 + 32 * (ch & 1) +
+                                     (g & 31)) * 16u;
+      buffer_dma16(xr, g < 0 || g >= 32 * p.nbx ? 0x80000000u : at, xs + i - lane);
+      col += dcol;
+      r += drow;
+      if (r >= R) {
+        r -= R;
+        ++col;
+      }
+    }
+    __builtin_amdgcn_s_waitcnt(CV3_VM(0));
+    __syncthreads();
+    int tap = tap0, cs = cs0;  // the next step of x
+    auto read = [&](int buf) {
+      const uint4* from = xs + (cs * 2 + h) * R + (lane & 31) + tap * p.dil;
+#pragma unroll
+      for (int pl = 0; pl < 3; ++pl)
+#pragma unroll
+        for (int i = 0; i < RM; ++i) bx[buf][i][pl] = from[pl * cols * R + 32 * i];
+      if (++cs == p.SP) {
+        cs = 0;
+        tap = min(tap + 1, p.taps - 1);
+      }
+    };
+    if constexpr (XB == 2) read(0);
+    __builtin_amdgcn_sched_barrier(0);
+    for (int s = s0; s < s1; s += PF) {
+#pragma unroll
+      for (int j = 0; j < PF; ++j) {
+        if (s + j < s1) {
+          load((j + PF - 1) % PF);
+          read((j + 1) % XB);
+          mma_step<W_F32, RM, RN, false>(big, small, bx[j % XB], bw[j]);
+          if constexpr (XB == 2) {
+            interleave<0x100, 1, 0x8, 1, 3 * RM>();
+            interleave<0x20, 1, 0x8, 1, 3>();
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+    }
+  }
+  __syncthreads();  // every wave has read its x
+  // the waves' partial sums meet in LDS, in wave order; each wave finishes its share of the groups
+  constexpr int GROUPS = RM * RN * 4, G = GROUPS > WK ? GROUPS / WK : 1;
+  int m[G], n[G];
+  float4 bias[G], res[G], alpha[G];
+#pragma unroll
+  for (int q = 0; q < G; ++q) {
+    const int id = min(wave * G + q, GROUPS - 1), blk = id >> 2;
+    m[q] = (tm * RM + blk / RN) * 32 + (lane & 31);
+    n[q] = (tn * RN + blk % RN) * 32 + 8 * (id & 3) + 4 * h;
+    const int mm = min(m[q], p.m - 1), nn = min(n[q], p.n - 4);
+    bias[q] = *reinterpret_cast<const float4*>(p.bias + nn);
+    if (p.res) res[q] = *reinterpret_cast<const float4*>(p.res + (int64_t)mm * p.n + nn);
+    if (p.yp) alpha[q] = *reinterpret_cast<const float4*>(p.alpha + nn);
+  }
+#pragma unroll
+  for (int i = 0; i < RM; ++i)
+#pragma unroll
+    for (int j = 0; j < RN; ++j)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        float o[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = big[i][j][4 * g + e] + small[i][j][4 * g + e];
+        red[wave][((i * RN + j) * 4 + g) * 64 + lane] = make_float4(o[0], o[1], o[2], o[3]);
+      }
+  __syncthreads();
+  if (wave * G >= GROUPS) return;  // more waves than groups: the first ones finish
+#pragma unroll
+  for (int q = 0; q < G; ++q) {
+    const int id = wave * G + q;
+    float4 v = red[0][id * 64 + lane];
+#pragma unroll
+    for (int u = 1; u < WK; ++u) {
+      const float4 t = red[u][id * 64 + lane];
+      v = make_float4(v.x + t.x, v.y + t.y, v.z + t.z, v.w + t.w);
+    }
+    if (m[q] >= p.m || n[q] >= p.n) continue;
+    v = make_float4(v.x + bias[q].x, v.y + bias[q].y, v.z + bias[q].z, v.w + bias[q].w);
+    if (p.res) v = make_float4(res[q].x + v.x, res[q].y + v.y, res[q].z + v.z, res[q].w + v.w);
+    if (p.y) *reinterpret_cast<float4*>(p.y + (int64_t)m[q] * p.n + n[q]) = v;
+    if (p.yp) {
+      uint2 hi, mid, lo;
+      split_x3(snake(v.x, alpha[q].x, p.eps), snake(v.y, alpha[q].y, p.eps), hi.x, mid.x, lo.x);
+      split_x3(snake(v.z, alpha[q].z, p.eps), snake(v.w, alpha[q].w, p.eps), hi.y, mid.y, lo.y);
+      const int64_t at =
+          (((int64_t)(m[q] >> 5) * (p.n >> 4) + (n[q] >> 4)) * 64 + (m[q] & 31) + 32 * ((n[q] >> 3) & 1)) * 2 +
+          ((n[q] >> 2) & 1);
+      p.yp[at] = hi;
+      p.yp[at + p.ypl] = mid;
+      p.yp[at + 2 * p.ypl] = lo;
+    }
+  }
+}
+
+// Snake of x (+ add, kept in sum) with up to three alphas, each as planes: one pass where a resblock
+// group forks.  A thread owns eight channels of a row, the 16 bytes of each plane.
+struct SnakePlanes {
+  const float* alpha[3];
+  uint4* planes[3];
+};
+
+__global__ __launch_bounds__(256) void k_snake_planes(const float* x, const float* add, float* sum, int64_t t, int c,
+                                                      float eps, int count, SnakePlanes o, int64_t per_plane) {
+  const int SC = c / 16;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < per_plane;
+       i += (int64_t)gridDim.x * blockDim.x) {
+    const int l = (int)(i & 63);
+    const int64_t b = (i >> 6) / SC;
+    const int k0 = 16 * (int)((i >> 6) - b * SC) + 8 * (l >> 5);
+    const int64_t row = b * 32 + (l & 31);
+    float4 u = make_float4(0.f, 0.f, 0.f, 0.f), v = u;
+    if (row < t) {
+      const int64_t at = row * c + k0;
+      u = *reinterpret_cast<const float4*>(x + at);
+      v = *reinterpret_cast<const float4*>(x + at + 4);
+      if (add) {
+        const float4 a = *reinterpret_cast<const float4*>(add + at), d = *reinterpret_cast<const float4*>(add + at + 4);
+        u = make_float4(u.x + a.x, u.y + a.y, u.z + a.z, u.w + a.w);
+        v = make_float4(v.x + d.x, v.y + d.y, v.z + d.z, v.w + d.w);
+      }
+      if (sum) {
+        *reinterpret_cast<float4*>(sum + at) = u;
+        *reinterpret_cast<float4*>(sum + at + 4) = v;
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      if (j >= count) break;
+      const float4 a = *reinterpret_cast<const float4*>(o.alpha[j] + k0);
+      const float4 d = *reinterpret_cast<const float4*>(o.alpha[j] + k0 + 4);
+      uint4 hi, mid, lo;
+      split_x3(make_float4(snake(u.x, a.x, eps), snake(u.y, a.y, eps), snake(u.z, a.z, eps), snake(u.w, a.w, eps)),
+               make_float4(snake(v.x, d.x, eps), snake(v.y, d.y, eps), snake(v.z, d.z, eps), snake(v.w, d.w, eps)), hi,
+               mid, lo);
+      o.planes[j][i] = hi;
+      o.planes[j][i + per_plane] = mid;
+      o.planes[j][i + 2 * per_plane] = lo;
+    }
+  }
+}
+
+// leaky((((x0 + x1) + x2) ..) / count): the resblocks' mean and the activation its one reader applies
+struct MeanInputs {
+  const float* x[4];
+};
+
+__global__ __launch_bounds__(256) void k_mean_leaky(MeanInputs in, int count, float* y, int64_t n4, float slope) {
+  const float by = (float)count;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n4; i += (int64_t)gridDim.x * blockDim.x) {
+    float4 v = reinterpret_cast<const float4*>(in.x[0])[i];
+#pragma unroll
+    for (int j = 1; j < 4; ++j) {
+      if (j >= count) break;
+      const float4 a = reinterpret_cast<const float4*>(in.x[j])[i];
+      v = make_float4(v.x + a.x, v.y + a.y, v.z + a.z, v.w + a.w);
+    }
+    v = make_float4(v.x / by, v.y / by, v.z / by, v.w / by);
+    reinterpret_cast<float4*>(y)[i] = make_float4(v.x >= 0.f ? v.x : slope * v.x, v.y >= 0.f ? v.y : slope * v.y,
+                                                  v.z >= 0.f ? v.z : slope * v.z, v.w >= 0.f ? v.w : slope * v.w);
+  }
+}
+
 }  // namespace
 
 extern "C" {
@@ -1104,6 +1349,121 @@ int cv3_qwen2_prefill(const cv3_qwen2_model* m, const cv3_qwen2_state* st, const
                          st->logits, hd.rows, nullptr, s)))
     return rc;
   hipLaunchKernelGGL(k_set_pos, dim3(1), dim3(1), 0, stream, st->pos, pos0 + t - 1);
+  CV3_LAUNCHED();
+  return CV3_OK;
+}
+
+// ---- vocoder ----
+int cv3_conv_planes(const uint16_t* x, int64_t t, int64_t cin, const uint16_t* w_frag, int64_t cout, int64_t k,
+                    int64_t dilation, const float* bias, const float* residual, float* y, const float* alpha,
+                    float eps, uint16_t* y_planes, cv3_stream_t s) {
+  CV3_ALIVE();
+  CV3_REQUIRE(x && w_frag && bias && (y || y_planes) && t >= 0 && cin > 0 && cout > 0 && k > 0 && dilation > 0,
+              CV3_EINVAL, "bad plane convolution");
+  CV3_REQUIRE(cin % 16 == 0 && k * cin % 64 == 0 && cout % 16 == 0, CV3_EUNSUPPORTED,
+              "plane convolution needs C %% 16 == 0 and K %% 64 == 0");
+  CV3_REQUIRE(!y_planes || alpha, CV3_EINVAL, "planes out need an alpha");
+  CV3_REQUIRE(((uintptr_t)x | (uintptr_t)w_frag | (uintptr_t)bias | (uintptr_t)residual | (uintptr_t)y | (uintptr_t)alpha |
+               (uintptr_t)y_planes) % 16 == 0, CV3_EUNSUPPORTED, "plane convolution needs 16-byte alignment");
+  const int64_t rows = ceil_div(t, 32) * 32, bytes = 6 * rows * cin;
+  CV3_REQUIRE(bytes < (1ll << 31) && 6 * rows * cout < (1ll << 34) && (k - 1) * dilation < (1 << 24) && k * cin < (1 << 24),
+              CV3_EUNSUPPORTED, "plane convolution over 2^31 bytes or more");
+  if (!t) return CV3_OK;
+  ConvPlaneParams p{};
+  p.x = reinterpret_cast<const uint4*>(x);
+  p.w = reinterpret_cast<const uint4*>(w_frag);
+  p.xpl = rows * cin / 8;
+  p.wpl = ceil_div(cout, 32) * 32 * k * cin / 8;
+  p.xbytes = (uint32_t)bytes;
+  p.S = (int)(k * cin / 16);
+  p.SC = (int)(cin / 16);
+  p.taps = (int)k;
+  p.dil = (int)dilation;
+  p.m = (int)t;
+  p.n = (int)cout;
+  p.nbx = (int)(rows / 32);
+  p.nbw = (int)ceil_div(cout, 32);
+  p.bias = bias;
+  p.res = residual;
+  p.alpha = alpha;
+  p.eps = eps;
+  p.y = y;
+  p.yp = reinterpret_cast<uint2*>(y_planes);
+  p.ypl = rows / 32 * (cout / 16) * 128;
+  // 256 workgroups at a time, shared with two more launches (a stage's resblocks, or windows, run side by
+  // side; 1 to 8 of them change a decode by 3 %), each as long as its products and its weight's fetch; ties to
+  // the larger tile
+  auto tiles = [&](int rm) { return 3. * (double)(ceil_div(p.nbx, rm) * p.nbw); };
+  auto cost = [&](int rm) { return std::max(1., tiles(rm) / 256) * (rm + 1); };
+  const int rm = cost(2) <= cost(1) ? 2 : 1;
+  // x of one pass in LDS: all channels while a CU has one workgroup anyway, else at most half of the LDS, so that
+  // a second workgroup's products run under this one's fetch (10 s whole: one workgroup to a CU 3.4 ms, two 2.75)
+  const int64_t most = (tiles(rm) <= 256 ? 160 : 80) << 10, per_step = (32 * rm + (k - 1) * dilation) * 96;
+  p.SP = p.SC;
+  while (p.SP > 1 && p.SP * per_step > most) p.SP = p.SP % 2 ? 1 : p.SP / 2;
+  const int64_t lds = std::max<int64_t>(p.SP * per_step, 8 * rm * 4096);
+  CV3_REQUIRE(lds <= 160 << 10, CV3_EUNSUPPORTED, "plane convolution: a tile with its halo needs %lld bytes of LDS",
+              (long long)lds);
+  p.tiles_m = (int)ceil_div(p.nbx, rm);
+  p.tiles_n = p.nbw;
+  // each XCD's L2 fetches its own columns of the weight and rows of x: the split of the eight that fetches least
+  // (440 rows of 256 channels, K = 2816: 4.4 MB each in row runs, 1.2 in columns)
+  double least = 0.;
+  for (int cx = 1; cx <= 8 && cx <= p.tiles_n; cx *= 2) {
+    const double fetch = (double)p.wpl / cx + (double)p.xpl / std::min(8 / cx, p.tiles_m);
+    if (cx > 1 && fetch >= least) continue;
+    least = fetch;
+    p.cx = cx;
+  }
+  p.rows_x = (int)ceil_div(p.tiles_m, 8 / p.cx);
+  p.cols_x = (int)ceil_div(p.tiles_n, p.cx);
+  const dim3 grid((unsigned)(8 * p.rows_x * p.cols_x));
+  hipStream_t st = stream_of(s);
+  if (rm == 2)
+    hipLaunchKernelGGL((k_conv_planes<2, 2, 1>), grid, dim3(512), (uint32_t)lds, st, p);
+  else
+    hipLaunchKernelGGL((k_conv_planes<1, 4, 2>), grid, dim3(512), (uint32_t)lds, st, p);
+  CV3_LAUNCHED();
+  return CV3_OK;
+}
+
+int cv3_snake_planes(const float* x, const float* add, float* sum, int64_t t, int64_t c, float eps, int count,
+                     const float* const* alphas, uint16_t* const* planes, cv3_stream_t s) {
+  CV3_ALIVE();
+  CV3_REQUIRE(x && t >= 0 && c > 0 && c < (1 << 24) && count >= 1 && count <= 3 && alphas && planes, CV3_EINVAL,
+              "bad snake planes");
+  CV3_REQUIRE(c % 16 == 0 && ((uintptr_t)x | (uintptr_t)add | (uintptr_t)sum) % 16 == 0, CV3_EUNSUPPORTED,
+              "snake planes need C %% 16 == 0 and 16-byte alignment");
+  SnakePlanes o{};
+  for (int j = 0; j < count; ++j) {
+    CV3_REQUIRE(alphas[j] && planes[j] && ((uintptr_t)alphas[j] | (uintptr_t)planes[j]) % 16 == 0, CV3_EINVAL,
+                "bad snake planes output %d", j);
+    o.alpha[j] = alphas[j];
+    o.planes[j] = reinterpret_cast<uint4*>(planes[j]);
+  }
+  const int64_t per_plane = ceil_div(t, 32) * 32 * c / 8;
+  if (!per_plane) return CV3_OK;
+  const int64_t blocks = std::min<int64_t>(ceil_div(per_plane, 256), 65536);
+  hipLaunchKernelGGL(k_snake_planes, dim3((unsigned)blocks), dim3(256), 0, stream_of(s), x, add, sum, t, (int)c, eps,
+                     count, o, per_plane);
+  CV3_LAUNCHED();
+  return CV3_OK;
+}
+
+int cv3_mean_leaky(int count, const float* const* x, float* y, int64_t n, float slope, cv3_stream_t s) {
+  CV3_ALIVE();
+  CV3_REQUIRE(count >= 1 && count <= 4 && x && y && n >= 0, CV3_EINVAL, "bad mean");
+  MeanInputs in{};
+  uintptr_t all = (uintptr_t)y;
+  for (int j = 0; j < count; ++j) {
+    CV3_REQUIRE(x[j], CV3_EINVAL, "null input %d of a mean", j);
+    in.x[j] = x[j];
+    all |= (uintptr_t)x[j];
+  }
+  CV3_REQUIRE(n % 4 == 0 && all % 16 == 0, CV3_EUNSUPPORTED, "mean needs multiples of 16 bytes");
+  if (!n) return CV3_OK;
+  hipLaunchKernelGGL(k_mean_leaky, dim3((unsigned)std::min<int64_t>(ceil_div(n / 4, 256), 65536)), dim3(256), 0,
+                     stream_of(s), in, count, y, n / 4, slope);
   CV3_LAUNCHED();
   return CV3_OK;
 }

@@ -27,6 +27,7 @@ epilogue -> causal conv with the residual x added in its epilogue  (hift.py:114-
 from __future__ import annotations
 
 import ctypes
+import math
 from typing import List, Optional
 
 import numpy as np
@@ -36,14 +37,14 @@ from .device import DeviceArray, Event, Graph, Stream, to_device, wait_event
 
 ACT = _lib.ACT
 F4 = 4
-# The whole-input spectral stack's independent branches (each stage's source branch beside its
-# upsampling conv, and its resblocks side by side) run on side streams forked off the thread's
-# stream when the stack is recorded and captured; in the graph the forks and joins are edges.
-# 10 s whole: 4.12 -> 3.37 ms.  The 1 s windows already run side by side on WINDOW_STREAMS
-# streams, and their stacks with branches took 12.0 ms against 7.76, so they keep none.
+# The whole-input spectral stack's independent branches (all source branches from the start, and
+# each stage's resblocks side by side) run on side streams forked off the thread's stream when the
+# stack is recorded and captured; in the graph the forks and joins are edges.  1.1 s whole: the
+# source branches forked stage by stage 1.02 ms, all at once 0.76.  The 1 s windows already run side
+# by side on WINDOW_STREAMS streams, and their stacks with branches took longer, so they keep none.
 BRANCHES = True
 WINDOW_STREAMS = 16  # vocoder windows replayed side by side (one stream each, default priority); a
-                     # 10 s decode in 1 s windows: 4 streams 10.1 ms, 10 or 16 streams 7.4 ms
+                     # 10 s decode in 1 s windows: 5.6 ms
 
 
 def causal_pad(kernel_size: int, dilation: int = 1) -> int:
@@ -187,19 +188,19 @@ class DeviceHiFT:
         self._arena = None       # while recording or capturing: every intermediate of the stack
         self._arena_i = -1       # >= 0 while capturing: the next arena entry to hand out
 
-    def _new(self, shape) -> DeviceArray:
+    def _new(self, shape, dtype=np.float32) -> DeviceArray:
         """A fresh intermediate.  While a stack is recorded, every intermediate is kept
         (the arena); while it is captured, the recorded arrays are handed out again in
         order, so the capture allocates and frees nothing and the graph owns its memory."""
         if self._arena is None:
-            return DeviceArray(shape)
+            return DeviceArray(shape, dtype)
         if self._arena_i >= 0:
             a = self._arena[self._arena_i]
             self._arena_i += 1
-            if a.shape != tuple(shape):
+            if a.shape != tuple(shape) or a.dtype != dtype:
                 raise RuntimeError(f"captured stack diverged from its recording: {a.shape} vs {tuple(shape)}")
             return a
-        a = DeviceArray(shape)
+        a = DeviceArray(shape, dtype)
         self._arena.append(a)
         return a
 
@@ -264,10 +265,55 @@ class DeviceHiFT:
         _lib.call("snake_cl", x.ptr, self.w[key].ptr, y.ptr, x.shape[0], x.shape[1], 1e-9, st)
         return y
 
-    def _act(self, x: DeviceArray, name: str, param: float) -> DeviceArray:
-        y = self._new(x.shape)
-        _lib.call("act", ACT[name], float(param), x.ptr, y.ptr, x.size, None)
-        return y
+    def _planes_of(self, x: DeviceArray) -> DeviceArray:
+        """A buffer for (t, c) rows as three bfloat16 planes in fragment order (whole 32-row blocks)."""
+        t, c = x.shape
+        return self._new((3 * -(-t // 32) * 32 * c,), np.uint16)
+
+    def _on_planes(self, group: str, idx: int, kernel: int, dilations, t: int) -> bool:
+        """Whether a resblock over t rows runs on activation planes: its weights are split, its planes stay
+        below the 2^31 bytes a buffer descriptor covers, and a tile with its halo fits the LDS."""
+        base = f"{group}.{idx}."
+        for j in range(len(dilations)):
+            for conv in ("convs1", "convs2"):
+                key = f"{base}{conv}.{j}.weight"
+                cout, cin, k = self.shape[key]
+                halo = (k - 1) * (dilations[j] if conv == "convs1" else 1)
+                if (key not in self.wpx or cout != cin or cin % 16 or 6 * (t + 31) * cin >= 1 << 31
+                        or 96 * (64 + halo) > 80 << 10):
+                    return False
+        return t > 0
+
+    def _snake_planes(self, x: DeviceArray, keys, add: Optional[DeviceArray] = None, total: Optional[DeviceArray] = None,
+                      st: Optional[int] = None) -> List[DeviceArray]:
+        """Snake of x (+ add, kept in ``total``) with up to three alphas, as planes."""
+        outs = [self._planes_of(x) for _ in keys]
+        P = ctypes.c_void_p * len(keys)
+        _lib.call("snake_planes", x.ptr, add.ptr if add is not None else None, total.ptr if total is not None else None,
+                  x.shape[0], x.shape[1], 1e-9, len(keys), P(*(self.w[k].ptr for k in keys)),
+                  P(*(o.ptr for o in outs)), st)
+        return outs
+
+    def _resblock_planes(self, group: str, idx: int, x: DeviceArray, xp: DeviceArray, kernel: int, dilations,
+                         st: Optional[int] = None) -> DeviceArray:
+        """_resblock from x and its first Snake's planes: two launches a step, each conv leaving the next
+        one's planes behind.  With the planes split again for every tap and column tile, Snake and split-K
+        sums as launches of their own, a step was five launches and 41 us at 55 frames."""
+        base = f"{group}.{idx}."
+        t, c = x.shape
+        yp = self._planes_of(x)
+        cur = x
+        for j, d in enumerate(dilations):
+            k1, k2 = base + f"convs1.{j}", base + f"convs2.{j}"
+            last = j + 1 == len(dilations)
+            _lib.call("conv_planes", xp.ptr, t, c, self.wpx[k1 + ".weight"].ptr, c, kernel, d, self.w[k1 + ".bias"].ptr,
+                      None, None, self.w[base + f"activations2.{j}.alpha"].ptr, 1e-9, yp.ptr, st)
+            out = self._new(x.shape) if cur is x else cur   # in place after the first step
+            _lib.call("conv_planes", yp.ptr, t, c, self.wpx[k2 + ".weight"].ptr, c, kernel, 1, self.w[k2 + ".bias"].ptr,
+                      cur.ptr, out.ptr, None if last else self.w[base + f"activations1.{j + 1}.alpha"].ptr, 1e-9,
+                      None if last else xp.ptr, st)
+            cur = out
+        return cur
 
     def _resblock(self, group: str, idx: int, x: DeviceArray, kernel: int, dilations,
                   st: Optional[int] = None) -> DeviceArray:
@@ -284,6 +330,20 @@ class DeviceHiFT:
             cur = self._conv(y, base + f"convs2.{j}", pad=(causal_pad(kernel, 1), 0), residual=cur, out=out, st=st)
         return cur
 
+    def _source_branch(self, i: int, s_stft: DeviceArray, st: Optional[int] = None) -> DeviceArray:
+        """Stage i's source: the strided source_downs conv and its resblock (hift.py:146-152)."""
+        u = math.prod(self.rates[i + 1:])
+        key = f"source_downs.{i}"
+        ks = self.shape[key + ".weight"][2]
+        if u == 1:
+            si = self._conv_in(s_stft, key, pad=(causal_pad(ks), 0), st=st)
+        else:
+            si = self._conv_in(s_stft, key, stride=u, pad=(u - 1, 0), st=st)
+        if not self._on_planes("source_resblocks", i, self.src_k[i], self.src_d[i], si.shape[0]):
+            return self._resblock("source_resblocks", i, si, self.src_k[i], self.src_d[i], st=st)
+        sp, = self._snake_planes(si, [f"source_resblocks.{i}.activations1.0.alpha"], st=st)
+        return self._resblock_planes("source_resblocks", i, si, sp, self.src_k[i], self.src_d[i], st=st)
+
     def _branches(self, n: int):
         """n side streams and n + 1 events for forking independent branches off the thread's
         stream (inside a capture the forks and joins become graph edges)."""
@@ -297,24 +357,25 @@ class DeviceHiFT:
     def spectral(self, mel: DeviceArray, s_stft: DeviceArray) -> DeviceArray:
         """conv_pre .. conv_post: (80, T) -> (n_fft + 2, 120 T + 1) (hift.py:131-168)."""
         kpre = self.shape["conv_pre.weight"][2]
-        x = self._conv_in(mel, "conv_pre", pad=(0, causal_pad(kpre)))
-        downs = [1] + self.rates[::-1][:-1]
-        down_cum = list(np.cumprod(downs))[::-1]
         # branches only while a stack is recorded or captured: its arena keeps every
         # intermediate alive, so no buffer a side stream uses is freed and reused meanwhile
         branch = self._branch and self._arena is not None
+        if branch:
+            # the source branches read nothing of the main path: all of them fork here, beside
+            # conv_pre and the stages before theirs
+            nb = self.nk - 1
+            side, ev = self._branches(nb + len(self.rates))
+            ev[0].record(None)
+            sources = []
+            for i in range(len(self.rates)):
+                side[nb + i].wait(ev[0])
+                sources.append(self._source_branch(i, s_stft, side[nb + i].handle))
+                ev[nb + i + 1].record(side[nb + i])
+        xl = self._conv_in(mel, "conv_pre", pad=(0, causal_pad(kpre)), act="leaky", act_param=self.slope)
         for i, r in enumerate(self.rates):
-            if branch:  # the source branch beside the leaky + upsampling conv
-                side, ev = self._branches(max(1, self.nk - 1))
-                sst = side[0].handle
-                ev[0].record(None)
-                side[0].wait(ev[0])
-            else:
-                sst = None
-            xl = self._act(x, "leaky", self.slope)
             k = self.shape[f"ups.{i}.weight"][2]
             cout = self.shape[f"ups.{i}.weight"][0]
-            t_up = x.shape[0] * r
+            t_up = xl.shape[0] * r
             if i == len(self.rates) - 1:
                 # reflect pad (1, 0): rows 1.. hold the conv, row 0 copies row 2 (hift.py:144)
                 xu = self._new((t_up + 1, cout))
@@ -324,45 +385,56 @@ class DeviceHiFT:
                           None)
             else:
                 xu = self._conv(xl, f"ups.{i}", up=r, pad=(k - 1, 0))
-            u = int(down_cum[i])
-            ks = self.shape[f"source_downs.{i}.weight"][2]
-            if u == 1:
-                si = self._conv_in(s_stft, f"source_downs.{i}", pad=(causal_pad(ks), 0), st=sst)
-            else:
-                si = self._conv_in(s_stft, f"source_downs.{i}", stride=u, pad=(u - 1, 0), st=sst)
-            si = self._resblock("source_resblocks", i, si, self.src_k[i], self.src_d[i], st=sst)
             if branch:
-                ev[1].record(side[0])
-                wait_event(ev[1])
+                si = sources[i]
+                wait_event(ev[nb + i + 1])
+            else:
+                si = self._source_branch(i, s_stft)
             if si.shape != xu.shape:
                 raise ValueError(f"stage {i}: source branch {si.shape} vs upsampled {xu.shape}")
             xs = self._new(xu.shape)
-            _lib.call("binary", 0, xu.ptr, si.ptr, xs.ptr, xs.size, 0.0, 0.0, None)
+            on = self.nk <= 3 and all(self._on_planes("resblocks", i * self.nk + j, self.rb_k[j], self.rb_d[j],
+                                                      xu.shape[0]) for j in range(self.nk))
+            if on:
+                xps = self._snake_planes(
+                    xu, [f"resblocks.{i * self.nk + j}.activations1.0.alpha" for j in range(self.nk)], si, xs)
+            else:
+                _lib.call("binary", 0, xu.ptr, si.ptr, xs.ptr, xs.size, 0.0, 0.0, None)
             # the resblocks read xs and write their own buffers: resblock j > 0 on side stream
             # j - 1, joined before the sum
             if branch:
                 ev[0].record(None)
-                for sd in side:
+                for sd in side[:nb]:
                     sd.wait(ev[0])
-            rs = [self._resblock("resblocks", i * self.nk + j, xs, self.rb_k[j], self.rb_d[j],
-                                 st=side[j - 1].handle if branch and j > 0 else None)
-                  for j in range(self.nk)]
+            rs = []
+            for j in range(self.nk):
+                jst = side[j - 1].handle if branch and j > 0 else None
+                args = (self.rb_k[j], self.rb_d[j], jst)
+                rs.append(self._resblock_planes("resblocks", i * self.nk + j, xs, xps[j], *args) if on
+                          else self._resblock("resblocks", i * self.nk + j, xs, *args))
             if branch:
-                for j, sd in enumerate(side):
+                for j, sd in enumerate(side[:nb]):
                     ev[j + 1].record(sd)
                     wait_event(ev[j + 1])
+            # ((r0 + r1) + r2) / 3 (hift.py:161-165) and the leaky relu of its one reader: the next
+            # stage's upsampling (slope lrelu_slope) or conv_post (0.01)
+            slope = 0.01 if i == len(self.rates) - 1 else self.slope
+            xl = self._new(xs.shape)
+            if 2 <= self.nk <= 4 and xs.size % 4 == 0:
+                _lib.call("mean_leaky", self.nk, (ctypes.c_void_p * self.nk)(*(r.ptr for r in rs)), xl.ptr, xl.size,
+                          slope, None)
+                continue
             acc = rs[0]
             for j in range(1, self.nk):
                 nxt = self._new(xs.shape)
-                if j == self.nk - 1:   # ((r0 + r1) + r2) / 3 (hift.py:161-165)
+                if j == self.nk - 1:
                     _lib.call("binary", 4, acc.ptr, rs[j].ptr, nxt.ptr, nxt.size, float(self.nk), 0.0, None)
                 else:
                     _lib.call("binary", 0, acc.ptr, rs[j].ptr, nxt.ptr, nxt.size, 0.0, 0.0, None)
                 acc = nxt
-            x = acc
-        x = self._act(x, "leaky", 0.01)
+            _lib.call("act", ACT["leaky"], slope, acc.ptr, xl.ptr, xl.size, None)
         kpost = self.shape["conv_post.weight"][2]
-        return self._conv(x, "conv_post", pad=(causal_pad(kpost), 0), channels_first_out=True)
+        return self._conv(xl, "conv_post", pad=(causal_pad(kpost), 0), channels_first_out=True)
 
     def _stack(self, w: int, slot: int = 0, branches: bool = False):
         """The spectral stack for a w-frame input, captured once per (w, slot): its staging

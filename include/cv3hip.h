@@ -209,6 +209,18 @@ int cv3_linear_code_planes(const uint16_t* x, int64_t m, int64_t k, const uint16
 int cv3_linear_rows_planes(int kind, const float* x, int64_t m, int64_t k, int64_t ldx, const uint16_t* frag,
                            const float* scales_t, int64_t block, int64_t n, const float* bias, float* y, int64_t ldy,
                            const cv3_epilogue* epi, cv3_stream_t s);
+/* The vocoder's causal conv1d (hift.py:114-129, ops.py:165-219) on x [t, cin] as planes in fragment order, with
+ * the weight (cout, k, cin) as planes of cv3_split_x3_frag: conv + bias, + residual [t, cout], to float rows y
+ * and / or Snake(alpha) of them as planes y_planes. */
+int cv3_conv_planes(const uint16_t* x, int64_t t, int64_t cin, const uint16_t* w_frag, int64_t cout, int64_t k,
+                    int64_t dilation, const float* bias, const float* residual, float* y, const float* alpha,
+                    float eps, uint16_t* y_planes, cv3_stream_t s);
+/* Snake (ops.py:38-45) of x + add [t, c] (add or null; the sum kept in sum unless null) with each of count <= 3
+ * alphas, as planes in fragment order. */
+int cv3_snake_planes(const float* x, const float* add, float* sum, int64_t t, int64_t c, float eps, int count,
+                     const float* const* alphas, uint16_t* const* planes, cv3_stream_t s);
+/* y = leaky_relu(((x0 + x1) + ..) / count), count <= 4 (hift.py:161-165 and the activation after it). */
+int cv3_mean_leaky(int count, const float* const* x, float* y, int64_t n, float slope, cv3_stream_t s);
 /* AdaLN (dit.py:168-169) and RMSNorm (ops.py:101-104) whose result is [rows, cols] planes in fragment
  * order; cols a multiple of 16, at most 1024, 16-byte aligned operands. */
 int cv3_layer_norm_planes(const float* x, uint16_t* planes, int64_t rows, int64_t cols, float eps, const float* shift,

@@ -258,3 +258,63 @@ def test_drop_in_linear_first_used_in_a_capture(lib):
         want = ops.linear(x, w).numpy()
         h.launch()
         np.testing.assert_array_equal(out[1].numpy(), want)
+
+
+def _from_planes(p: np.ndarray, t: int, c: int) -> np.ndarray:
+    """(3, blocks, c / 16, 64, 8) bfloat16 fragments -> (t, c) float64 (hi + mid + lo)."""
+    b = -(-t // 32)
+    v = (p.astype(np.uint32) << 16).view(np.float32).astype(np.float64).reshape(3, b, c // 16, 2, 32, 8).sum(0)
+    return v.transpose(0, 3, 1, 2, 4).reshape(b * 32, c)[:t]
+
+
+@pytest.mark.parametrize("c,k,d", [(16, 4, 2), (64, 3, 1), (64, 11, 5), (80, 4, 3), (128, 7, 3), (256, 11, 1), (256, 11, 5)])
+@pytest.mark.parametrize("t", [1, 31, 65, 440, 8231])
+def test_vocoder_conv_on_planes(lib, t, c, k, d):
+    """Snake planes, then the causal conv with each of its outputs, at the edges of the three tiles."""
+    _lib, to_device, empty = lib
+    if t > 1000 and c > 64:
+        t = 4000 + c     # 64-row tiles, their channels in passes
+    rng = np.random.default_rng([t, c, k])
+    x, add = rng.normal(size=(t, c)).astype(np.float32), rng.normal(size=(t, c)).astype(np.float32)
+    w = (rng.normal(size=(c, c, k)) / np.sqrt(c * k)).astype(np.float32)
+    bias, a1, a2 = (rng.uniform(0.2, 1.5, size=c).astype(np.float32) for _ in range(3))
+
+    def snake(v, a):
+        return v + np.sin(a.astype(np.float64) * v) ** 2 / (a.astype(np.float64) + 1e-9)
+
+    ne = ctypes.c_int64()
+    _lib.call("x3_frag_elems", c, k * c, ctypes.addressof(ne))
+    frag, wd = empty((ne.value,), np.uint16), to_device(np.ascontiguousarray(w.transpose(0, 2, 1)))
+    _lib.call("split_x3_frag", wd.ptr, c, k * c, k * c, frag.ptr, None)
+    planes = [empty((3 * -(-t // 32) * 32 * c,), np.uint16) for _ in range(3)]
+    xd, ad, a1d, a2d, bd, total = to_device(x), to_device(add), to_device(a1), to_device(a2), to_device(bias), empty((t, c))
+    P = ctypes.c_void_p * 2
+    _lib.call("snake_planes", xd.ptr, ad.ptr, total.ptr, t, c, 1e-9, 2, P(a1d.ptr, a2d.ptr),
+              P(planes[0].ptr, planes[1].ptr), None)
+    np.testing.assert_array_equal(total.numpy(), x + add)
+    s64 = (x + add).astype(np.float64)
+    assert rel_err(_from_planes(planes[0].numpy(), t, c), snake(s64, a1)) < 1e-6
+    assert rel_err(_from_planes(planes[1].numpy(), t, c), snake(s64, a2)) < 1e-6
+    xin = np.vstack([np.zeros(((k - 1) * d, c)), _from_planes(planes[0].numpy(), t, c)])
+    want = bias + sum(xin[j * d:j * d + t] @ w[:, :, j].T.astype(np.float64) for j in range(k))
+    y = empty((t, c))
+    _lib.call("conv_planes", planes[0].ptr, t, c, frag.ptr, c, k, d, bd.ptr, None, y.ptr, None, 1e-9, None, None)
+    assert rel_err(y.numpy(), want) < 1e-6
+    # in place on the residual, and the next conv's planes
+    _lib.call("conv_planes", planes[0].ptr, t, c, frag.ptr, c, k, d, bd.ptr, total.ptr, total.ptr, a2d.ptr, 1e-9,
+              planes[2].ptr, None)
+    assert rel_err(total.numpy(), want + s64) < 1e-6
+    assert rel_err(_from_planes(planes[2].numpy(), t, c), snake(want + s64, a2)) < 2e-6
+
+
+def test_vocoder_mean_leaky(lib):
+    _lib, to_device, empty = lib
+    rng = np.random.default_rng(0)
+    xs = [rng.normal(size=(7, 36)).astype(np.float32) for _ in range(4)]
+    ds, y = [to_device(x) for x in xs], empty((7, 36))
+    for n in (1, 2, 3, 4):
+        _lib.call("mean_leaky", n, (ctypes.c_void_p * n)(*(d.ptr for d in ds[:n])), y.ptr, y.size, 0.1, None)
+        v = sum(xs[1:n], xs[0]) / np.float32(n)
+        np.testing.assert_allclose(y.numpy(), np.where(v >= 0, v, np.float32(0.1) * v), rtol=2e-7)
+    with pytest.raises(NotImplementedError):
+        _lib.call("mean_leaky", 1, (ctypes.c_void_p * 1)(ds[0].ptr + 4), y.ptr, 4, 0.1, None)
