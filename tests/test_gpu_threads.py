@@ -110,8 +110,11 @@ def test_block_freed_at_home_waits_for_its_stream(gpu):
     """A block freed on the one stream that used it goes back to that stream at once, and to another
     thread's stream only when the first has run dry."""
     import cv3amd.ops as ops
+    from cv3amd import _lib
     from cv3amd.device import DeviceArray, synchronize, to_device
-    nbytes = 37 << 20   # a size class of its own
+    nbytes = 37 << 20   # a size class of its own, with nothing cached in it
+    synchronize()
+    _lib.call("empty_cache")
     rng = np.random.default_rng(2)
     x = to_device(rng.normal(size=(3000, 1024)).astype(np.float32))
     w = rng.normal(size=(4096, 1024)).astype(np.float32)
