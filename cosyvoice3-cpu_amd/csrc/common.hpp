@@ -21,6 +21,12 @@ hipStream_t stream_of(cv3_stream_t s);
 // no entry point may enqueue work any more.
 bool shut_down();
 
+// Memory for the launches that one entry point makes on st, from the caching allocator: ordered behind the block's
+// earlier uses on st itself, given back behind st (scratch_free follows the last launch), owned by the graph if st
+// is capturing.
+int scratch_alloc(void** ptr, size_t bytes, hipStream_t st);
+int scratch_free(void* ptr, hipStream_t st);
+
 constexpr int kWave = 64;
 
 __device__ __forceinline__ float wave_sum(float v) {

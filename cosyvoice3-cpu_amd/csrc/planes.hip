@@ -1249,17 +1249,17 @@ int cv3_linear_rows_planes(int kind, const float* x, int64_t m, int64_t k, int64
               "rows split into planes need K %% 64 == 0 and 16-byte alignment");
   if (!m || !n) return CV3_OK;
   hipStream_t st = stream_of(s);
+  CV3_REQUIRE(st, CV3_EHIP, "no stream");
   void* ws = nullptr;
-  int rc = cv3_malloc(&ws, (size_t)(6 * ceil_div(m, 32) * 32 * k));
+  int rc = scratch_alloc(&ws, (size_t)(6 * ceil_div(m, 32) * 32 * k), st);
   if (rc) return rc;
-  if (s) rc = cv3_record_stream(ws, s);
   uint16_t* planes = reinterpret_cast<uint16_t*>(ws);
-  if (!rc) rc = split_x3_frag(x, m, k, ldx, planes, st);
+  rc = split_x3_frag(x, m, k, ldx, planes, st);
   if (!rc) {
     const int wk = kind == CV3_KIND_F32 ? W_F32 : block >= k ? W_ROW : block == 64 ? W_B64 : W_B32;
     rc = plane_linear(wk, planes, m, k, frag, scales_t, n, bias, y, ldy, nullptr, epi, 0, st, x, ldx);
   }
-  const int rf = cv3_free(ws);
+  const int rf = scratch_free(ws, st);
   return rc ? rc : rf;
 }
 

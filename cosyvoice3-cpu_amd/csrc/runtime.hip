@@ -71,6 +71,12 @@ static bool capturing(hipStream_t st) {
   return hipStreamIsCapturing(st, &cs) == hipSuccess && cs == hipStreamCaptureStatusActive;
 }
 
+// The capture st is part of: its origin stream and every stream forked off it share one id.
+static bool capture_of(hipStream_t st, unsigned long long& id) {
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  return hipStreamGetCaptureInfo(st, &cs, &id) == hipSuccess && cs == hipStreamCaptureStatusActive;
+}
+
 // ---------------------------------------------------------------------------
 // Caching allocator.  hipFree synchronises the whole device, so the drop-in
 // per-op path (which allocates temporaries on every call) keeps freed blocks in
@@ -87,13 +93,18 @@ static bool capturing(hipStream_t st) {
 // of 331 float32 rows 24.3 and 15.9, sdpa over 333 rows 15.0 and 12.0): its home takes it again in stream order, any other
 // stream only once the home has nothing left to do.
 //
-// Graph capture: a block freed while the freeing thread's stream is capturing is
-// still referenced by the graph being built.  It stays allocated and belongs to
-// that graph from cv3_graph_end on; cv3_graph_destroy returns it to the cache
+// Graph capture: a block freed while the freeing thread's stream, or a stream the block was
+// used on, is capturing is still referenced by the graph being built.  It stays allocated and
+// belongs to that graph from cv3_graph_end on; cv3_graph_destroy returns it to the cache
 // behind the graph's last launch.  Allocation during capture reuses only blocks
 // whose pending frees were all recorded on the capturing stream itself (no
 // cross-stream wait inside a capture); a captured graph is launched on its
 // capture stream, or after that stream has been synchronised.
+//
+// Scratch (scratch_alloc / scratch_free): memory that a library call needs between its own
+// launches on a stream, which need not be the calling thread's.  The caller never sees the
+// block, so nothing but the allocator can order it: the stream itself waits for the block's
+// earlier uses, and the free is recorded there.
 // ---------------------------------------------------------------------------
 struct Block {
   size_t size;
@@ -107,7 +118,9 @@ struct Block {
 static std::multimap<size_t, void*> g_free;            // size class -> ptr
 static std::unordered_map<void*, Block> g_blocks;      // every live or cached block
 static size_t g_in_use = 0, g_cached = 0;
-static thread_local std::vector<void*> g_tls_deferred;  // freed during this thread's capture
+static std::unordered_map<unsigned long long, std::vector<void*>> g_deferred;  // capture -> blocks freed during it
+static thread_local unsigned long long g_tls_capture;  // the last capture this thread began
+static thread_local bool g_tls_begun = false;          // ... and has not ended
 
 struct GraphExec {
   hipGraphExec_t exec;
@@ -156,6 +169,15 @@ static int release_locked(void* ptr, Block& b, const std::vector<hipStream_t>& s
   return CV3_OK;
 }
 
+// Parks a block that only its home stream has used: no event.  Caller holds g_mu.
+static void park_quiet_locked(void* ptr, Block& b) {
+  b.pending.clear();
+  b.quiet = true;
+  g_free.emplace(b.size, ptr);
+  g_in_use -= b.size;
+  g_cached += b.size;
+}
+
 // Whether a thread's stream has nothing left to do.  Never asks a stream under capture (cv3_graph_begin holds
 // g_mu, as the callers do).
 static bool idle(hipStream_t s) {
@@ -169,6 +191,94 @@ static void add_stream(std::vector<hipStream_t>& v, hipStream_t s) {
   for (hipStream_t x : v)
     if (x == s) return;
   v.push_back(s);
+}
+
+// Gives a block back behind `streams`: to the cache, or, if one of them is capturing, to that capture (whose
+// graph refers to the block).  Caller holds g_mu.
+static int give_back_locked(void* ptr, Block& b, const std::vector<hipStream_t>& streams) {
+  for (hipStream_t s : streams) {
+    unsigned long long id;
+    if (!capture_of(s, id)) continue;
+    g_deferred[id].push_back(ptr);
+    return CV3_OK;
+  }
+  return release_locked(ptr, b, streams);
+}
+
+// A cached block of class sz for work on st, or null: st waits for its earlier uses.  `query`: other threads'
+// streams may be asked whether they are idle.  A quiet block's home is a thread's own stream, which lives until
+// cv3_shutdown.  Caller holds g_mu.
+static void* take_cached_locked(size_t sz, hipStream_t st, bool cap, bool query, hipError_t& err) {
+  auto range = g_free.equal_range(sz);
+  for (auto it = range.first; it != range.second; ++it) {
+    void* p = it->second;
+    Block& b = g_blocks[p];
+    bool ok = !b.quiet || b.home == st || (query && idle(b.home));
+    if (cap)
+      for (auto& pe : b.pending) ok = ok && pe.first == st;
+    if (!ok) continue;
+    for (auto& pe : b.pending)
+      if (pe.first != st && (err = hipStreamWaitEvent(st, pe.second, 0)) != hipSuccess) return nullptr;
+    g_free.erase(it);
+    b.pending.clear();
+    b.quiet = false;
+    b.users.clear();
+    g_cached -= sz;
+    g_in_use += sz;
+    return p;
+  }
+  return nullptr;
+}
+
+int scratch_alloc(void** ptr, size_t bytes, hipStream_t st) {
+  const size_t sz = size_class(bytes ? bytes : 1);
+  hipStream_t own = stream_of(nullptr);
+  CV3_REQUIRE(own, CV3_EHIP, "could not create the calling thread's stream");
+  const bool cap = capturing(st), cap_own = st == own ? cap : capturing(own);
+  hipError_t e = hipSuccess;
+  {
+    std::lock_guard<std::mutex> lk(g_mu);
+    void* p = take_cached_locked(sz, st, cap, !cap && !cap_own, e);
+    if (e != hipSuccess) return fail(CV3_EHIP, "hipStreamWaitEvent failed: %s", hipGetErrorString(e));
+    if (p) {
+      Block& b = g_blocks[p];
+      b.home = own;
+      if (st != own) b.users.push_back(st);
+      *ptr = p;
+      return CV3_OK;
+    }
+  }
+  void* p = nullptr;
+  e = hipMalloc(&p, sz);
+  if (e != hipSuccess && !cap && !cap_own) {
+    cv3_empty_cache();
+    (void)hipGetLastError();
+    e = hipMalloc(&p, sz);
+  }
+  if (e != hipSuccess) return fail(CV3_EHIP, "hipMalloc(%zu) failed: %s", sz, hipGetErrorString(e));
+  std::lock_guard<std::mutex> lk(g_mu);
+  Block b{sz, own};
+  if (st != own) b.users.push_back(st);
+  g_blocks[p] = b;
+  g_in_use += sz;
+  *ptr = p;
+  return CV3_OK;
+}
+
+int scratch_free(void* ptr, hipStream_t st) {
+  unsigned long long id;
+  const bool cap = capture_of(st, id);
+  std::lock_guard<std::mutex> lk(g_mu);
+  Block& b = g_blocks[ptr];
+  if (cap) {
+    g_deferred[id].push_back(ptr);
+    return CV3_OK;
+  }
+  if (st == b.home) {
+    park_quiet_locked(ptr, b);
+    return CV3_OK;
+  }
+  return release_locked(ptr, b, {st});
 }
 
 }  // namespace cv3
@@ -210,31 +320,19 @@ int cv3_malloc(void** ptr, size_t bytes) {
   hipStream_t cur = stream_of(nullptr);
   CV3_REQUIRE(cur, CV3_EHIP, "could not create the calling thread's stream");
   const bool cap = capturing(cur);
+  hipError_t e = hipSuccess;
   {
     std::lock_guard<std::mutex> lk(g_mu);
-    auto range = g_free.equal_range(sz);
-    for (auto it = range.first; it != range.second; ++it) {
-      void* p = it->second;
-      Block& b = g_blocks[p];
-      bool ok = !b.quiet || b.home == cur || (!cap && idle(b.home));
-      if (cap)
-        for (auto& pe : b.pending) ok = ok && pe.first == cur;
-      if (!ok) continue;
-      for (auto& pe : b.pending)
-        if (pe.first != cur) CV3_HIP(hipStreamWaitEvent(cur, pe.second, 0));
-      g_free.erase(it);
-      b.pending.clear();
-      b.quiet = false;
-      b.home = cur;
-      b.users.clear();
-      g_cached -= sz;
-      g_in_use += sz;
+    void* p = take_cached_locked(sz, cur, cap, !cap, e);
+    CV3_HIP(e);
+    if (p) {
+      g_blocks[p].home = cur;
       *ptr = p;
       return CV3_OK;
     }
   }
   void* p = nullptr;
-  hipError_t e = hipMalloc(&p, sz);
+  e = hipMalloc(&p, sz);
   if (e != hipSuccess && !cap) {
     // Out of memory: release the cache and try once more.
     cv3_empty_cache();
@@ -243,7 +341,7 @@ int cv3_malloc(void** ptr, size_t bytes) {
   }
   if (e != hipSuccess) return fail(CV3_EHIP, "hipMalloc(%zu) failed: %s", sz, hipGetErrorString(e));
   std::lock_guard<std::mutex> lk(g_mu);
-  g_blocks[p] = Block{sz, cur, {}, {}, {}, false};
+  g_blocks[p] = Block{sz, cur};
   g_in_use += sz;
   *ptr = p;
   return CV3_OK;
@@ -263,28 +361,19 @@ int cv3_free(void* ptr) {
   if (!ptr || g_shut.load()) return CV3_OK;
   hipStream_t cur = stream_of(nullptr);
   CV3_REQUIRE(cur, CV3_EHIP, "could not create the calling thread's stream");
-  if (capturing(cur)) {   // the graph being captured may still refer to it
-    std::lock_guard<std::mutex> lk(g_mu);
-    CV3_REQUIRE(g_blocks.count(ptr), CV3_EINVAL, "cv3_free of a pointer not from cv3_malloc");
-    g_tls_deferred.push_back(ptr);
-    return CV3_OK;
-  }
+  const bool cap = capturing(cur);
   std::lock_guard<std::mutex> lk(g_mu);
   auto it = g_blocks.find(ptr);
   CV3_REQUIRE(it != g_blocks.end(), CV3_EINVAL, "cv3_free of a pointer not from cv3_malloc");
   Block& b = it->second;
-  if (cur == b.home && b.users.empty()) {
-    b.pending.clear();
-    b.quiet = true;
-    g_free.emplace(b.size, ptr);
-    g_in_use -= b.size;
-    g_cached += b.size;
+  if (cur == b.home && b.users.empty() && !cap) {
+    park_quiet_locked(ptr, b);
     return CV3_OK;
   }
   std::vector<hipStream_t> streams{b.home};
   for (hipStream_t u : b.users) add_stream(streams, u);
   add_stream(streams, cur);
-  return release_locked(ptr, b, streams);
+  return give_back_locked(ptr, b, streams);
 }
 
 int cv3_empty_cache(void) {
@@ -437,10 +526,12 @@ int cv3_stream_capturing(cv3_stream_t s, int* yes) {
 
 int cv3_graph_begin(cv3_stream_t s) {
   CV3_ALIVE();
-  CV3_REQUIRE(g_tls_deferred.empty(), CV3_EINVAL, "a capture is already in progress on this thread");
   hipStream_t st = stream_of(s);
   std::lock_guard<std::mutex> lk(g_mu);   // against idle()
+  CV3_REQUIRE(!g_tls_begun || !g_deferred.count(g_tls_capture), CV3_EINVAL,
+              "a capture is already in progress on this thread");
   CV3_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
+  g_tls_begun = capture_of(st, g_tls_capture);
   return CV3_OK;
 }
 
@@ -449,7 +540,17 @@ int cv3_graph_end(cv3_stream_t s, void** exec) {
   hipGraph_t g = nullptr;
   hipStream_t st = stream_of(s);
   std::vector<void*> owned;
-  owned.swap(g_tls_deferred);
+  {
+    std::lock_guard<std::mutex> lk(g_mu);
+    unsigned long long id;
+    const bool active = capture_of(st, id);   // not once the capture is invalid: the thread's own record of it then
+    auto it = active || g_tls_begun ? g_deferred.find(active ? id : g_tls_capture) : g_deferred.end();
+    if (it != g_deferred.end()) {
+      owned.swap(it->second);
+      g_deferred.erase(it);
+    }
+    g_tls_begun = false;
+  }
   hipError_t e = hipStreamEndCapture(st, &g);
   hipGraphExec_t x = nullptr;
   if (e == hipSuccess) {
@@ -461,7 +562,11 @@ int cv3_graph_end(cv3_stream_t s, void** exec) {
     std::lock_guard<std::mutex> lk(g_mu);
     for (void* p : owned) {
       auto it = g_blocks.find(p);
-      if (it != g_blocks.end()) release_locked(p, it->second, {it->second.home, st});
+      if (it == g_blocks.end()) continue;
+      std::vector<hipStream_t> streams{it->second.home};
+      for (hipStream_t u : it->second.users) add_stream(streams, u);
+      add_stream(streams, st);
+      give_back_locked(p, it->second, streams);
     }
     return fail(CV3_EHIP, "graph capture failed: %s", hipGetErrorString(e));
   }
@@ -493,7 +598,7 @@ int cv3_graph_destroy(void* exec) {
       std::vector<hipStream_t> streams{it->second.home};
       for (hipStream_t u : it->second.users) add_stream(streams, u);
       if (w->last) add_stream(streams, w->last);
-      release_locked(p, it->second, streams);
+      give_back_locked(p, it->second, streams);
     }
   }
   hipError_t e = hipGraphExecDestroy(w->exec);
@@ -519,6 +624,7 @@ int cv3_shutdown(void) {
   }
   g_blocks.clear();
   g_free.clear();
+  g_deferred.clear();
   g_in_use = g_cached = 0;
   for (hipStream_t st : g_thread_streams) hipStreamDestroy(st);
   g_thread_streams.clear();

@@ -72,7 +72,7 @@ const char* cv3_last_error(void);
 int cv3_init(int device);
 int cv3_device_info(int* cu_count, int64_t* hbm_bytes, char* arch_name, int name_len);
 int cv3_malloc(void** ptr, size_t bytes); /* stream-aware caching allocator */
-int cv3_free(void* ptr);    /* behind every stream the block was used on; deferred to the graph if capturing */
+int cv3_free(void* ptr);    /* behind every stream the block was used on; deferred to the graph if one is capturing */
 /* Marks a block as used on stream s too, so its free waits for s (no counterpart in the reference, whose
  * arrays are host memory: the device analogue of a tensor used on a second stream). */
 int cv3_record_stream(void* ptr, cv3_stream_t s);
@@ -205,7 +205,8 @@ int cv3_linear_code_planes(const uint16_t* x, int64_t m, int64_t k, const uint16
                            const cv3_epilogue* epi, int64_t plan_rows, cv3_stream_t s);
 /* ops.linear (ops.py:121-123, quant.py:156-204) on float32 rows with such a weight: x is split into planes in a
  * workspace of the caching allocator, then multiplied as above.  kind: the weight's (float32 planes of
- * cv3_split_x3_frag, or codes).  Rows with infinities give what float32 products of them give. */
+ * cv3_split_x3_frag, or codes).  Rows with infinities give what float32 products of them give.  The workspace is
+ * the call's own: ordered on s, whichever stream that is, and the graph's if s is capturing. */
 int cv3_linear_rows_planes(int kind, const float* x, int64_t m, int64_t k, int64_t ldx, const uint16_t* frag,
                            const float* scales_t, int64_t block, int64_t n, const float* bias, float* y, int64_t ldy,
                            const cv3_epilogue* epi, cv3_stream_t s);

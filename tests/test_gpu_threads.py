@@ -142,3 +142,108 @@ def test_block_freed_at_home_waits_for_its_stream(gpu):
         c, late = other.submit(fresh).result()
         assert late == ptr
         del b, c, y
+
+
+def _rows_planes(x, w, y, stream):
+    """ops.linear's plane call on an explicit stream, without a bias: x [m, k], w the cached float32 weight."""
+    from cv3amd import _lib, weights
+    n, k = w.shape
+    p = weights.device_planes(w, weights.device_f32(w))
+    _lib.call("linear_rows_planes", p.kind_code, x.ptr, x.shape[0], k, k, p.frag.ptr, p.scales_ptr, p.block, n, None,
+              y.ptr, n, None, stream.handle if stream is not None else None)
+
+
+def _plane_linear_case(seed, m=2500, k=1024, n=2048):
+    from cv3amd.device import to_device
+    import cv3amd.ops as ops
+    rng = np.random.default_rng(seed)
+    w = rng.standard_normal((n, k), dtype=np.float32) * np.float32(0.02)
+    w.flags.writeable = False
+    xs = [to_device(rng.standard_normal((m, k), dtype=np.float32)) for _ in range(2)]
+    return w, xs, [ops.linear(x, w).numpy() for x in xs]
+
+
+def test_call_scratch_is_ordered_on_its_own_stream(gpu):
+    """A linear on a stream that is not the thread's splits its rows into scratch that the thread's stream gave
+    back a moment ago, or the other way round: each waits for the other's use of it."""
+    from cv3amd.device import DeviceArray, Stream, synchronize
+    w, (x0, x1), (want0, want1) = _plane_linear_case(5)
+    side = Stream()
+    y = [DeviceArray(want0.shape) for _ in range(4)]
+    synchronize()
+    for _ in range(8):
+        _rows_planes(x0, w, y[0], None)
+        _rows_planes(x1, w, y[1], side)
+        _rows_planes(x0, w, y[2], None)
+        _rows_planes(x1, w, y[3], side)
+        _sync(side)
+        synchronize()
+        for got, want in zip(y, (want0, want1, want0, want1)):
+            np.testing.assert_array_equal(got.numpy(), want)
+            got.zero_()
+        synchronize()
+
+
+def _sync(stream):
+    from cv3amd import _lib
+    _lib.call("stream_sync", stream.handle)
+
+
+def test_call_scratch_on_a_capturing_stream_belongs_to_the_graph(gpu):
+    """The same call captured on such a stream, while the thread's own is not: eager calls of the same shape
+    between the replays never share its scratch."""
+    import ctypes
+    from cv3amd import _lib
+    from cv3amd.device import DeviceArray, Stream, synchronize
+    w, (x0, x1), (want0, want1) = _plane_linear_case(6)
+    side = Stream()
+    y, z = DeviceArray(want0.shape), DeviceArray(want0.shape)
+    synchronize()
+    _rows_planes(x0, w, y, side)    # the stream has scratch of its own in the cache
+    _sync(side)
+    _lib.call("graph_begin", side.handle)
+    _rows_planes(x0, w, y, side)
+    x = ctypes.c_void_p()
+    _lib.call("graph_end", side.handle, ctypes.addressof(x))
+    for _ in range(4):
+        y.zero_()
+        synchronize()
+        _lib.call("graph_launch", x.value, side.handle)
+        for _ in range(3):
+            _rows_planes(x1, w, z, None)
+        _sync(side)
+        synchronize()
+        np.testing.assert_array_equal(y.numpy(), want0)
+        np.testing.assert_array_equal(z.numpy(), want1)
+    synchronize()
+    in_use, _ = _lib.mem_stats()
+    _lib.call("graph_destroy", x.value)
+    assert _lib.mem_stats()[0] < in_use     # the scratch was the graph's until now
+
+
+def test_block_dropped_during_another_streams_capture_belongs_to_its_graph(gpu):
+    """A block recorded on a stream under capture and dropped meanwhile, from a thread whose own stream is not
+    capturing, stays with that graph."""
+    import ctypes
+    from cv3amd import _lib
+    from cv3amd.device import DeviceArray, Stream, synchronize
+    nbytes = 5 << 20
+    side = Stream()
+    a = DeviceArray((nbytes // 4,)).record_stream(side)
+    pa = a.ptr
+    synchronize()
+    _lib.call("graph_begin", side.handle)
+    _lib.call("fill_zero", a.ptr, a.nbytes, side.handle)
+    del a
+    x = ctypes.c_void_p()
+    _lib.call("graph_end", side.handle, ctypes.addressof(x))
+    b = DeviceArray((nbytes // 4,)).copy_from(np.ones(nbytes // 4, np.float32))
+    assert b.ptr != pa, "a block the graph refers to was handed out again"
+    for _ in range(2):
+        _lib.call("graph_launch", x.value, side.handle)
+        _sync(side)
+    assert float(b.numpy().min()) == 1.0
+    in_use0, _ = _lib.mem_stats()
+    _lib.call("graph_destroy", x.value)
+    assert in_use0 - _lib.mem_stats()[0] == nbytes
+    del b
