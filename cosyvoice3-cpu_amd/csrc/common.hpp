@@ -23,7 +23,8 @@ bool shut_down();
 
 // Memory for the launches that one entry point makes on st, from the caching allocator: ordered behind the block's
 // earlier uses on st itself, given back behind st (scratch_free follows the last launch), owned by the graph if st
-// is capturing.
+// is capturing (where the next call on st takes it again).  CV3_ENOMEM if there is none: out of memory, or nothing
+// cached and the thread or st is capturing.
 int scratch_alloc(void** ptr, size_t bytes, hipStream_t st);
 int scratch_free(void* ptr, hipStream_t st);
 

@@ -104,7 +104,8 @@ static bool capture_of(hipStream_t st, unsigned long long& id) {
 // Scratch (scratch_alloc / scratch_free): memory that a library call needs between its own
 // launches on a stream, which need not be the calling thread's.  The caller never sees the
 // block, so nothing but the allocator can order it: the stream itself waits for the block's
-// earlier uses, and the free is recorded there.
+// earlier uses, and the free is recorded there.  hipMalloc is refused during a capture, so a
+// capture's calls on one stream share what the first of them found in the cache, in stream order.
 // ---------------------------------------------------------------------------
 struct Block {
   size_t size;
@@ -113,6 +114,7 @@ struct Block {
   std::vector<hipEvent_t> events;                          // event pool, grows to #streams
   std::vector<std::pair<hipStream_t, hipEvent_t>> pending;  // recorded at the last free
   bool quiet = false;  // last freed on its home stream, used on no other: no event was recorded
+  hipStream_t scratch = nullptr;  // waiting for its capture to end: scratch that this stream is done with
 };
 
 static std::multimap<size_t, void*> g_free;            // size class -> ptr
@@ -238,6 +240,18 @@ int scratch_alloc(void** ptr, size_t bytes, hipStream_t st) {
   hipError_t e = hipSuccess;
   {
     std::lock_guard<std::mutex> lk(g_mu);
+    unsigned long long id;
+    if (cap && capture_of(st, id)) {  // what an earlier call of this capture used on this stream, and is done with
+      std::vector<void*>& held = g_deferred[id];
+      for (size_t i = 0; i < held.size(); ++i) {
+        Block& b = g_blocks[held[i]];
+        if (b.scratch != st || b.size != sz) continue;
+        *ptr = held[i];
+        b.scratch = nullptr;
+        held.erase(held.begin() + i);
+        return CV3_OK;
+      }
+    }
     void* p = take_cached_locked(sz, st, cap, !cap && !cap_own, e);
     if (e != hipSuccess) return fail(CV3_EHIP, "hipStreamWaitEvent failed: %s", hipGetErrorString(e));
     if (p) {
@@ -249,13 +263,18 @@ int scratch_alloc(void** ptr, size_t bytes, hipStream_t st) {
     }
   }
   void* p = nullptr;
+  // hipMalloc is refused to a thread that captures, and would spoil the capture
+  CV3_REQUIRE(!cap && !cap_own, CV3_ENOMEM, "no scratch of %zu bytes is cached, and none can be allocated in a capture", sz);
   e = hipMalloc(&p, sz);
-  if (e != hipSuccess && !cap && !cap_own) {
+  if (e != hipSuccess) {
     cv3_empty_cache();
     (void)hipGetLastError();
     e = hipMalloc(&p, sz);
   }
-  if (e != hipSuccess) return fail(CV3_EHIP, "hipMalloc(%zu) failed: %s", sz, hipGetErrorString(e));
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    return fail(CV3_ENOMEM, "hipMalloc(%zu) failed: %s", sz, hipGetErrorString(e));
+  }
   std::lock_guard<std::mutex> lk(g_mu);
   Block b{sz, own};
   if (st != own) b.users.push_back(st);
@@ -271,6 +290,7 @@ int scratch_free(void* ptr, hipStream_t st) {
   std::lock_guard<std::mutex> lk(g_mu);
   Block& b = g_blocks[ptr];
   if (cap) {
+    b.scratch = st;
     g_deferred[id].push_back(ptr);
     return CV3_OK;
   }
@@ -339,7 +359,10 @@ int cv3_malloc(void** ptr, size_t bytes) {
     (void)hipGetLastError();
     e = hipMalloc(&p, sz);
   }
-  if (e != hipSuccess) return fail(CV3_EHIP, "hipMalloc(%zu) failed: %s", sz, hipGetErrorString(e));
+  if (e != hipSuccess) {
+    (void)hipGetLastError();   // or the next launch would report it
+    return fail(CV3_EHIP, "hipMalloc(%zu) failed: %s", sz, hipGetErrorString(e));
+  }
   std::lock_guard<std::mutex> lk(g_mu);
   g_blocks[p] = Block{sz, cur};
   g_in_use += sz;
@@ -549,6 +572,7 @@ int cv3_graph_end(cv3_stream_t s, void** exec) {
       owned.swap(it->second);
       g_deferred.erase(it);
     }
+    for (void* p : owned) g_blocks[p].scratch = nullptr;
     g_tls_begun = false;
   }
   hipError_t e = hipStreamEndCapture(st, &g);

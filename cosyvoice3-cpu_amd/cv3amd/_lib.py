@@ -22,7 +22,7 @@ LIB_PATH = os.environ.get("CV3HIP_LIB", os.path.join(HERE, "libcv3hip.so"))
 _ROOT = os.path.dirname(os.path.dirname(HERE))
 HEADER = os.path.join(_ROOT, "include", "cv3hip.h")
 
-OK, EINVAL, EINDEX, EASSERT, EHIP, EUNSUPPORTED = 0, 1, 2, 3, 4, 5
+OK, EINVAL, EINDEX, EASSERT, EHIP, EUNSUPPORTED, ENOMEM = 0, 1, 2, 3, 4, 5, 6
 F32, F16 = 0, 1
 KIND_F32, KIND_F16, KIND_Q8, KIND_Q4 = 0, 1, 2, 3
 ACT = {"none": 0, "silu": 1, "sigmoid": 2, "gelu_tanh": 3, "gelu": 4, "mish": 5, "elu": 6,
@@ -98,6 +98,10 @@ class HIPError(RuntimeError):
     pass
 
 
+class ScratchError(HIPError):
+    """No memory for a call's own scratch: nothing was enqueued."""
+
+
 def _raise(rc: int, what: str):
     msg = lib().cv3_last_error().decode(errors="replace")
     if rc == EINDEX:
@@ -108,7 +112,7 @@ def _raise(rc: int, what: str):
         raise AssertionError(msg)
     if rc == EUNSUPPORTED:
         raise NotImplementedError(msg)
-    raise HIPError(f"{what}: {msg}")
+    raise (ScratchError if rc == ENOMEM else HIPError)(f"{what}: {msg}")
 
 
 def call(name: str, *args):

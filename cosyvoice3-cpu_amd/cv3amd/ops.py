@@ -188,14 +188,18 @@ def _linear_planes(xd, m, k, weight, dev, n, bd, y) -> bool:
     """y = x . W^T + bias on the bfloat16 matrix cores, x split into planes on the way, for a cached weight
     whose planes the device keeps beside it.  More than four rows: up to four are the GEMV's.  The float32
     kernels walk K serially and run at half the rate: [3000, 1024] x [3072, 1024] q8 196 us, here 94;
-    [40, 4864] x [896, 4864] 120, here 23; [331, 1024] x [2048, 1024] float32 25, here 16."""
+    [40, 4864] x [896, 4864] 120, here 23; [331, 1024] x [2048, 1024] float32 25, here 16.  False where those
+    kernels serve: no planes, or no memory to split x into (a capture takes it from the cache only)."""
     if xd.ptr % 16 or (bd is not None and bd.ptr % 16):
         return False
     w = _w.device_planes(weight, dev)
     if w is None:
         return False
-    _lib.call("linear_rows_planes", w.kind_code, xd.ptr, m, k, k, w.frag.ptr, w.scales_ptr, w.block, n,
-              bd.ptr if bd is not None else None, y.ptr, n, None, None)
+    try:
+        _lib.call("linear_rows_planes", w.kind_code, xd.ptr, m, k, k, w.frag.ptr, w.scales_ptr, w.block, n,
+                  bd.ptr if bd is not None else None, y.ptr, n, None, None)
+    except _lib.ScratchError:
+        return False
     return True
 
 

@@ -101,8 +101,9 @@ def device_planes(weight, dev) -> Optional[DevicePlanes]:
     beside that copy on first use and kept and released with it.  None for what the plane linear does not
     take, for K up to 512 (two launches: 10.7 us against 8.6 of the one float32 kernel at K = 256, within 15 %
     of each other either way at 512, 13.5 against 21.5 at 1024, whatever m; q8 more), for a first use inside
-    a capture (packing waits for the device), and for weights that are not cached: a writeable array, or one
-    that lives on the device (its owner may write to it between calls)."""
+    a capture (packing waits for the device), for weights that are not cached: a writeable array, or one
+    that lives on the device (its owner may write to it between calls), and for a weight whose planes found no
+    memory (6 bytes a float32 weight, 2 a code)."""
     quantised = isinstance(dev, DeviceQ)
     if quantised:
         cached = not isinstance(weight.q, DeviceArray) and not isinstance(weight.scales, DeviceArray)
@@ -117,7 +118,7 @@ def device_planes(weight, dev) -> Optional[DevicePlanes]:
     key = ("planes", id(weight))
     hit = _CACHE.get(key)
     if hit is not None:
-        return hit
+        return hit or None
     with _UPLOAD:
         hit = _CACHE.get(key)
         if hit is None:
@@ -125,22 +126,28 @@ def device_planes(weight, dev) -> Optional[DevicePlanes]:
             _lib.call("stream_capturing", None, ctypes.addressof(capturing))
             if capturing.value:
                 return None
-            hit = _CACHE[key] = _pack_planes(dev, n, k, block)
+            hit = _CACHE[key] = _pack_planes(dev, n, k, block) or False
             weakref.finalize(weight, _CACHE.pop, key, None)
-    return hit
+    return hit or None
 
 
-def _pack_planes(dev, n: int, k: int, block: int) -> DevicePlanes:
+def _pack_planes(dev, n: int, k: int, block: int) -> Optional[DevicePlanes]:
     ne, ns = ctypes.c_int64(), ctypes.c_int64()
-    if isinstance(dev, DeviceQ):
+    quantised = isinstance(dev, DeviceQ)
+    if quantised:
         _lib.call("code_planes_elems", n, k, block, ctypes.addressof(ne), ctypes.addressof(ns))
-        frag, scales = DeviceArray((ne.value,), np.uint16), DeviceArray((ns.value,))
+    else:
+        _lib.call("x3_frag_elems", n, k, ctypes.addressof(ne))
+    try:
+        frag = DeviceArray((ne.value,), np.uint16)
+        scales = DeviceArray((ns.value,)) if quantised else None
+    except _lib.HIPError:
+        return None
+    if quantised:
         _lib.call("pack_code_planes", dev.kind_code, dev.q.ptr, n, k, dev.scales.ptr, dev.scale_code, dev.kp, block, 0,
                   0, frag.ptr, scales.ptr, None)
         out = DevicePlanes(dev.kind_code, frag, scales.ptr, block, scales)
     else:
-        _lib.call("x3_frag_elems", n, k, ctypes.addressof(ne))
-        frag = DeviceArray((ne.value,), np.uint16)
         _lib.call("split_x3_frag", dev.ptr, n, k, k, frag.ptr, None)
         out = DevicePlanes(_lib.KIND_F32, frag, None, k)
     _lib.call("stream_sync", None)   # another thread's stream may read it next

@@ -8,6 +8,7 @@
  * Status codes map onto the exceptions the reference raises:
  *   CV3_EINVAL  -> ValueError      CV3_EINDEX -> IndexError
  *   CV3_EASSERT -> AssertionError  CV3_EHIP   -> RuntimeError (HIP failure)
+ *   CV3_ENOMEM  -> RuntimeError (no memory for a call's own scratch; nothing was enqueued)
  *
  * The reference (cv3cpu) has no FFI of its own: its kernels are the module
  * functions of cv3cpu/ops.py and cv3cpu/quant.py, which the models resolve at
@@ -27,7 +28,7 @@ extern "C" {
 
 typedef struct cv3_stream_opaque* cv3_stream_t;
 
-enum { CV3_OK = 0, CV3_EINVAL = 1, CV3_EINDEX = 2, CV3_EASSERT = 3, CV3_EHIP = 4, CV3_EUNSUPPORTED = 5 };
+enum { CV3_OK = 0, CV3_EINVAL = 1, CV3_EINDEX = 2, CV3_EASSERT = 3, CV3_EHIP = 4, CV3_EUNSUPPORTED = 5, CV3_ENOMEM = 6 };
 
 /* element / weight kinds */
 enum { CV3_F32 = 0, CV3_F16 = 1 };
@@ -206,7 +207,8 @@ int cv3_linear_code_planes(const uint16_t* x, int64_t m, int64_t k, const uint16
 /* ops.linear (ops.py:121-123, quant.py:156-204) on float32 rows with such a weight: x is split into planes in a
  * workspace of the caching allocator, then multiplied as above.  kind: the weight's (float32 planes of
  * cv3_split_x3_frag, or codes).  Rows with infinities give what float32 products of them give.  The workspace is
- * the call's own: ordered on s, whichever stream that is, and the graph's if s is capturing. */
+ * the call's own: ordered on s, whichever stream that is, and the graph's if s is capturing.  CV3_ENOMEM if there
+ * is none to be had (a capture takes it from the cache only): the float32 kernels need no workspace. */
 int cv3_linear_rows_planes(int kind, const float* x, int64_t m, int64_t k, int64_t ldx, const uint16_t* frag,
                            const float* scales_t, int64_t block, int64_t n, const float* bias, float* y, int64_t ldy,
                            const cv3_epilogue* epi, cv3_stream_t s);

@@ -244,6 +244,7 @@ def test_drop_in_linear_first_used_in_a_capture(lib):
     w.flags.writeable = False
     x = to_device(rng.normal(size=(40, 640)).astype(np.float32))
     ops.linear(x.rows(0, 2), w)   # the weight is on the device, its planes are not
+    [empty((40, 96)) for _ in range(3)]   # results to be had from the cache: a capture allocates nothing
     out = []
     with Graph() as g:
         out.append(ops.linear(x, w))
@@ -258,6 +259,39 @@ def test_drop_in_linear_first_used_in_a_capture(lib):
         want = ops.linear(x, w).numpy()
         h.launch()
         np.testing.assert_array_equal(out[1].numpy(), want)
+
+
+def test_captured_linears_find_their_scratch(lib):
+    """A capture cannot allocate: its linears share the one piece of scratch in the cache, and with none there
+    they run the float32 kernels, as they do when memory is short.  Replays with eager calls between them."""
+    import cv3amd.ops as ops
+    from cv3amd.device import Graph, synchronize
+    _lib, to_device, empty = lib
+    rng = np.random.default_rng(9)
+    m, k, n = 700, 1024, 2048    # 5.6 MB of results, 4.3 of scratch: size classes of their own
+    w = (0.02 * rng.normal(size=(n, k))).astype(np.float32)
+    w.flags.writeable = False
+    xs = [to_device(rng.normal(size=(m, k)).astype(np.float32)) for _ in range(3)]
+    want = [x.numpy().astype(np.float64) @ w.T.astype(np.float64) for x in xs]
+    ops.linear(xs[0], w)         # the weight's planes are there
+    for scratch in (1, 0):
+        synchronize()
+        _lib.call("empty_cache")
+        eager = [ops.linear(x, w) for x in xs] if scratch else [empty((m, n)) for _ in xs]
+        del eager                # three results in the cache, and one piece of scratch or none
+        with Graph() as g:
+            out = [ops.linear(x, w) for x in xs]
+        for _ in range(3):
+            for y in out:
+                y.zero_()
+            g.launch()
+            other = ops.linear(xs[2], w).numpy()
+            for y, a in zip(out, want):
+                assert rel_err(y.numpy(), a) < TOL
+            assert rel_err(other, want[2]) < TOL
+        if scratch:
+            np.testing.assert_array_equal(out[2].numpy(), other)
+        del out, y, g
 
 
 def _from_planes(p: np.ndarray, t: int, c: int) -> np.ndarray:

@@ -170,3 +170,32 @@ def test_vocoder_windows_with_receptive_history_equal_the_full_context():
     full = h.spectral_chunked(mel, s, 50, 64)
     assert np.array_equal(h.spectral_chunked(mel, s, 50, R), full)
     assert np.array_equal(h.spectral(mel, s), full)
+
+
+def test_linear_without_memory_for_planes(monkeypatch):
+    """A weight whose planes find no memory is asked once and keeps the float32 kernel; a linear whose rows find
+    none does too."""
+    from cv3amd import _lib, ops, weights
+    asked = []
+
+    def call(name, *args):
+        asked.append(name)
+        if name == "linear_rows_planes":
+            raise _lib.ScratchError("no scratch")
+
+    def no_memory(*a, **kw):
+        raise _lib.HIPError("hipMalloc failed")
+
+    class Dev:
+        shape, ptr = (96, 640), 1 << 20
+
+    monkeypatch.setattr(_lib, "call", call)
+    monkeypatch.setattr(weights, "DeviceArray", no_memory)
+    w = np.zeros((96, 640), np.float32)
+    w.flags.writeable = False
+    assert weights.device_planes(w, Dev) is None and "x3_frag_elems" in asked
+    del asked[:]
+    assert weights.device_planes(w, Dev) is None and not asked
+    monkeypatch.setattr(weights, "device_planes", lambda *a: weights.DevicePlanes(0, Dev, None, 640))
+    assert ops._linear_planes(Dev, 40, 640, w, Dev, 96, None, Dev) is False
+    assert asked == ["linear_rows_planes"]
