@@ -37,6 +37,35 @@ __device__ __forceinline__ void split_x3(const float4& a, const float4& b, uint4
   split_x3(b.z, b.w, hi.w, mid.w, lo.w);
 }
 
+// The same planes for a weight or a linear's rows, whose largest values count too: past the largest bfloat16 (3.39e38)
+// the rounding above is an infinity, and x - inf loses the value.  Here hi stays at that largest and mid and lo hold
+// the rest, exact as everywhere; an infinity is (inf, 0, 0), so that lo + mid + hi, summed in this order, is x.
+__device__ __forceinline__ void split_x3_full(float a, uint16_t& hi, uint16_t& mid, uint16_t& lo) {
+  const float top = 3.3895313892515355e38f;
+  const bool finite = fabsf(a) <= 3.4028234663852886e38f;
+  const __bf16 h = (__bf16)(finite ? fminf(fmaxf(a, -top), top) : a);
+  const float r1 = finite ? a - (float)h : 0.f;
+  const __bf16 m = (__bf16)r1;
+  const __bf16 l = (__bf16)(r1 - (float)m);
+  hi = __builtin_bit_cast(uint16_t, h);
+  mid = __builtin_bit_cast(uint16_t, m);
+  lo = __builtin_bit_cast(uint16_t, l);
+}
+
+__device__ __forceinline__ void split_x3_full(const float4& a, const float4& b, uint4& hi, uint4& mid, uint4& lo) {
+  const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+  uint32_t *h = &hi.x, *m = &mid.x, *l = &lo.x;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    uint16_t p[2][3];
+    split_x3_full(v[2 * i], p[0][0], p[0][1], p[0][2]);
+    split_x3_full(v[2 * i + 1], p[1][0], p[1][1], p[1][2]);
+    h[i] = p[0][0] | (uint32_t)p[1][0] << 16;
+    m[i] = p[0][1] | (uint32_t)p[1][1] << 16;
+    l[i] = p[0][2] | (uint32_t)p[1][2] << 16;
+  }
+}
+
 // Scheduling groups: R times, N1 instructions of class M1, then N2 of class M2 (0x8 MFMA, 0x20 VMEM read,
 // 0x100 LDS read).
 template <int M, int N>

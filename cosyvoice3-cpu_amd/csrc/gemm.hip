@@ -840,7 +840,7 @@ __global__ __launch_bounds__(256) void k_split_x3_frag(const float* w, int64_t n
       b = *reinterpret_cast<const float4*>(w + row * ldw + k0 + 4);
     }
     uint4 hi, mid, lo;
-    split_x3(a, b, hi, mid, lo);
+    split_x3_full(a, b, hi, mid, lo);
     frag[i] = hi;
     frag[per_plane + i] = mid;
     frag[2 * per_plane + i] = lo;
@@ -1092,7 +1092,7 @@ __global__ __launch_bounds__(256) void k_split_x3(const float* w, int64_t n, int
     const float4 a = *reinterpret_cast<const float4*>(src);
     const float4 b = *reinterpret_cast<const float4*>(src + 4);
     uint4 hi, mid, lo;
-    split_x3(a, b, hi, mid, lo);
+    split_x3_full(a, b, hi, mid, lo);
     uint16_t* dst = pb + row * ldp + k0;
     *reinterpret_cast<uint4*>(dst) = hi;
     *reinterpret_cast<uint4*>(dst + pstride) = mid;

@@ -219,9 +219,9 @@ struct PlaneEpilogue {
       for (int e = 0; e < 4; ++e) {
         const int r = nn + e;
         const int64_t at = (((int64_t)(r >> 5) * p.S + (k >> 4)) * 64 + (r & 31) + 32 * ((k >> 3) & 1)) * 8 + (k & 7);
-        float v = 0.f;
+        float v = 0.f;   // lo + mid + hi: exact in this order
 #pragma unroll
-        for (int pl = 0; pl < NPW; ++pl) v += __uint_as_float((uint32_t)w[at + pl * p.wpl * 8] << 16);
+        for (int pl = NPW - 1; pl >= 0; --pl) v += __uint_as_float((uint32_t)w[at + pl * p.wpl * 8] << 16);
         if constexpr (KIND == W_ROW) v *= e == 0 ? row.x : e == 1 ? row.y : e == 2 ? row.z : row.w;
         if constexpr (FOLD > 0) v *= p.scales[(int64_t)(k / (16 * FOLD)) * p.nbw * 32 + r];
         a[e] = fmaf(x, v, a[e]);

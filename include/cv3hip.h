@@ -206,7 +206,8 @@ int cv3_linear_code_planes(const uint16_t* x, int64_t m, int64_t k, const uint16
                            const cv3_epilogue* epi, int64_t plan_rows, cv3_stream_t s);
 /* ops.linear (ops.py:121-123, quant.py:156-204) on float32 rows with such a weight: x is split into planes in a
  * workspace of the caching allocator, then multiplied as above.  kind: the weight's (float32 planes of
- * cv3_split_x3_frag, or codes).  Rows with infinities give what float32 products of them give.  The workspace is
+ * cv3_split_x3_frag, or codes).  Infinities and the largest floats, in rows or a float32
+ * weight, give what float32 products of them give.  The workspace is
  * the call's own: ordered on s, whichever stream that is, and the graph's if s is capturing.  CV3_ENOMEM if there
  * is none to be had (a capture takes it from the cache only): the float32 kernels need no workspace. */
 int cv3_linear_rows_planes(int kind, const float* x, int64_t m, int64_t k, int64_t ldx, const uint16_t* frag,

@@ -233,6 +233,39 @@ def test_drop_in_linear_on_planes(lib, m, k, n, kind):
             assert np.abs(got[r] - want[r])[ok[r]].max() <= TOL * np.abs(want[r][ok[r]]).max()
 
 
+@pytest.mark.parametrize("m,k,n", [(5, 576, 64), (40, 640, 96), (331, 1024, 2048), (1500, 1024, 1152)])
+def test_drop_in_linear_with_a_weight_past_bfloat16(lib, m, k, n):
+    """A cached float32 weight with infinities, a NaN and values between the largest bfloat16 and the largest
+    float: what the float32 kernel gives (a weight that lives on the device keeps it), whatever the row count."""
+    import cv3amd.ops as ops
+    _lib, to_device, empty = lib
+    rng = np.random.default_rng([m, k, n])
+    x, w = rng.normal(size=(m, k)).astype(np.float32), (0.02 * rng.normal(size=(n, k))).astype(np.float32)
+    top = np.finfo(np.float32).max
+    w[1, 3], w[2, 5], w[3, 7], w[7, 0] = np.inf, -np.inf, np.nan, np.inf
+    w[4, 9], w[5, k - 1], w[6, 64], w[n - 1, 33] = top, -top, 3.395e38, 3.3961775e38
+    x[:, [9, k - 1, 64, 33]] *= np.float32(0.1)     # finite products: |x| < 1
+    x[0, :] = 0.0                                   # 0 * inf
+    x[2, 9] = 4.0                                   # and one past the range
+    w.flags.writeable = False
+    b = rng.normal(size=n).astype(np.float32)
+    xd, wd = to_device(x), to_device(w)
+    got, want = ops.linear(xd, w, b).numpy(), ops.linear(xd, wd, b).numpy()
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
+    np.testing.assert_array_equal(got[np.isinf(want)], want[np.isinf(want)])
+    ok = np.isfinite(want)
+    assert ok[:, 4].any() and np.isinf(want[2, 4]) and np.isnan(want[0, 1])
+    for c in range(n):
+        r = ok[:, c]
+        if r.any():
+            assert np.abs(got[r, c].astype(np.float64) - want[r, c]).max() <= TOL * np.abs(want[r, c].astype(np.float64)).max()
+    # and the planes themselves: exact
+    p = to_planes(lib, w)
+    back, finite = from_planes(p, n, k), np.isfinite(w)
+    np.testing.assert_array_equal(back[finite], w[finite].astype(np.float64))
+    np.testing.assert_array_equal(back[np.isinf(w)], w[np.isinf(w)])
+
+
 def test_drop_in_linear_first_used_in_a_capture(lib):
     """A weight that a capture meets first keeps the float32 kernel there; its planes come with the next
     eager call, and both give the same layer."""
