@@ -277,7 +277,9 @@ __global__ __launch_bounds__(256 * NKG) void k_flash64(AttnParams p, int nq) {
     for (int i = 0; i < 4; ++i) orow[db * 16 + 4 * g + i] = oacc[db][i] / l_tot;
 }
 
-// One query of any head dim <= 256 by one wave, 64 keys per step; qs: the scaled query in LDS.
+// One query of any head dim <= 256 by one wave, 64 keys per step; qs: the scaled query in LDS.  EVERY: values before
+// the first key it sees count too, with probability zero (an infinity or NaN among them makes the output NaN).
+template <bool EVERY>
 __device__ __forceinline__ void attend_row(const AttnParams& p, int b, int hq, int hkv, int64_t qi, int lane, const float* qs) {
   const float* kbase = p.k + b * p.k_sb + hkv * p.k_sh;
   const float* vbase = p.v + b * p.v_sb + hkv * p.v_sh;
@@ -296,9 +298,10 @@ __device__ __forceinline__ void attend_row(const AttnParams& p, int b, int hq, i
     }
     const float mx = wave_max(s);
     const float m_new = fmaxf(m_run, mx);
-    if (m_new == -INFINITY) continue;
-    const float alpha = expf(m_run - m_new);
-    const float pj = expf(s - m_new);
+    const bool none = m_new == -INFINITY;
+    if (!EVERY && none) continue;
+    const float alpha = none ? 1.f : expf(m_run - m_new);
+    const float pj = none ? 0.f : expf(s - m_new);
     l_run = l_run * alpha + wave_sum(pj);
 #pragma unroll
     for (int r = 0; r < 4; ++r) acc[r] *= alpha;
@@ -362,6 +365,8 @@ __device__ __forceinline__ void mfma6(const bf16x8_t& ah, const bf16x8_t& am, co
   small = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, bh, small, 0, 0, 0);
 }
 
+// A stage that no query of the workgroup sees is skipped, but for its values' exponents: a masked key counts with
+// probability zero, and zero times an infinity or NaN is NaN in that dim of every output, whichever tile it is in.
 // AGAIN: outputs that come out not finite are formed again in float32.
 template <int QWN, bool AGAIN>
 __global__ __launch_bounds__(512) void k_flash64x(AttnParams p, int nq) {
@@ -370,7 +375,9 @@ __global__ __launch_bounds__(512) void k_flash64x(AttnParams p, int nq) {
   static_assert(NKG * WKT == STAGE, "the key groups share a stage");
   __shared__ uint4 Ks[TILES][3][KT * 8];
   __shared__ uint4 Vs[TILES][3][KT * 8];
+  __shared__ uint32_t skipped[2];  // dims with an infinity or NaN among the values of the skipped stages
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  if (tid < 2) skipped[tid] = 0;
   const int qw = wave % QWN, kg = wave / QWN;
   const int wt = kg * WKT / KT, wr = kg * WKT % KT;  // the group's tile and its first key there
   const int ntiles = (int)gridDim.x;
@@ -558,6 +565,24 @@ __global__ __launch_bounds__(512) void k_flash64x(AttnParams p, int nq) {
   for (int db = 0; db < 4; ++db) oacc[db] = ob[db] + os[db];
   // merge the key groups through LDS, as k_flash64
   __syncthreads();
+  {
+    // thread -> dims 4 dq .. + 3 of every 32nd row; rows past the end clamp to the last one
+    const int rows0 = (int)(st0 * STAGE), at1 = (int)(nstages * STAGE), rows1 = max((int)p.m - at1, 0);
+    float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
+    auto scan = [&](int from, int rows) {
+      for (int r = tid >> 4; r < rows; r += 4 * 32) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const float4 v = *reinterpret_cast<const float4*>(vbase + (int64_t)(from + min(r + 32 * u, rows - 1)) * p.v_sm + 4 * dq);
+          z = make_float4(fmaf(v.x, 0.f, z.x), fmaf(v.y, 0.f, z.y), fmaf(v.z, 0.f, z.z), fmaf(v.w, 0.f, z.w));
+        }
+      }
+    };
+    scan(0, min(rows0, (int)p.m));
+    scan(at1, rows1);
+    const uint32_t bits = (z.x != z.x) | (z.y != z.y) << 1 | (z.z != z.z) << 2 | (z.w != z.w) << 3;
+    if (bits) atomicOr(&skipped[dq >> 3], bits << (4 * (dq & 7)));
+  }
   float* mb = reinterpret_cast<float*>(&Ks[0][0][0]);
   static_assert((NKG - 1) * QWN * 64 * 18 * 4 <= (int)sizeof(Ks), "merge slots fit the K tiles");
   if (kg > 0) {
@@ -590,6 +615,11 @@ __global__ __launch_bounds__(512) void k_flash64x(AttnParams p, int nq) {
   }
   float l_tot = l_run + __shfl_xor(l_run, 16, 64);
   l_tot += __shfl_xor(l_tot, 32, 64);
+  const uint32_t lost[2] = {skipped[0], skipped[1]};
+  auto value = [&](int db, int i) {
+    const bool nan = lost[db >> 1] >> (16 * (db & 1) + 4 * g + i) & 1;
+    return nan ? __builtin_nanf("") : oacc[db][i] / l_tot;
+  };
   if (p.op && qvalid) {
     // row b n + qi of [batch n, 64 h] rows as the fragments a plane linear reads: four neighbouring
     // columns are half of a lane's 16 bytes
@@ -600,8 +630,8 @@ __global__ __launch_bounds__(512) void k_flash64x(AttnParams p, int nq) {
       const int64_t at = (((row >> 5) * (4 * p.h) + (col >> 4)) * 64 + (row & 31) + 32 * ((col >> 3) & 1)) * 2 +
                          ((col >> 2) & 1);
       uint2 hi, mid, lo;
-      split_x3(oacc[db][0] / l_tot, oacc[db][1] / l_tot, hi.x, mid.x, lo.x);
-      split_x3(oacc[db][2] / l_tot, oacc[db][3] / l_tot, hi.y, mid.y, lo.y);
+      split_x3(value(db, 0), value(db, 1), hi.x, mid.x, lo.x);
+      split_x3(value(db, 2), value(db, 3), hi.y, mid.y, lo.y);
       p.op[at] = hi;
       p.op[at + p.opl] = mid;
       p.op[at + 2 * p.opl] = lo;
@@ -615,7 +645,7 @@ __global__ __launch_bounds__(512) void k_flash64x(AttnParams p, int nq) {
     for (int db = 0; db < 4; ++db)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const float y = oacc[db][i] / l_tot;
+        const float y = value(db, i);
         orow[db * 16 + 4 * g + i] = y;
         bad |= !(fabsf(y) <= 3.4028235e38f);
       }
@@ -630,7 +660,7 @@ __global__ __launch_bounds__(512) void k_flash64x(AttnParams p, int nq) {
       todo &= todo - 1;
       qs[lane] = p.q[b * p.q_sb + hq * p.q_sh + row * p.q_sn + lane] * p.scale;
       __builtin_amdgcn_wave_barrier();
-      attend_row(p, b, hq, hkv, row, lane, qs);
+      attend_row<true>(p, b, hq, hkv, row, lane, qs);
       __builtin_amdgcn_wave_barrier();
     }
   }
@@ -649,7 +679,7 @@ __global__ __launch_bounds__(256) void k_attn_generic(AttnParams p) {
   for (int d = lane; d < p.d; d += 64) qs[d] = qvalid ? qrow[d] * p.scale : 0.f;
   __syncthreads();
   if (!qvalid) return;
-  attend_row(p, b, hq, hkv, qi, lane, qs);
+  attend_row<false>(p, b, hq, hkv, qi, lane, qs);
 }
 
 }  // namespace

@@ -302,8 +302,8 @@ int cv3_attention_x3(const float* q, const float* k, const float* v, float* out,
                      const int64_t* v_strides, const int64_t* o_strides, float scale, int mask_kind,
                      int64_t mask_a, int64_t mask_b, cv3_stream_t s);
 /* ops.sdpa itself: contiguous (h, n, d) and (hk, m, d), as cv3_attention_x3.  Outputs that come out not finite
- * are formed again in float32, so infinities give what float32 products of them give; keys that no query of a
- * tile sees are not read. */
+ * are formed again in float32, so infinities give what float32 products of them give: a masked key counts with
+ * probability zero, so an infinity or NaN among its values is NaN in that dim of the head's outputs. */
 int cv3_sdpa(const float* q, const float* k, const float* v, float* out, int h, int hk, int64_t n, int64_t m, int d,
              float scale, int mask_kind, int64_t mask_a, int64_t mask_b, cv3_stream_t s);
 /* cv3_attention_x3 with the output [batch * n, 64 h] as bfloat16 planes in fragment order, for the plane

@@ -671,3 +671,47 @@ def test_sdpa_tiles_and_masks(lib, h, hk, n, m, mask):
         np.testing.assert_array_equal(g[np.isinf(w)], w[np.isinf(w)])
         ok = np.isfinite(w)
         assert not ok.any() or np.abs(g - w)[ok].max() <= 2e-6 * max(1.0, np.abs(w[ok]).max())
+
+
+@pytest.mark.parametrize("entry", ["sdpa", "attention_x3", "attention_x3_planes"])
+@pytest.mark.parametrize("mask", [("causal", 0), ("causal", 70), ("causal", -3), ("chunk", 25, 1), ("chunk", 50, 0)], ids=str)
+@pytest.mark.parametrize("h,hk,n,m", [(14, 2, 33, 37), (14, 2, 333, 403), (14, 2, 700, 700), (3, 1, 300, 900)])
+def test_masked_values_count_with_probability_zero(lib, entry, h, hk, n, m, mask):
+    """An infinity or NaN among the values is NaN in its dim for every query of its heads that masks it (the
+    oracle's 0 * inf), wherever the key lies: in a stage the tile computes, before or after it."""
+    import cv3amd.ops as ops
+    _lib, to_device, empty = lib
+    rng = np.random.default_rng([h, n, m])
+    q, k, v = (rng.normal(size=s).astype(np.float32) for s in ((h, n, 64), (hk, m, 64), (hk, m, 64)))
+    code = {"causal": (1, mask[1], 0), "chunk": (2, mask[1], mask[-1])}[mask[0]]
+    for j, value, dim in ((0, np.inf, 63), (m // 2, np.nan, 0), (m - 1, -np.inf, 21), (m - 1, np.nan, 40)):
+        a = v.copy()
+        a[hk - 1, j, dim] = value
+        with np.errstate(all="ignore"):
+            want = ref.sdpa(q, k, a, mask)
+        if entry == "sdpa":
+            got = ops.sdpa(q, k, a, mask)
+        else:
+            S3 = ctypes.c_int64 * 3
+            sq, sk, so = S3(0, n * 64, 64), S3(0, m * 64, 64), S3(0, 64, h * 64)
+            d = [to_device(t) for t in (q, k, a)]
+            if entry == "attention_x3":
+                y = empty((n, h, 64))
+                _lib.call(entry, *(t.ptr for t in d), y.ptr, 1, h, hk, n, m, 64, sq, sk, sk, so, 0.125, *code, None)
+                got = y.numpy()
+            else:
+                ne = ctypes.c_int64()
+                _lib.call("x3_frag_elems", n, 64 * h, ctypes.byref(ne))
+                p = empty((ne.value,), np.uint16)
+                _lib.call(entry, *(t.ptr for t in d), p.ptr, 1, h, hk, n, m, 64, sq, sk, sk, 0.125, *code, None)
+                with np.errstate(invalid="ignore"):
+                    f = bf16_value(p.numpy()).reshape(3, -1, 4 * h, 2, 32, 8).astype(np.float64).sum(0)
+                got = f.transpose(0, 3, 1, 2, 4).reshape(-1, h, 64)[:n]
+            got = got.transpose(1, 0, 2)
+        keep = np.isfinite(want)
+        if entry == "sdpa":
+            np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
+            np.testing.assert_array_equal(got[np.isinf(want)], want[np.isinf(want)])
+        else:   # an infinity that a query sees has no planes: NaN
+            np.testing.assert_array_equal(np.isfinite(got), keep)
+        assert not keep.any() or np.abs(got[keep] - want[keep]).max() <= 2e-6 * max(1.0, np.abs(want[keep]).max())
