@@ -277,32 +277,40 @@ __global__ __launch_bounds__(256 * NKG) void k_flash64(AttnParams p, int nq) {
     for (int i = 0; i < 4; ++i) orow[db * 16 + 4 * g + i] = oacc[db][i] / l_tot;
 }
 
-// One query of any head dim <= 256 by one wave, 64 keys per step; qs: the scaled query in LDS.  EVERY: values before
-// the first key it sees count too, with probability zero (an infinity or NaN among them makes the output NaN).
-template <bool EVERY>
+__device__ __forceinline__ float wave_total(float v) { return wave_sum(v); }
+__device__ __forceinline__ double wave_total(double v) { return wave_sum_d(v); }
+__device__ __forceinline__ float wave_most(float v) { return wave_max(v); }
+__device__ __forceinline__ double wave_most(double v) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, kWave));
+  return v;
+}
+
+// One query of any head dim <= 256 by one wave, 64 keys per step; qs: the scaled query in LDS; T: the sums' type.
+// EVERY: values before the first key it sees count too, with probability zero (an infinity or NaN among them makes
+// the output NaN).
+template <bool EVERY, typename T>
 __device__ __forceinline__ void attend_row(const AttnParams& p, int b, int hq, int hkv, int64_t qi, int lane, const float* qs) {
   const float* kbase = p.k + b * p.k_sb + hkv * p.k_sh;
   const float* vbase = p.v + b * p.v_sb + hkv * p.v_sh;
-  float acc[4] = {0.f, 0.f, 0.f, 0.f};
-  float m_run = -INFINITY, l_run = 0.f;
+  T acc[4] = {0, 0, 0, 0};
+  T m_run = -INFINITY, l_run = 0;
   int64_t klo, khi;
   visible_keys(p, qi, klo, khi);
   for (int64_t c0 = 0; c0 < p.m; c0 += 64) {
     const int64_t kj = c0 + lane;
-    float s = -INFINITY;
+    T s = -INFINITY;
     if (kj >= klo && kj < khi) {
       const float* kr = kbase + kj * p.k_sm;
-      float t = 0.f;
-      for (int d = 0; d < p.d; ++d) t = fmaf(qs[d], kr[d], t);
-      s = t;
+      s = 0;
+      for (int d = 0; d < p.d; ++d) s = fma((T)qs[d], (T)kr[d], s);
     }
-    const float mx = wave_max(s);
-    const float m_new = fmaxf(m_run, mx);
+    const T m_new = max(m_run, wave_most(s));
     const bool none = m_new == -INFINITY;
     if (!EVERY && none) continue;
-    const float alpha = none ? 1.f : expf(m_run - m_new);
-    const float pj = none ? 0.f : expf(s - m_new);
-    l_run = l_run * alpha + wave_sum(pj);
+    const float alpha = none ? 1.f : expf((float)(m_run - m_new));
+    const float pj = none ? 0.f : expf((float)(s - m_new));
+    l_run = l_run * alpha + wave_total((T)pj);
 #pragma unroll
     for (int r = 0; r < 4; ++r) acc[r] *= alpha;
     const int64_t cnt = p.m - c0 < 64 ? p.m - c0 : 64;
@@ -312,7 +320,7 @@ __device__ __forceinline__ void attend_row(const AttnParams& p, int b, int hq, i
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int d = lane + 64 * r;
-        if (d < p.d) acc[r] = fmaf(pb, vr[d], acc[r]);
+        if (d < p.d) acc[r] = fma((T)pb, (T)vr[d], acc[r]);
       }
     }
     m_run = m_new;
@@ -321,7 +329,7 @@ __device__ __forceinline__ void attend_row(const AttnParams& p, int b, int hq, i
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const int d = lane + 64 * r;
-    if (d < p.d) orow[d] = acc[r] / l_run;
+    if (d < p.d) orow[d] = (float)(acc[r] / l_run);
   }
 }
 
@@ -367,7 +375,8 @@ __device__ __forceinline__ void mfma6(const bf16x8_t& ah, const bf16x8_t& am, co
 
 // A stage that no query of the workgroup sees is skipped, but for its values' exponents: a masked key counts with
 // probability zero, and zero times an infinity or NaN is NaN in that dim of every output, whichever tile it is in.
-// AGAIN: outputs that come out not finite are formed again in float32.
+// AGAIN: outputs that come out not finite, or smaller than planes of the values hold in full, are formed again from
+// the floats, with sums in 64 bits (a lone wave's serial sums in 32 were off by 1.4e-6, the tiles' are by 4e-7).
 template <int QWN, bool AGAIN>
 __global__ __launch_bounds__(512) void k_flash64x(AttnParams p, int nq) {
   constexpr int NKG = 8 / QWN, NS = QWN, WKT = 16 * NS;  // key groups; a group's sub-tiles and keys
@@ -647,11 +656,12 @@ __global__ __launch_bounds__(512) void k_flash64x(AttnParams p, int nq) {
       for (int i = 0; i < 4; ++i) {
         const float y = value(db, i);
         orow[db * 16 + 4 * g + i] = y;
-        bad |= !(fabsf(y) <= 3.4028235e38f);
+        bad |= !in_range(magnitude(y));
       }
   }
   if constexpr (AGAIN) {
-    // infinities and the largest floats have no planes (inf - inf): the whole wave does those queries again
+    // infinities and the largest floats have no planes here (inf - inf), values below 2^-110 not all their bits: the
+    // whole wave does those queries again
     uint64_t todo = __ballot(bad);
     todo = (todo | todo >> 16 | todo >> 32 | todo >> 48) & 0xffff;
     float* qs = reinterpret_cast<float*>(&Vs[0][0][0]) + 64 * qw;
@@ -660,7 +670,7 @@ __global__ __launch_bounds__(512) void k_flash64x(AttnParams p, int nq) {
       todo &= todo - 1;
       qs[lane] = p.q[b * p.q_sb + hq * p.q_sh + row * p.q_sn + lane] * p.scale;
       __builtin_amdgcn_wave_barrier();
-      attend_row<true>(p, b, hq, hkv, row, lane, qs);
+      attend_row<true, double>(p, b, hq, hkv, row, lane, qs);
       __builtin_amdgcn_wave_barrier();
     }
   }
@@ -679,7 +689,7 @@ __global__ __launch_bounds__(256) void k_attn_generic(AttnParams p) {
   for (int d = lane; d < p.d; d += 64) qs[d] = qvalid ? qrow[d] * p.scale : 0.f;
   __syncthreads();
   if (!qvalid) return;
-  attend_row<false>(p, b, hq, hkv, qi, lane, qs);
+  attend_row<false, float>(p, b, hq, hkv, qi, lane, qs);
 }
 
 }  // namespace

@@ -1,7 +1,10 @@
 // Three-plane bfloat16 form of float32 values: x = hi + mid + lo, each plane the
 // round-to-nearest bfloat16 of what the planes before it leave.  Each residual is
 // exact in float32 (x minus a rounding of x to fewer bits), so |x - (hi + mid + lo)|
-// <= 2^-8 |x - hi - mid| <= 2^-24 |x|: the planes carry all 24 bits of the float.
+// <= 2^-8 |x - hi - mid| <= 2^-24 |x|: the planes carry all 24 bits of the float, from 2^-110 up.
+// Below, the last bits fall under the smallest bfloat16 and |x - (hi + mid + lo)| <= 2^-134 instead:
+// 2e-6 of a value of 2^-116, 4e-5 of one of 2^-120 (the matrix cores keep subnormal operands).
+// ops.linear and ops.sdpa form such outputs again in float32; the models' own layers do not.
 // A product a.b is then the six plane products whose weights reach 2^-16
 // (hh, hm, mh, hl, mm, lh), each exact in the matrix core's float32 accumulate;
 // the three dropped (ml, lm, ll) weigh at most ~2^-23 |a b|.
@@ -64,6 +67,16 @@ __device__ __forceinline__ void split_x3_full(const float4& a, const float4& b, 
     m[i] = p[0][1] | (uint32_t)p[1][1] << 16;
     l[i] = p[0][2] | (uint32_t)p[1][2] << 16;
   }
+}
+
+// Whether outputs of one row are what planes give in full: all finite, and all zero or one of 2^-90 or more.
+__device__ __forceinline__ bool in_range(uint32_t largest) {
+  const uint32_t low = (127u - 90u) << 23;
+  return largest == 0 || largest - low <= 0x7f7fffffu - low;
+}
+__device__ __forceinline__ uint32_t magnitude(float v) { return __float_as_uint(v) & 0x7fffffffu; }
+__device__ __forceinline__ bool in_range(const float4& v) {
+  return in_range(max(max(magnitude(v.x), magnitude(v.y)), max(magnitude(v.z), magnitude(v.w))));
 }
 
 // Scheduling groups: R times, N1 instructions of class M1, then N2 of class M2 (0x8 MFMA, 0x20 VMEM read,

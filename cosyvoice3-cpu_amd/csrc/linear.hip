@@ -1,6 +1,8 @@
 // ops.linear / quant.qmatmul entry points (cv3cpu/ops.py:121-123,
 // cv3cpu/quant.py:156-204): GEMV for up to four activation rows, the MFMA GEMM
 // above that (fp32, q8 and q4 weights alike).
+#include <algorithm>
+
 #include "common.hpp"
 
 namespace cv3 {
@@ -32,6 +34,21 @@ int gemm_x3q(const float* a, int64_t m, int64_t k, int64_t lda, const int8_t* q,
 }  // namespace cv3
 
 using namespace cv3;
+
+namespace {
+
+// Sets *small if a row's largest magnitude lies above zero and below 2^-80.  One wave a row.
+__global__ __launch_bounds__(256) void k_rows_fit(const float* w, int64_t n, int64_t k, int64_t ldw, int* small) {
+  const int lane = threadIdx.x & 63;
+  for (int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); row < n; row += (int64_t)gridDim.x * 4) {
+    float most = 0.f;
+    for (int64_t j = lane; j < k; j += 64) most = fmaxf(most, fabsf(w[row * ldw + j]));
+    most = wave_max(most);
+    if (lane == 0 && most > 0.f && most < 8.2718061255302767e-25f) atomicOr(small, 1);
+  }
+}
+
+}  // namespace
 
 static constexpr int64_t kGemvRows = 4;  // quant.py:43 THREAD_ROW_LIMIT: the decode regime
 
@@ -99,6 +116,29 @@ int cv3_split_x3_frag(const float* w, int64_t n, int64_t k, int64_t ldw, uint16_
   CV3_REQUIRE(n >= 0 && k > 0 && ldw >= k, CV3_EINVAL, "bad plane split shape n=%lld k=%lld", (long long)n,
               (long long)k);
   return split_x3_frag(w, n, k, ldw, frag, stream_of(s));
+}
+
+int cv3_x3_rows_fit(const float* w, int64_t n, int64_t k, int64_t ldw, int* fit, cv3_stream_t s) {
+  CV3_ALIVE();
+  CV3_REQUIRE(fit && n >= 0 && k > 0 && ldw >= k && (w || !n), CV3_EINVAL, "bad row check shape n=%lld k=%lld", (long long)n,
+              (long long)k);
+  *fit = 1;
+  if (!n) return CV3_OK;
+  hipStream_t st = stream_of(s);
+  CV3_REQUIRE(st, CV3_EHIP, "no stream");
+  void* flag = nullptr;
+  int rc = scratch_alloc(&flag, sizeof(int), st);
+  if (rc) return rc;
+  rc = cv3_fill_zero(flag, sizeof(int), reinterpret_cast<cv3_stream_t>(st));
+  if (!rc) {
+    hipLaunchKernelGGL(k_rows_fit, dim3((unsigned)std::min<int64_t>(ceil_div(n, 4), 65536)), dim3(256), 0, st, w, n, k, ldw,
+                       reinterpret_cast<int*>(flag));
+    int small = 0;
+    rc = cv3_copy_d2h(&small, flag, sizeof(int), reinterpret_cast<cv3_stream_t>(st));
+    *fit = !small;
+  }
+  const int rf = scratch_free(flag, st);
+  return rc ? rc : rf;
 }
 
 int cv3_x3_frag_elems(int64_t n, int64_t k, int64_t* elems) {

@@ -58,9 +58,10 @@ struct PlaneParams {
   float *kc, *vc;
   int heads, kv_heads, cap, pos0;
   const float *cos, *sin;  // [cap][64]
-  // the float32 rows x was split from, or null: an infinity and the largest floats have no planes (inf - inf),
-  // and code products may pass the range before their scale: outputs that come out not finite are formed
-  // again from these
+  // the float32 rows x was split from, or null.  Outputs that come out not finite are formed again from these:
+  // an infinity times a plane of zero is NaN, and code products may pass the range before their scale.  So are
+  // those below 2^-90: rows below 2^-110 have fewer than 24 bits in their planes, which shows (2^-134 an element)
+  // only in outputs this small, unless an output's weights sum to more than 2^20.
   const float* fx;
   int64_t ldfx;
   int tiles_m, tiles_n, gm;
@@ -276,11 +277,19 @@ struct PlaneEpilogue {
     for (int q = 0; q < G; ++q) {
       if constexpr (KIND == W_ROW)
         v[q] = make_float4(v[q].x * scale[q].x, v[q].y * scale[q].y, v[q].z * scale[q].z, v[q].w * scale[q].w);
-      if (p.fx) {
-        const float top = 3.4028235e38f;
-        const bool fine = fabsf(v[q].x) <= top && fabsf(v[q].y) <= top && fabsf(v[q].z) <= top && fabsf(v[q].w) <= top;
-        if (!fine && m[q] < p.m && n[q] < p.n) v[q] = again(p, m[q], n[q], scale[q]);
+    }
+    if (p.fx) {  // a row's four outputs are small together: its rows' fault (a weight's such rows have no planes)
+      bool fine = true;
+#pragma unroll
+      for (int q = 0; q < G; ++q) fine &= in_range(v[q]);
+      if (!fine) {
+#pragma unroll
+        for (int q = 0; q < G; ++q)
+          if (!in_range(v[q]) && m[q] < p.m && n[q] < p.n) v[q] = again(p, m[q], n[q], scale[q]);
       }
+    }
+#pragma unroll
+    for (int q = 0; q < G; ++q) {
       if (p.bias) v[q] = make_float4(v[q].x + bias[q].x, v[q].y + bias[q].y, v[q].z + bias[q].z, v[q].w + bias[q].w);
     }
     if constexpr (ACT == A_QKV) return store_qkv(p, v);

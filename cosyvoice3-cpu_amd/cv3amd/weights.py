@@ -102,8 +102,8 @@ def device_planes(weight, dev) -> Optional[DevicePlanes]:
     take, for K up to 512 (two launches: 10.7 us against 8.6 of the one float32 kernel at K = 256, within 15 %
     of each other either way at 512, 13.5 against 21.5 at 1024, whatever m; q8 more), for a first use inside
     a capture (packing waits for the device), for weights that are not cached: a writeable array, or one
-    that lives on the device (its owner may write to it between calls), and for a weight whose planes found no
-    memory (6 bytes a float32 weight, 2 a code)."""
+    that lives on the device (its owner may write to it between calls), for a weight whose planes found no
+    memory (6 bytes a float32 weight, 2 a code), and for one with a row too small for them (cv3_x3_rows_fit)."""
     quantised = isinstance(dev, DeviceQ)
     if quantised:
         cached = not isinstance(weight.q, DeviceArray) and not isinstance(weight.scales, DeviceArray)
@@ -139,6 +139,11 @@ def _pack_planes(dev, n: int, k: int, block: int) -> Optional[DevicePlanes]:
     else:
         _lib.call("x3_frag_elems", n, k, ctypes.addressof(ne))
     try:
+        if not quantised:
+            fit = ctypes.c_int()
+            _lib.call("x3_rows_fit", dev.ptr, n, k, k, ctypes.addressof(fit), None)
+            if not fit.value:
+                return None
         frag = DeviceArray((ne.value,), np.uint16)
         scales = DeviceArray((ns.value,)) if quantised else None
     except _lib.HIPError:

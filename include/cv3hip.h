@@ -153,6 +153,9 @@ int cv3_linear_x3(const float* x, int64_t m, int64_t k, int64_t ldx, const uint1
  * same bits as cv3_linear_x3 on the same weight.  K % 64 == 0, 16-byte aligned rows. */
 int cv3_split_x3_frag(const float* w, int64_t n, int64_t k, int64_t ldw, uint16_t* frag, cv3_stream_t s);
 int cv3_x3_frag_elems(int64_t n, int64_t k, int64_t* elems);
+/* *fit (host) = 1 if no row's largest magnitude lies above zero and below 2^-80: what planes hold of such rows'
+ * smaller elements, and of products that small, is less than the 24 bits of a float (below 2^-110).  Waits for s. */
+int cv3_x3_rows_fit(const float* w, int64_t n, int64_t k, int64_t ldw, int* fit, cv3_stream_t s);
 int cv3_linear_x3_frag(const float* x, int64_t m, int64_t k, int64_t ldx, const uint16_t* frag, int64_t n,
                        const float* bias, float* y, int64_t ldy, const cv3_epilogue* epi, cv3_stream_t s);
 /* quant.qmatmul on q8 weights (quant.py:165-190) on the bfloat16 matrix cores: the activation as
@@ -207,8 +210,8 @@ int cv3_linear_code_planes(const uint16_t* x, int64_t m, int64_t k, const uint16
 /* ops.linear (ops.py:121-123, quant.py:156-204) on float32 rows with such a weight: x is split into planes in a
  * workspace of the caching allocator, then multiplied as above.  kind: the weight's (float32 planes of
  * cv3_split_x3_frag, or codes).  Infinities and the largest floats, in rows or a float32
- * weight, give what float32 products of them give.  The workspace is
- * the call's own: ordered on s, whichever stream that is, and the graph's if s is capturing.  CV3_ENOMEM if there
+ * weight, give what float32 products of them give, and so do rows too small for their planes (outputs below 2^-90,
+ * before the bias, are formed again; a weight's rows: cv3_x3_rows_fit).  The workspace is the call's own: ordered on s, whichever stream that is, and the graph's if s is capturing.  CV3_ENOMEM if there
  * is none to be had (a capture takes it from the cache only): the float32 kernels need no workspace. */
 int cv3_linear_rows_planes(int kind, const float* x, int64_t m, int64_t k, int64_t ldx, const uint16_t* frag,
                            const float* scales_t, int64_t block, int64_t n, const float* bias, float* y, int64_t ldy,
@@ -302,7 +305,7 @@ int cv3_attention_x3(const float* q, const float* k, const float* v, float* out,
                      const int64_t* v_strides, const int64_t* o_strides, float scale, int mask_kind,
                      int64_t mask_a, int64_t mask_b, cv3_stream_t s);
 /* ops.sdpa itself: contiguous (h, n, d) and (hk, m, d), as cv3_attention_x3.  Outputs that come out not finite
- * are formed again in float32, so infinities give what float32 products of them give: a masked key counts with
+ * or below 2^-90 are formed again from the floats, so infinities give what float32 products of them give: a masked key counts with
  * probability zero, so an infinity or NaN among its values is NaN in that dim of the head's outputs. */
 int cv3_sdpa(const float* q, const float* k, const float* v, float* out, int h, int hk, int64_t n, int64_t m, int d,
              float scale, int mask_kind, int64_t mask_a, int64_t mask_b, cv3_stream_t s);

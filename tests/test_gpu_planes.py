@@ -266,6 +266,49 @@ def test_drop_in_linear_with_a_weight_past_bfloat16(lib, m, k, n):
     np.testing.assert_array_equal(back[np.isinf(w)], w[np.isinf(w)])
 
 
+@pytest.mark.parametrize("kind", ["f32", "q8_rows", "q8_block", "q4"])
+@pytest.mark.parametrize("m,k,n", [(5, 640, 64), (70, 1024, 96), (1500, 640, 1152)])
+def test_drop_in_linear_below_the_planes_range(lib, m, k, n, kind):
+    """Rows, and rows of a float32 weight, whose planes hold fewer than 24 bits: within the float32 kernels' error
+    of float64 (their sums of k terms; 9e-7 measured), row by row, beside ordinary rows and zeros."""
+    import cv3amd.ops as ops
+    import cv3amd.quant as quant
+    _lib, to_device, empty = lib
+    rng = np.random.default_rng([m, k])
+    x, w = rng.normal(size=(m, k)).astype(np.float32), rng.normal(size=(n, k)).astype(np.float32)
+    for r, e in enumerate((0, -89, -104, -111, -116)):
+        x[r] *= np.float32(2.0 ** e)
+    x[m - 1, :k // 2] = 0.0
+    if kind == "f32":
+        small = w.copy()
+        small[1] *= np.float32(2.0 ** -118)
+        small[2] = 0.0
+        cases = [(w, w.astype(np.float64)), (small, small.astype(np.float64))]
+        for a, _ in cases:
+            a.flags.writeable = False
+    else:
+        if kind == "q4":
+            q, s, _ = quant.quantize_q4(w)
+            block = 32
+        else:
+            block = 64 if kind == "q8_block" else k
+            q, s, _ = quant.quantize_q8(w, block, np.float16 if kind == "q8_block" else np.float32)
+        t = quant.QTensor("q4" if kind == "q4" else "q8", q, s, (n, k), block)
+        cases = [(t, t.dequant().astype(np.float64))]
+    for a, w64 in cases:
+        got, want = ops.linear(to_device(x), a).numpy(), x.astype(np.float64) @ w64.T
+        for r in range(m):
+            for c0, c1 in ((0, 1), (1, 2), (2, 3), (3, n)):
+                if np.abs(want[r, c0:c1]).max() > 1e-36:    # float32's own subnormals aside
+                    assert rel_rows(got[r, c0:c1], want[r, c0:c1], x[r], w64[c0:c1]) < 2e-6, (r, c0)
+        assert not got[:, 2].any() or w64[2].any()
+
+
+def rel_rows(got, want, x, w64):
+    """max |error| over sum |x| |w|, the scale that rounding errors of a sum follow."""
+    return float((np.abs(got - want) / (np.abs(x.astype(np.float64)) @ np.abs(w64).T)).max())
+
+
 def test_drop_in_linear_first_used_in_a_capture(lib):
     """A weight that a capture meets first keeps the float32 kernel there; its planes come with the next
     eager call, and both give the same layer."""
