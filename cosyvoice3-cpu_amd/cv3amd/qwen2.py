@@ -175,11 +175,16 @@ class _Stacked:
 class DeviceQwen2:
     """Qwen2 body + CosyVoice3 LM head resident on the device, decoding greedily."""
 
-    def __init__(self, weights, prefix: str = "llm.", cap: int = 1024, widen_q4: bool = False):
+    def __init__(self, weights, prefix: str = "llm.", cap: int = 1024, widen_q4: bool = False,
+                 prompt_planes: bool = True):
         """A q4 body (the tiny profile) is held in HBM as the checkpoint's packed nibbles; the
         one-launch step decodes it at the int8 body's rate.  ``widen_q4`` holds it as int8
         codes with the same blocks and scales instead (identical weights, twice the bytes),
-        which the five-kernel step reads a little faster."""
+        which the five-kernel step reads a little faster.
+
+        ``prompt_planes`` keeps the body a second time, laid out for ``prefill`` at two bytes a code
+        (``prompt_nbytes``: 0.72 GB for Qwen2-0.5B beside 0.2 - 0.4 GB).  Without it, or without the
+        memory for it, prompts run on the decode's rows (500 tokens 8.2 ms against 2.7)."""
         _lib.init()
         m = weights.meta["qwen2"]
         self.layers = int(m["num_hidden_layers"])
@@ -230,7 +235,12 @@ class DeviceQwen2:
         p0 = self.ints.ptr
         self.state = State(self.k_cache.ptr, self.v_cache.ptr, self.cap, p0, p0 + 8, p0 + 16, self.x.ptr,
                            self.logits.ptr, self.workspace.ptr, nws)
-        self._prompt = self._prompt_planes()
+        self._prompt, self._prompt_arrays = None, []
+        if prompt_planes:
+            try:
+                self._prompt = self._prompt_planes()
+            except _lib.HIPError:    # out of memory
+                self._prompt_arrays = []
         self._graph: Optional[Graph] = None
         self._pos_host = 0
         # sampler control block: [start, stop step + 1, PCG64 state hi, lo, inc hi, lo]
@@ -253,7 +263,7 @@ class DeviceQwen2:
         if not ok:
             return None
         turned = (self.heads + self.kv_heads) * dh
-        p, self._prompt_arrays = Planes(), []
+        p = Planes()
         for name, w, span, limit in (("qkv", self.qkv, dh, turned), ("o", self.o, 0, 0),
                                      ("gate_up", self.gate_up, 2 * I, 2 * I), ("down", self.down, 0, 0)):
             frag, scales = w.planes(span, limit)
@@ -265,6 +275,11 @@ class DeviceQwen2:
         self._prompt_arrays.append(bias)
         p.qkv_bias = bias.ptr
         return p
+
+    @property
+    def prompt_nbytes(self) -> int:
+        """Bytes held in HBM for ``prefill`` alone."""
+        return sum(a.nbytes for a in self._prompt_arrays)
 
     # -- weights streamed per token (the HBM roofline numerator) -----------
     def bytes_per_token(self, length: int) -> dict:

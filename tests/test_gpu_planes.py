@@ -195,6 +195,34 @@ def test_prompt_on_code_planes(gpu, profile, t, pos0):
     assert not got[0][1][:, :, pos0 + t:].any() and not got[0][2][:, :, pos0 + t:].any()
 
 
+@pytest.mark.parametrize("why", ["asked", "memory"])
+def test_prompt_without_its_planes(gpu, monkeypatch, why):
+    """The LM without the prompt's second copy of the body, by choice or for want of memory: the same logits from
+    the decode's rows."""
+    import cv3amd.quant as quant
+    from cv3amd import _lib, qwen2, synth
+    from cv3amd.weights import WeightStore
+    tensors = synth.quantize_store(synth.qwen2_tensors(layers=2), "per_channel", quant.quantize_q8, quant.quantize_q4)
+    store = WeightStore(dict(tensors), synth.qwen2_meta(layers=2), quant.QTensor)
+    x = np.random.default_rng(8).normal(size=(37, 896)).astype(np.float32)
+    full = qwen2.DeviceQwen2(store, cap=64)
+    body, rows = 2 * (1152 * 896 + 896 * 896 + 9728 * 896 + 896 * 4864), 2 * (1152 + 896 + 9728 + 896)
+    assert full.prompt_nbytes == 2 * body + 4 * rows + 4 * 2 * 1152    # codes, a scale a row, the bias of qkv
+    if why == "memory":
+        real = qwen2._Stacked.planes
+
+        def planes(self, *a):
+            if self.k == 4864:
+                raise _lib.HIPError("hipMalloc failed")
+            return real(self, *a)
+        monkeypatch.setattr(qwen2._Stacked, "planes", planes)
+    bare = qwen2.DeviceQwen2(store, cap=64, prompt_planes=why != "asked")
+    assert bare._prompt is None and bare.prompt_nbytes == 0
+    full.prefill(x, 0)
+    bare.prefill(x, 0)
+    assert rel_err(bare.logits.numpy(), full.logits.numpy()) < TOL
+
+
 @pytest.mark.parametrize("kind", ["f32", "q8_rows", "q8_block", "q4"])
 @pytest.mark.parametrize("m,k,n", [(5, 576, 64), (33, 896, 1152), (130, 1024, 68), (331, 1024, 2048), (40, 4864, 896)])
 def test_drop_in_linear_on_planes(lib, m, k, n, kind):
