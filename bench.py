@@ -366,7 +366,10 @@ def bench_flow(args, tensors, meta):
     M, K, N = 2 * T, d.dim, 3 * d.dim
     def qkv_sweep():
         for i in range(d.depth):
-            d.qkv[i](d.n.ptr, M, K, d.qkvb.ptr, N)
+            if d.qkv_frag:    # as the solve runs it: the norm leaves planes
+                d.qkv[i].from_planes(d.np[0].ptr, M, d.qkvb.ptr, N)
+            else:
+                d.qkv[i](d.n.ptr, M, K, d.qkvb.ptr, N)
     run = replayer(args.graph, qkv_sweep)
     run()
     synchronize()
@@ -378,7 +381,7 @@ def bench_flow(args, tensors, meta):
     kflops = 2.0 * M * N * K
     log(f"flow: QKV GEMM {kms * 1e3:.1f} us/launch, {kflops / (kms / 1e3) / 1e12:.1f} TFLOP/s")
     planes = d.qkv[0].planes is not None if d.depth else False
-    name = ("k_gemm_x3f (float32 GEMM as six bfloat16 plane products, weight fragments straight to registers, "
+    name = ("plane linear (float32 GEMM as six bfloat16 plane products, both operands as planes in fragment order, "
             "fused QKV 1000x3072x1024)" if planes
             else "k_gemm<0> (fp32 MFMA GEMM, fused QKV 1000x3072x1024)")
     return {"ms": ms, "flops": flops, "by_unit": by_unit, "T": T, "depth": d.depth,
@@ -473,7 +476,6 @@ def bench_kernels(args):
     f4 = 4
     S3 = ctypes.c_int64 * 3
     qs = S3(T * 3 * D, dh, 3 * D)
-    os_ = S3(T * D, dh, D)
     scale = float(np.float32(1.0 / math.sqrt(dh)))
     rope_epi = _lib.epilogue(rope=(d.cos.ptr, d.sin.ptr, T, D, dh, 2 * D))
     g = d.mods.ptr   # any AdaLN row: the timing does not depend on its values
@@ -484,25 +486,27 @@ def bench_kernels(args):
     lin_peak, lin_unit = ((SPLIT_BF16_PEAK, "split-bf16") if d.qkv[0].planes is not None
                           else (FP32_MFMA_PEAK, "fp32 MFMA"))
     f32 = (FP32_MFMA_PEAK, "fp32 MFMA")
+    if not (d.qkv_frag and d.out_frag and d.ff2_frag):
+        raise RuntimeError("the block's launches are timed as the solve makes them, on activation planes")
+    nx, ax, fx = d.np[0].ptr, d.attp[0].ptr, d.ffp[0].ptr   # norm, attention and feed-forward planes
+    gelu = _lib.epilogue("gelu_tanh")
     launches = {
-        "layer_norm + AdaLN [1000, 1024]": (
-            lambda: _lib.call("layer_norm", d.h.ptr, d.n.ptr, BT, D, 1e-6, None, None, g, g + D * f4, 0, 0, None),
-            None, None),
-        f"QKV GEMM [{BT}, {D}] x [{3 * D}, {D}]^T + rotary": (
-            lambda: d.qkv[0](d.n.ptr, BT, D, d.qkvb.ptr, 3 * D, rope_epi), 2.0 * BT * 3 * D * D, (lin_peak, lin_unit)),
-        f"QKV GEMM [{BT}, {D}] x [{3 * D}, {D}]^T, bias only": (
-            lambda: d.qkv[0](d.n.ptr, BT, D, d.qkvb.ptr, 3 * D), 2.0 * BT * 3 * D * D, (lin_peak, lin_unit)),
-        f"flash attention B={B} H={H} T={T} d={dh}": (
-            lambda: _lib.call("attention_x3" if d.planes else "attention", d.qkvb.ptr, d.qkvb.ptr + D * f4,
-                              d.qkvb.ptr + 2 * D * f4, d.att.ptr, B, H, H, T, T, dh, qs, qs, qs, os_, scale, 0, 0, 0,
-                              None), 4.0 * B * H * T * T * dh, (lin_peak, lin_unit)),
-        f"out GEMM [{BT}, {D}] x [{D}, {D}]^T + gated residual": (
-            lambda: d.out[0](d.att.ptr, BT, D, d.z1.ptr, D, res_epi), 2.0 * BT * D * D, (lin_peak, lin_unit)),
-        f"ff1 GEMM [{BT}, {D}] x [{F}, {D}]^T + GELU": (
-            lambda: d.ff1[0](d.n.ptr, BT, D, d.ffb.ptr, F, _lib.epilogue("gelu_tanh")), 2.0 * BT * F * D,
+        "layer_norm + AdaLN [1000, 1024] into planes": (
+            lambda: _lib.call("layer_norm_planes", d.h.ptr, nx, BT, D, 1e-6, g, g + D * f4, None), None, None),
+        f"QKV linear [{BT}, {D}] x [{3 * D}, {D}]^T + rotary": (
+            lambda: d.qkv[0].from_planes(nx, BT, d.qkvb.ptr, 3 * D, epi=rope_epi), 2.0 * BT * 3 * D * D,
             (lin_peak, lin_unit)),
-        f"ff2 GEMM [{BT}, {F}] x [{D}, {F}]^T + gated residual": (
-            lambda: d.ff2[0](d.ffb.ptr, BT, F, d.z1.ptr, D, res_epi), 2.0 * BT * D * F, (lin_peak, lin_unit)),
+        f"QKV linear [{BT}, {D}] x [{3 * D}, {D}]^T, bias only": (
+            lambda: d.qkv[0].from_planes(nx, BT, d.qkvb.ptr, 3 * D), 2.0 * BT * 3 * D * D, (lin_peak, lin_unit)),
+        f"flash attention B={B} H={H} T={T} d={dh} into planes": (
+            lambda: _lib.call("attention_x3_planes", d.qkvb.ptr, d.qkvb.ptr + D * f4, d.qkvb.ptr + 2 * D * f4, ax, B, H, H,
+                              T, T, dh, qs, qs, qs, scale, 0, 0, 0, None), 4.0 * B * H * T * T * dh, (lin_peak, lin_unit)),
+        f"out linear [{BT}, {D}] x [{D}, {D}]^T + gated residual": (
+            lambda: d.out[0].from_planes(ax, BT, d.z1.ptr, D, epi=res_epi), 2.0 * BT * D * D, (lin_peak, lin_unit)),
+        f"ff1 linear [{BT}, {D}] x [{F}, {D}]^T + GELU into planes": (
+            lambda: d.ff1[0].from_planes(nx, BT, y_planes=fx, epi=gelu), 2.0 * BT * F * D, (lin_peak, lin_unit)),
+        f"ff2 linear [{BT}, {F}] x [{D}, {F}]^T + gated residual": (
+            lambda: d.ff2[0].from_planes(fx, BT, d.z1.ptr, D, epi=res_epi), 2.0 * BT * D * F, (lin_peak, lin_unit)),
         f"grouped causal conv k={k} groups={d.conv_groups} [{B}, {T}, {D}] + Mish": (
             lambda: _lib.call("conv1d_cl_x3f" if d.conv_planes else "conv1d_cl", d.h.ptr, B, T, D, D,
                               d.conv_w[0].ptr, D, k, d.conv_groups, k - 1, d.conv_b[0].ptr, d.z1.ptr, D,

@@ -90,7 +90,7 @@ class DeviceLinear:
     ``frag_x=True`` also readies the weight for activations that come as bfloat16 planes in fragment
     order (``from_planes``, cv3_linear_x3_planes / cv3_linear_code_planes), where ``takes_planes`` says
     it can: float32 planes as they are, q8 codes (64-code blocks or one scale a row) widened to
-    bfloat16 beside the packed codes.
+    bfloat16 beside the packed codes.  ``keep`` leaves the one of the two that its caller reads.
     """
 
     def __init__(self, weights: List[object], biases: List[Optional[np.ndarray]], planes: bool = False,
@@ -98,6 +98,7 @@ class DeviceLinear:
         ws = list(weights)
         self.planes = None
         self.codes16: Optional[DeviceArray] = None
+        self.scales_t: Optional[DeviceArray] = None
         self.rexp: Optional[DeviceArray] = None
         if all(_is_q(w) for w in ws):
             kinds = {w.kind for w in ws}
@@ -181,11 +182,20 @@ class DeviceLinear:
             _lib.call("linear_x3_planes", x, m, self.k, self.planes.ptr, self.n, b, y, ldy, y_planes, e,
                       plan_rows, st)
 
+    def keep(self, planes: bool):
+        """Release what a q8 linear holds for the other kind of activation: planes (True) or float rows."""
+        if self.codes16 is None:
+            return
+        if planes:
+            self.q = self.scales = None
+        else:
+            self.codes16 = self.scales_t = None
+            self.takes_planes = False
+
     @property
     def nbytes(self) -> int:
         if self.q8:
-            wide = self.codes16.nbytes + self.scales_t.nbytes if self.codes16 is not None else 0
-            return self.q.nbytes + self.scales.nbytes + wide
+            return sum(a.nbytes for a in (self.q, self.scales, self.codes16, self.scales_t) if a is not None)
         return self.planes.nbytes if self.planes is not None else self.w.nbytes
 
     def __call__(self, x: int, m: int, ldx: int, y: int, ldy: int, epi=None, rexp_given: bool = False,
@@ -195,6 +205,8 @@ class DeviceLinear:
         (cv3_layer_norm_rexp); ``st``: a stream handle (None: the calling thread's)."""
         b = self.bias.ptr if self.bias is not None else None
         e = ctypes.byref(epi) if epi is not None else None
+        if self.q8 and self.q is None:
+            raise ValueError("this linear was kept for activations in planes (from_planes)")
         if self.q8_digits:
             if self.rexp is None or self.rexp.size < rexp_row0 + m:
                 raise ValueError("the digit-plane linear needs an int32 workspace of m entries (rexp)")
@@ -323,6 +335,10 @@ class DeviceDiT:
                          and all(lin.takes_planes for lin in self.out))
         self.ff2_frag = self.ff1_frag and self.ff_dim % 16 == 0 and all(lin.takes_planes for lin in self.ff2)
         self.proj_out_frag = norms and self.proj_out.takes_planes
+        for lins, planes in ((self.qkv, self.qkv_frag), (self.out, self.out_frag), (self.ff1, self.ff1_frag),
+                             (self.ff2, self.ff2_frag), ([self.proj_out], self.proj_out_frag)):
+            for lin in lins:
+                lin.keep(planes)
         self._T = None
         self._graph = None
         self.halves = False                  # set by prepare() from HALVES and T
@@ -347,14 +363,15 @@ class DeviceDiT:
         if self._T != T:
             self._T = T
             self.h = DeviceArray((B * T, D))
-            self.n = DeviceArray((B * T, D))
             self.qkvb = DeviceArray((B * T, 3 * D))
-            self.att = DeviceArray((B * T, D))
-            self.ffb = DeviceArray((B * T, self.ff_dim))
-            # the same as planes in fragment order, for all rows and for one batch row of its own
-            # (fragments hold 32 rows, so a batch row cannot start inside one)
-            self.np, self.attp, self.ffp = ([self._planes(r, k) for r in (B * T, T)]
-                                            for k in (D, D, self.ff_dim))
+            # norm, attention and feed-forward outputs: float rows, planes in fragment order or both, as
+            # their readers take them
+            norms = (self.qkv_frag, self.ff1_frag, self.proj_out_frag)
+            self.n = None if all(norms) else DeviceArray((B * T, D))
+            self.att = None if self.out_frag else DeviceArray((B * T, D))
+            self.ffb = None if self.ff2_frag else DeviceArray((B * T, self.ff_dim))
+            self.np, self.attp, self.ffp = ([self._planes(B * T, k)] if on else []
+                                            for k, on in ((D, any(norms)), (D, self.out_frag), (self.ff_dim, self.ff2_frag)))
             self.z1 = DeviceArray((B * T, D))
             self.outb = DeviceArray((B * T, mel))
             self.outT = DeviceArray((B, mel, T))
@@ -374,6 +391,14 @@ class DeviceDiT:
         self.stemb = DeviceArray((S, D))
         self.mods = DeviceArray((S, self.ld_mod))
         self._graph = None
+
+    def _row_planes(self):
+        """Planes for a batch row of its own, while the two rows run apart (fragments hold 32 rows, so the second
+        cannot start inside one)."""
+        if self.halves:
+            for held, k in ((self.np, self.dim), (self.attp, self.dim), (self.ffp, self.ff_dim)):
+                if len(held) == 1:
+                    held.append(self._planes(self._T, k))
 
     @staticmethod
     def _planes(rows: int, k: int) -> DeviceArray:
@@ -407,8 +432,9 @@ class DeviceDiT:
         T, D, H, dh, f4 = self._T, self.dim, self.heads, self.dim_head, 4
         S3 = ctypes.c_int64 * 3
         rows = nb * T
-        h, n, att = (a.ptr + f4 * r0 * D for a in (self.h, self.n, self.att))
-        qkvb, ffb = self.qkvb.ptr + f4 * r0 * 3 * D, self.ffb.ptr + f4 * r0 * self.ff_dim
+        h, n, att, qkvb, ffb = (a.ptr + f4 * r0 * w if a is not None else None
+                                for a, w in ((self.h, D), (self.n, D), (self.att, D), (self.qkvb, 3 * D),
+                                             (self.ffb, self.ff_dim)))
         qs = S3(T * 3 * D, dh, 3 * D)
         os_ = S3(T * D, dh, D)
         scale = float(np.float32(1.0 / math.sqrt(dh)))
@@ -416,7 +442,7 @@ class DeviceDiT:
         sh_a, sc_a, g_a, sh_m, sc_m, g_m = (base + j * D * f4 for j in range(6))
         slot = 1 if r0 else 0
         plan = dict(st=st, plan_rows=2 * T)
-        np_, attp, ffp = self.np[slot].ptr, self.attp[slot].ptr, self.ffp[slot].ptr
+        np_, attp, ffp = (held[slot].ptr if held else None for held in (self.np, self.attp, self.ffp))
         # partial rotary on q and k, channels 0..dh-1 (dit.py:119-120), in the GEMM epilogue
         rope_epi = _lib.epilogue(rope=(self.cos.ptr, self.sin.ptr, T, D, dh, 2 * D))
         if self.qkv_frag:
@@ -508,6 +534,7 @@ class DeviceDiT:
         """Euler solve from x0 (1, 80, T) (already scaled by the temperature); returns the
         resident (80, T) result.  ``graph=True`` replays one captured HIP graph."""
         self.x.copy_from(np.asarray(x0, np.float32).reshape(self.mel, self._T))
+        self._row_planes()
         if not graph:
             self._enqueue_solve()
             return self.x
@@ -523,6 +550,7 @@ class DeviceDiT:
         """One estimator evaluation at the s-th Euler time on the CFG pair built from x0 (1, 80, T);
         returns the (2, 80, T) velocity, i.e. ``DiT.forward`` (dit.py:144-180) without the update."""
         self.x.copy_from(np.asarray(x0, np.float32).reshape(self.mel, self._T))
+        self._row_planes()
         self._time_and_mod()
         self._step(s, 0.0, update=False)
         return self.outT.numpy()

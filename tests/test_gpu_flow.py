@@ -131,3 +131,32 @@ def test_cfg_halves_on_two_streams_change_nothing(gpu, profile):
         np.testing.assert_array_equal(d.solve(x0, graph=True).numpy(), want)
     d.prepare(mu[:, :, :500], spks, cond[:, :, :500])
     assert not d.halves
+
+
+@pytest.mark.parametrize("profile,layouts", [("f32", "pppp"), ("balanced", "pppp"), ("per_channel", "rprr")])
+def test_linears_hold_the_layout_they_are_read_in(gpu, profile, layouts):
+    """Each block linear keeps its weight for activations in planes (p) or in float rows (r), the workspace the
+    activations that some launch writes, and a batch row's own planes come with ``halves``, below the threshold too."""
+    import cv3amd.dit as dit
+    _, dev = _stores(2, profile)
+    T = 70
+    mu, cond, spks, x0 = _inputs(T, seed=11)
+    d = dit.DeviceDiT(dev, steps=2)
+    d.prepare(mu, spks, cond)
+    for lins, layout in zip((d.qkv, d.out, d.ff1, d.ff2), layouts):
+        for lin in lins:
+            assert lin.takes_planes == (layout == "p") or not lin.q8
+            if lin.q8:
+                assert (lin.q is None) == (layout == "p") and (lin.codes16 is None) == (layout == "r")
+                bytes_a_code = 2 if layout == "p" else 1
+                assert bytes_a_code <= lin.nbytes / (lin.n * lin.k) < bytes_a_code + 0.1
+    planes = "r" not in layouts
+    assert (d.n is None, d.att is None, d.ffb is None) == (planes, layouts[1] == "p", planes)
+    want = d.solve(x0).numpy().copy()
+    assert max(map(len, (d.np, d.attp, d.ffp))) == 1
+    d.halves = True
+    np.testing.assert_array_equal(d.solve(x0).numpy(), want)
+    assert max(map(len, (d.np, d.attp, d.ffp))) == 2
+    if profile == "balanced":
+        with pytest.raises(ValueError, match="planes"):
+            d.qkv[0](0, 1, d.dim, 0, 3 * d.dim)
