@@ -678,7 +678,10 @@ __global__ __launch_bounds__(256) void k_scales_t(const void* scales, int sf16, 
 // (a: one workgroup's step, b: a step with every CU busy; us).  The constants are least-squares fits to
 // every variant timed at [40 .. 3000] rows x (N, K) = (3072, 1024), (2048, 1024), (1024, 1024),
 // (1024, 2048), weights from HBM, within 4-9 %; the pick is the fastest variant or on average 0.9 % behind
-// it.  E.g. float32, us: [40, 1024] x 1024: 10.3 (1 x 1) against 17.3 (2 x 2) and 31 (128 x 128);
+// it.  Weights of 32-code blocks fold twice as often and have no fit of their own: they take the 64-code row.  The
+// LM's shapes (K or N 896, 4864, 9728) were not in the fit either.  For both the pick is known to beat the float32
+// kernels it took the place of, at 5 .. 3000 rows (q4 by 1.15 to 6 times), not to be the best of the six.  E.g.
+// float32, us: [40, 1024] x 1024: 10.3 (1 x 1) against 17.3 (2 x 2) and 31 (128 x 128);
 // [1000, 3072] x 1024: 36.9 (128 x 96) against 43.5 (2 x 2) and 66.7 (1 x 1).
 struct Variant {
   int tm, tn;  // blocks of 32
@@ -695,7 +698,7 @@ constexpr Variant kVariants[3][V_COUNT] = {
     {{1, 1, 0, 2.79f, 1.07f, 0.008f, 0.037f}, {1, 2, 0, 1.45f, 2.63f, 0.050f, 0.051f},
      {2, 2, 0, 1.28f, 3.56f, 0.091f, 0.091f}, {2, 4, 2, 7.27f, 0.00f, 0.115f, 0.193f},
      {4, 4, 1, 3.16f, 7.28f, 0.206f, 0.338f}, {4, 3, 1, 1.56f, 5.84f, 0.212f, 0.247f}},
-    // q8 weights, one scale per 64 codes
+    // q8 weights, one scale per 64 codes (and per 32)
     {{1, 1, 0, 2.15f, 1.70f, 0.040f, 0.043f}, {1, 2, 0, 1.58f, 2.65f, 0.058f, 0.062f},
      {2, 2, 0, 1.89f, 2.63f, 0.103f, 0.135f}, {2, 4, 2, 10.54f, 0.00f, 0.216f, 0.241f},
      {4, 4, 1, 5.85f, 0.00f, 0.503f, 0.571f}, {4, 3, 1, 5.93f, 0.00f, 0.424f, 0.445f}},
@@ -1184,6 +1187,22 @@ __global__ __launch_bounds__(256) void k_mean_leaky(MeanInputs in, int count, fl
 }  // namespace
 
 extern "C" {
+
+int cv3_plane_linear_tile(int kind, int64_t block, int64_t rows, int64_t k, int64_t n, int* tile, int* count,
+                          int* row_blocks, int* col_blocks, int* ring) {
+  CV3_REQUIRE(tile && count && row_blocks && col_blocks && ring && rows > 0 && k > 0 && n > 0 && rows < (1ll << 30) &&
+                  k < (1ll << 30) && n < (1ll << 30) && block > 0,
+              CV3_EINVAL, "bad plane linear shape");
+  const int wk = kind == CV3_KIND_F32 ? W_F32 : block >= k ? W_ROW : block == 64 ? W_B64 : W_B32;
+  const int v = plane_variant(wk, (int)ceil_div(rows, 32), (int)ceil_div(n, 32), (int)(k / 16));
+  const Variant& t = kVariants[std::min(wk, (int)W_B64)][v];
+  *tile = v;
+  *count = V_COUNT;
+  *row_blocks = t.tm;
+  *col_blocks = t.tn;
+  *ring = t.occ > 0;
+  return CV3_OK;
+}
 
 int cv3_linear_x3_planes(const uint16_t* x, int64_t m, int64_t k, const uint16_t* frag, int64_t n, const float* bias,
                          float* y, int64_t ldy, uint16_t* y_planes, const cv3_epilogue* epi, int64_t plan_rows,

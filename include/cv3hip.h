@@ -198,6 +198,10 @@ int cv3_linear_q8_digits(const float* x, int64_t m, int64_t k, int64_t ldx, cons
  * neither (GELU not with 32-code blocks).  plan_rows (0: m): the rows that the tile, and with it the order of
  * the sums, is chosen for; parts of one batch launched side by side pass the batch's, fill the machine as its
  * tiles do and return its bits. */
+/* The tile that rule picks for (rows, K, n) and a weight kind (block as above; CV3_KIND_F32 ignores it): *tile is an
+ * index below *count, row_blocks x col_blocks its blocks of 32, ring whether it goes through LDS stages. */
+int cv3_plane_linear_tile(int kind, int64_t block, int64_t rows, int64_t k, int64_t n, int* tile, int* count,
+                          int* row_blocks, int* col_blocks, int* ring);
 int cv3_linear_x3_planes(const uint16_t* x, int64_t m, int64_t k, const uint16_t* frag, int64_t n, const float* bias,
                          float* y, int64_t ldy, uint16_t* y_planes, const cv3_epilogue* epi, int64_t plan_rows,
                          cv3_stream_t s);

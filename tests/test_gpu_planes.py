@@ -3,7 +3,8 @@
 The planes of a float32 value are the rounding chain test_gpu_x3.py pins bit for bit, and reproduce it to
 2^-24; so every result is compared with float64 (or the oracle) at the bar of the other float32 kernels,
 max |error| / max |reference| <= 1e-5.  Shapes sit at the edges of the 32-row fragments, of each kernel's
-tile (32 x 32 up to 128 x 128) and of its K ranges, and reach every variant the shape rule picks.
+tile (32 x 32 up to 128 x 128) and of its K ranges; that every tile of the shape rule runs for every kind of
+weight is asked of the rule itself (test_every_tile_of_the_rule, test_prompt_on_every_tile).
 """
 
 import ctypes
@@ -55,7 +56,7 @@ def ptr(d):
     return d.ptr if d is not None else None
 
 
-# (rows, K, N): one row, fragment and tile edges, few rows to many, every variant of the shape rule
+# (rows, K, N): one row, fragment and tile edges, few rows to many
 SHAPES = [(1, 128, 32), (31, 256, 68), (33, 1024, 96), (65, 320, 1024), (97, 1024, 3072), (302, 2048, 1024),
           (500, 1024, 1024), (700, 1024, 3072), (1001, 1024, 2048), (1500, 1024, 1028), (2100, 1024, 3072)]
 KINDS = ["f32", "q8_rows", "q8_block"]
@@ -102,6 +103,110 @@ def test_linear_from_planes(lib, m, k, n, kind):
     yp = empty((elems(lib, m, n),), np.uint16)
     run(bd.ptr, None, 0, yp.ptr, ctypes.byref(_lib.epilogue("gelu_tanh")), 0, None)
     assert rel_err(from_planes(yp, m, n), ref.gelu_tanh(want)) < TOL
+
+
+def tile_of(lib, kind, m, k, n):
+    """(tile, tiles, row blocks, column blocks, through LDS) of the shape rule."""
+    _lib = lib[0]
+    v = [ctypes.c_int() for _ in range(5)]
+    code = _lib.KIND_F32 if kind == "f32" else _lib.KIND_Q4 if kind == "q4" else _lib.KIND_Q8
+    block = {"f32": 1, "q8_rows": k, "q8_block": 64, "q4": 32}[kind]
+    _lib.call("plane_linear_tile", code, block, m, k, n, *(ctypes.addressof(a) for a in v))
+    return tuple(a.value for a in v)
+
+
+def shape_for(lib, kind, tile, k):
+    """The least work whose shape takes the tile, its last row and column blocks partial: rows 32 j + 1, columns
+    32 j + 16."""
+    found = [(m * n, m, n) for n in (1040, 1168, 2064, 3088, 9744) for m in range(33, 4000, 32)
+             if tile_of(lib, kind, m, k, n)[0] == tile]
+    return min(found)[1:] if found else None
+
+
+@pytest.mark.parametrize("tile", range(6))
+@pytest.mark.parametrize("kind", ["f32", "q8_rows", "q8_block", "q4"])
+def test_every_tile_of_the_rule(lib, kind, tile):
+    """Each tile with each kind of weight, at both tails of its K loops (K / 64 even and odd; thirds for the
+    float32 ring of three): float rows, a gated residual in place, GELU into planes."""
+    _lib, to_device, empty = lib
+    assert tile_of(lib, kind, 1, 1024, 1024)[1] == 6
+    ran = 0
+    for k in (896, 832, 960, 2048, 2112):
+        shape = shape_for(lib, kind, tile, k)
+        if shape is None:
+            continue
+        m, n = shape
+        ran += 1
+        rng = np.random.default_rng([m, k, n])
+        x, w = rng.normal(size=(m, k)).astype(np.float32), (0.02 * rng.normal(size=(n, k))).astype(np.float32)
+        b = rng.normal(size=n).astype(np.float32)
+        xp, bd = to_planes(lib, x), to_device(b)
+        if kind == "f32":
+            wd, w64 = to_planes(lib, w), w.astype(np.float64)
+            run = lambda *a: _lib.call("linear_x3_planes", xp.ptr, m, k, wd.ptr, n, *a)  # noqa: E731
+        else:
+            import cv3amd.quant as quant
+            block = {"q8_rows": k, "q8_block": 64, "q4": 32}[kind]
+            sdt = np.float32 if kind == "q8_rows" else np.float16
+            q, s, kp = quant.quantize_q4(w) if kind == "q4" else quant.quantize_q8(w, block, sdt)
+            name, code = ("q4", _lib.KIND_Q4) if kind == "q4" else ("q8", _lib.KIND_Q8)
+            w64 = quant.QTensor(name, q, s, (n, k), block).dequant().astype(np.float64)
+            qd, sd = to_device(np.ascontiguousarray(q)), to_device(np.ascontiguousarray(s))
+            nc, ns = ctypes.c_int64(), ctypes.c_int64()
+            _lib.call("code_planes_elems", n, k, block, ctypes.byref(nc), ctypes.byref(ns))
+            wd, st = empty((nc.value,), np.uint16), empty((ns.value,))
+            _lib.call("pack_code_planes", code, qd.ptr, n, k, sd.ptr, _lib.F32 if kind == "q8_rows" else _lib.F16, kp, block,
+                      0, 0, wd.ptr, st.ptr, None)
+            run = lambda *a: _lib.call("linear_code_planes", xp.ptr, m, k, wd.ptr, st.ptr, block, n, *a)  # noqa: E731
+        want = x.astype(np.float64) @ w64.T + b
+        print(f"[tile] {kind} {tile} m={m} k={k} n={n}", flush=True)
+        y = empty((m, n))
+        run(bd.ptr, y.ptr, n, None, None, 0, None)
+        assert rel_err(y.numpy(), want) < TOL
+        h, gate = rng.normal(size=(m, n)).astype(np.float32), rng.normal(size=n).astype(np.float32)
+        hd, gd = to_device(h), to_device(gate)
+        epi = _lib.epilogue(residual=hd.ptr, ld_res=n, gate=gd.ptr, gate_stride=0, rows_per_gate=1)
+        run(bd.ptr, hd.ptr, n, None, ctypes.byref(epi), 0, None)
+        assert rel_err(hd.numpy(), h + gate * want) < TOL
+        if kind != "q4":    # no GELU with 32-code blocks
+            yp = empty((elems(lib, m, n),), np.uint16)
+            run(bd.ptr, None, 0, yp.ptr, ctypes.byref(_lib.epilogue("gelu_tanh")), 0, None)
+            assert rel_err(from_planes(yp, m, n), ref.gelu_tanh(want)) < TOL
+    assert ran, "no shape takes this tile: delete it from the rule"
+
+
+@pytest.mark.parametrize("profile,kind", [("per_channel", "q8_rows"), ("balanced", "q8_block"), ("tiny", "q4")])
+def test_prompt_on_every_tile(lib, profile, kind):
+    """Prompt lengths at which the four projections together take every tile that any length up to 1000 takes, so
+    that the prompt's own epilogues (rotary into the cache, SwiGLU into planes) run on each, against the decode's
+    rows."""
+    import cv3amd.quant as quant
+    from cv3amd import synth
+    from cv3amd.qwen2 import DeviceQwen2
+    from cv3amd.weights import WeightStore
+    shapes = dict(qkv=(896, 1152), o=(896, 896), gate_up=(896, 9728), down=(4864, 896))
+
+    def tiles(t):
+        return {(p, tile_of(lib, kind, t, k, n)[0]) for p, (k, n) in shapes.items()}
+
+    reach = {t: tiles(t) for t in range(1, 1001, 16)}
+    left, lengths = set().union(*reach.values()), []
+    while left:
+        t = max(reach, key=lambda a: (len(reach[a] & left), -a))
+        lengths.append(t)
+        left -= reach[t]
+    print(f"[tile] prompt {profile}: lengths {lengths}", flush=True)
+    tensors = synth.quantize_store(synth.qwen2_tensors(layers=1), profile, quant.quantize_q8, quant.quantize_q4)
+    lms = [DeviceQwen2(WeightStore(dict(tensors), synth.qwen2_meta(layers=1), quant.QTensor), cap=1024, prompt_planes=on)
+           for on in (True, False)]
+    for t in lengths:
+        x = np.random.default_rng(t).normal(size=(t, 896)).astype(np.float32)
+        got = []
+        for lm in lms:
+            lm.prefill(x, 0)
+            got.append((lm.logits.numpy(), lm.k_cache.numpy()[:, :, :t], lm.v_cache.numpy()[:, :, :t]))
+        for a, b in zip(*got):
+            assert rel_err(a, b) < TOL
 
 
 @pytest.mark.parametrize("rows_per_batch,m", [(151, 302), (29, 58), (400, 400)])
