@@ -464,6 +464,17 @@ def bench_kernels(args):
     nbytes = sum(lm.bytes_per_token(PREFILL + 12).values())   # the timed tokens' midpoint (KV 524)
     log(f"kernels: one-launch decode step {us:.1f} us per token ({nbytes / (us * 1e-6) / 1e9:.0f} GB/s)")
     out["decode_step_us"] = round(us, 2)
+    # prompts on code planes, seven launches a layer
+    for t in (37, 500):
+        emb = to_device(rng.standard_normal((t, lm.hidden), dtype=np.float32))
+        lm.prefill(emb, 0)
+        synchronize()
+        tm.start()
+        for _ in range(4):
+            lm.prefill(emb, 0)
+        us = tm.stop() / 4 * 1e3
+        log(f"kernels: prompt of {t} tokens: {us:.0f} us")
+        out[f"prompt_{t}_us"] = round(us, 1)
     del lm, lm_t
     tensors, meta = synth.dit_tensors(depth=2), synth.dit_meta(depth=2)
     d = DeviceDiT(WeightStore(tensors, meta, quant.QTensor))
@@ -526,8 +537,9 @@ def bench_kernels(args):
         log(f"kernels: {name}: {us:.1f} us" + (f", {rate:.1f} TFLOP/s ({rate / (pk[0] / 1e12):.1%} of the "
                                                    f"{pk[1]} peak)" if rate else ""))
         out[name] = {"us": round(us, 2), "tflops": round(rate, 2) if rate else None}
-    # the 30 s solve's q8 GEMMs (the activation's bfloat16 planes times the codes, held in the matrix
-    # cores' fragment order as the solve holds them): per-output-channel f32 scales and block-64 / f16
+    # the 30 s solve's q8 linears, per-output-channel f32 scales and block-64 / f16: on activation planes
+    # (every block-64 linear of the solve, and the per-channel out), from float rows (per-channel ff2) and
+    # on the int8 digit planes (per-channel QKV and ff1)
     T3 = 1500
     BT3 = B * T3
     rng = np.random.default_rng(0)
@@ -552,6 +564,27 @@ def bench_kernels(args):
             us = tm.stop() / (5 * reps) * 1e3
             rate = 2.0 * BT3 * n * kk / (us * 1e-6) / 1e12
             name = f"q8 {label} GEMM [{BT3}, {kk}] x [{n}, {kk}]^T ({what})"
+            log(f"kernels: {name}: {us:.1f} us, {rate:.1f} TFLOP/s ({rate / (SPLIT_Q8_PEAK / 1e12):.1%} of the "
+                f"split q8 peak)")
+            out[name] = {"us": round(us, 2), "tflops": round(rate, 2)}
+            nc, ns = ctypes.c_int64(), ctypes.c_int64()
+            _lib.call("code_planes_elems", n, kk, block, ctypes.byref(nc), ctypes.byref(ns))
+            cf, st = DeviceArray((nc.value,), np.uint16), DeviceArray((ns.value,))
+            _lib.call("pack_code_planes", _lib.KIND_Q8, qd.ptr, n, kk, sd.ptr, sdt_c, kp, block, 0, 0, cf.ptr, st.ptr, None)
+            _lib.call("x3_frag_elems", BT3, kk, ctypes.byref(nc))
+            ap = DeviceArray((nc.value,), np.uint16)
+            _lib.call("split_x3_frag", a_d.ptr, BT3, kk, F, ap.ptr, None)
+            fn = lambda: _lib.call("linear_code_planes", ap.ptr, BT3, kk, cf.ptr, st.ptr, block, n, None, y.ptr, n, None,
+                                   None, 0, None)
+            run = replayer(args.graph, lambda: [fn() for _ in range(reps)])
+            run()
+            synchronize()
+            tm.start()
+            for _ in range(5):
+                run()
+            us = tm.stop() / (5 * reps) * 1e3
+            rate = 2.0 * BT3 * n * kk / (us * 1e-6) / 1e12
+            name = f"q8 {label} linear [{BT3}, {kk}] x [{n}, {kk}]^T on planes ({what})"
             log(f"kernels: {name}: {us:.1f} us, {rate:.1f} TFLOP/s ({rate / (SPLIT_Q8_PEAK / 1e12):.1%} of the "
                 f"split q8 peak)")
             out[name] = {"us": round(us, 2), "tflops": round(rate, 2)}

@@ -277,40 +277,29 @@ __global__ __launch_bounds__(256 * NKG) void k_flash64(AttnParams p, int nq) {
     for (int i = 0; i < 4; ++i) orow[db * 16 + 4 * g + i] = oacc[db][i] / l_tot;
 }
 
-__device__ __forceinline__ float wave_total(float v) { return wave_sum(v); }
-__device__ __forceinline__ double wave_total(double v) { return wave_sum_d(v); }
-__device__ __forceinline__ float wave_most(float v) { return wave_max(v); }
-__device__ __forceinline__ double wave_most(double v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, kWave));
-  return v;
-}
-
-// One query of any head dim <= 256 by one wave, 64 keys per step; qs: the scaled query in LDS; T: the sums' type.
-// EVERY: values before the first key it sees count too, with probability zero (an infinity or NaN among them makes
-// the output NaN).
-template <bool EVERY, typename T>
+// One query of any head dim <= 256 by one wave, 64 keys per step; qs: the scaled query in LDS.
 __device__ __forceinline__ void attend_row(const AttnParams& p, int b, int hq, int hkv, int64_t qi, int lane, const float* qs) {
   const float* kbase = p.k + b * p.k_sb + hkv * p.k_sh;
   const float* vbase = p.v + b * p.v_sb + hkv * p.v_sh;
-  T acc[4] = {0, 0, 0, 0};
-  T m_run = -INFINITY, l_run = 0;
+  float acc[4] = {0.f, 0.f, 0.f, 0.f};
+  float m_run = -INFINITY, l_run = 0.f;
   int64_t klo, khi;
   visible_keys(p, qi, klo, khi);
   for (int64_t c0 = 0; c0 < p.m; c0 += 64) {
     const int64_t kj = c0 + lane;
-    T s = -INFINITY;
+    float s = -INFINITY;
     if (kj >= klo && kj < khi) {
       const float* kr = kbase + kj * p.k_sm;
-      s = 0;
-      for (int d = 0; d < p.d; ++d) s = fma((T)qs[d], (T)kr[d], s);
+      float t = 0.f;
+      for (int d = 0; d < p.d; ++d) t = fmaf(qs[d], kr[d], t);
+      s = t;
     }
-    const T m_new = max(m_run, wave_most(s));
-    const bool none = m_new == -INFINITY;
-    if (!EVERY && none) continue;
-    const float alpha = none ? 1.f : expf((float)(m_run - m_new));
-    const float pj = none ? 0.f : expf((float)(s - m_new));
-    l_run = l_run * alpha + wave_total((T)pj);
+    const float mx = wave_max(s);
+    const float m_new = fmaxf(m_run, mx);
+    if (m_new == -INFINITY) continue;
+    const float alpha = expf(m_run - m_new);
+    const float pj = expf(s - m_new);
+    l_run = l_run * alpha + wave_sum(pj);
 #pragma unroll
     for (int r = 0; r < 4; ++r) acc[r] *= alpha;
     const int64_t cnt = p.m - c0 < 64 ? p.m - c0 : 64;
@@ -320,7 +309,7 @@ __device__ __forceinline__ void attend_row(const AttnParams& p, int b, int hq, i
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int d = lane + 64 * r;
-        if (d < p.d) acc[r] = fma((T)pb, (T)vr[d], acc[r]);
+        if (d < p.d) acc[r] = fmaf(pb, vr[d], acc[r]);
       }
     }
     m_run = m_new;
@@ -329,8 +318,70 @@ __device__ __forceinline__ void attend_row(const AttnParams& p, int b, int hq, i
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const int d = lane + 64 * r;
-    if (d < p.d) orow[d] = (float)(acc[r] / l_run);
+    if (d < p.d) orow[d] = acc[r] / l_run;
   }
+}
+
+// k_flash64x's second pass: one query from the floats, 64 dims in 16-byte aligned rows, by one wave, with sums in
+// 64 bits (a lone wave's serial sums in 32 were off by 1.4e-6, the tiles' are by 4e-7).  qs: the scaled query in
+// LDS.  Every value counts, those of masked keys with probability zero.  Scores: a lane per key; values: 16 lanes
+// across a row, four keys at a time.  16 heads, 1500 rows, every query: 14.2 ms a key at a time, 2.4 so.
+__device__ __forceinline__ double wave_max_d(double v) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, kWave));
+  return v;
+}
+
+__device__ __forceinline__ void attend_again(const AttnParams& p, int b, int hq, int hkv, int64_t qi, int lane,
+                                             const float4* qs) {
+  const float* kbase = p.k + b * p.k_sb + hkv * p.k_sh;
+  const float* vbase = p.v + b * p.v_sb + hkv * p.v_sh;
+  const int dq = lane & 15, sub = lane >> 4;
+  double acc[4] = {0., 0., 0., 0.}, m_run = -INFINITY, l_run = 0.;
+  int64_t klo, khi;
+  visible_keys(p, qi, klo, khi);
+  for (int64_t c0 = 0; c0 < p.m; c0 += 64) {
+    const int64_t kj = c0 + lane;
+    double s = -INFINITY;
+    if (kj >= klo && kj < khi) {
+      const float4* kr = reinterpret_cast<const float4*>(kbase + kj * p.k_sm);
+      s = 0.;
+#pragma unroll 4
+      for (int d = 0; d < 16; ++d) {
+        const float4 k4 = kr[d], q4 = qs[d];
+        s = fma((double)q4.x, (double)k4.x, s);
+        s = fma((double)q4.y, (double)k4.y, s);
+        s = fma((double)q4.z, (double)k4.z, s);
+        s = fma((double)q4.w, (double)k4.w, s);
+      }
+    }
+    const double m_new = fmax(m_run, wave_max_d(s));
+    const bool none = m_new == -INFINITY;
+    const float alpha = none ? 1.f : expf((float)(m_run - m_new));
+    const float pj = none ? 0.f : expf((float)(s - m_new));
+    l_run = l_run * alpha + wave_sum_d((double)pj);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc[e] *= alpha;
+#pragma unroll 8
+    for (int j = 0; j < 16; ++j) {
+      const int key = 4 * j + sub;
+      const float pb = __shfl(pj, key, kWave);
+      float4 v = *reinterpret_cast<const float4*>(vbase + min(c0 + key, p.m - 1) * p.v_sm + 4 * dq);
+      if (c0 + key >= p.m) v = make_float4(0.f, 0.f, 0.f, 0.f);
+      acc[0] = fma((double)pb, (double)v.x, acc[0]);
+      acc[1] = fma((double)pb, (double)v.y, acc[1]);
+      acc[2] = fma((double)pb, (double)v.z, acc[2]);
+      acc[3] = fma((double)pb, (double)v.w, acc[3]);
+    }
+    m_run = m_new;
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    acc[e] += __shfl_xor(acc[e], 16, kWave);
+    acc[e] += __shfl_xor(acc[e], 32, kWave);
+  }
+  const double own = sub == 0 ? acc[0] : sub == 1 ? acc[1] : sub == 2 ? acc[2] : acc[3];
+  p.o[b * p.o_sb + hq * p.o_sh + qi * p.o_sn + 4 * dq + sub] = (float)(own / l_run);
 }
 
 // The same flash attention on the bfloat16 matrix cores (v_mfma_f32_16x16x32_bf16): q, k, v
@@ -376,7 +427,7 @@ __device__ __forceinline__ void mfma6(const bf16x8_t& ah, const bf16x8_t& am, co
 // A stage that no query of the workgroup sees is skipped, but for its values' exponents: a masked key counts with
 // probability zero, and zero times an infinity or NaN is NaN in that dim of every output, whichever tile it is in.
 // AGAIN: outputs that come out not finite, or smaller than planes of the values hold in full, are formed again from
-// the floats, with sums in 64 bits (a lone wave's serial sums in 32 were off by 1.4e-6, the tiles' are by 4e-7).
+// the floats (attend_again).
 template <int QWN, bool AGAIN>
 __global__ __launch_bounds__(512) void k_flash64x(AttnParams p, int nq) {
   constexpr int NKG = 8 / QWN, NS = QWN, WKT = 16 * NS;  // key groups; a group's sub-tiles and keys
@@ -647,7 +698,7 @@ __global__ __launch_bounds__(512) void k_flash64x(AttnParams p, int nq) {
     }
   }
   if (p.op) return;
-  [[maybe_unused]] bool bad = false;
+  [[maybe_unused]] uint32_t bad = 0;   // bit 4 db + i
   if (qvalid) {
     float* orow = p.o + b * p.o_sb + hq * p.o_sh + qi * p.o_sn;
 #pragma unroll
@@ -656,21 +707,36 @@ __global__ __launch_bounds__(512) void k_flash64x(AttnParams p, int nq) {
       for (int i = 0; i < 4; ++i) {
         const float y = value(db, i);
         orow[db * 16 + 4 * g + i] = y;
-        bad |= !in_range(magnitude(y));
+        bad |= (uint32_t)!in_range(magnitude(y)) << (4 * db + i);
       }
   }
   if constexpr (AGAIN) {
     // infinities and the largest floats have no planes here (inf - inf), values below 2^-110 not all their bits: the
-    // whole wave does those queries again
-    uint64_t todo = __ballot(bad);
+    // whole wave does those queries again, but for dims with a NaN among the values and queries with one, which are
+    // NaN as they stand
+    if (__any(bad)) {
+      const int sub = lane >> 4;
+      uint32_t nan = 0;
+      for (int r = sub; r < (int)p.m; r += 4) {
+        const float4 v = *reinterpret_cast<const float4*>(vbase + (int64_t)r * p.v_sm + 4 * c16);
+        nan |= (v.x != v.x) | (v.y != v.y) << 1 | (v.z != v.z) << 2 | (v.w != v.w) << 3;
+      }
+      nan |= __shfl_xor(nan, 16, 64);
+      nan |= __shfl_xor(nan, 32, 64);
+#pragma unroll
+      for (int db = 0; db < 4; ++db) bad &= ~(__shfl(nan, 4 * db + g, 64) << (4 * db));
+    }
+    uint64_t todo = __ballot(bad != 0);
     todo = (todo | todo >> 16 | todo >> 32 | todo >> 48) & 0xffff;
     float* qs = reinterpret_cast<float*>(&Vs[0][0][0]) + 64 * qw;
     while (todo) {
       const int64_t row = q0 + __builtin_ctzll(todo);
       todo &= todo - 1;
-      qs[lane] = p.q[b * p.q_sb + hq * p.q_sh + row * p.q_sn + lane] * p.scale;
+      const float x = p.q[b * p.q_sb + hq * p.q_sh + row * p.q_sn + lane] * p.scale;
+      if (__any(x != x)) continue;
+      qs[lane] = x;
       __builtin_amdgcn_wave_barrier();
-      attend_row<true, double>(p, b, hq, hkv, row, lane, qs);
+      attend_again(p, b, hq, hkv, row, lane, reinterpret_cast<const float4*>(qs));
       __builtin_amdgcn_wave_barrier();
     }
   }
@@ -689,7 +755,7 @@ __global__ __launch_bounds__(256) void k_attn_generic(AttnParams p) {
   for (int d = lane; d < p.d; d += 64) qs[d] = qvalid ? qrow[d] * p.scale : 0.f;
   __syncthreads();
   if (!qvalid) return;
-  attend_row<false, float>(p, b, hq, hkv, qi, lane, qs);
+  attend_row(p, b, hq, hkv, qi, lane, qs);
 }
 
 }  // namespace

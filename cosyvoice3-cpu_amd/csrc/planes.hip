@@ -58,7 +58,7 @@ struct PlaneParams {
   float *kc, *vc;
   int heads, kv_heads, cap, pos0;
   const float *cos, *sin;  // [cap][64]
-  // the float32 rows x was split from, or null.  Outputs that come out not finite are formed again from these:
+  // the float32 rows x was split from, or null (AGAIN kernels read them).  Outputs that come out not finite are formed again from these:
   // an infinity times a plane of zero is NaN, and code products may pass the range before their scale.  So are
   // those below 2^-90: rows below 2^-110 have fewer than 24 bits in their planes, which shows (2^-134 an element)
   // only in outputs this small, unless an output's weights sum to more than 2^20.
@@ -154,9 +154,10 @@ __device__ __forceinline__ float act_of(float v) {
 // Epilogue of G groups of four neighbouring outputs: group q of this lane is v[q], outputs
 // n[q] .. n[q] + 3 of row m[q].  Every operand is loaded before the first store (C may be the
 // residual itself), in k_pg_reg before the waves meet.  Order of operations as store_tile's
-// (gemm.hip): bias, rotary, activation, gate, residual.  GATED kernels take a gate and a residual;
-// the others spend no registers on them (which leaves the q8 64 x 128 tiles two workgroups per CU).
-template <int ACT, int KIND, bool GATED, int G>
+// (gemm.hip): bias, rotary, activation, gate, residual.  GATED kernels take a gate and a residual,
+// AGAIN kernels the float rows of fx; the others spend no registers on them (which leaves the q8
+// 64 x 128 tiles two workgroups per CU).
+template <int ACT, int KIND, bool GATED, bool AGAIN, int G>
 struct PlaneEpilogue {
   int m[G], n[G];
   float4 scale[G], bias[G], gate[G], res[G];
@@ -208,27 +209,90 @@ struct PlaneEpilogue {
     }
   }
 
-  // row m of fx times the weight's outputs n .. n + 3, in float32 (rarely run)
+  // Row mm of fx times the weight's outputs nn .. nn + 3 in float32, by the whole wave: a lane takes every 64th run
+  // of eight k, which is its 16 bytes of each plane.
   __device__ __forceinline__ float4 again(const PlaneParams& p, int mm, int nn, float4 row) const {
     constexpr int NPW = planes_of(KIND), FOLD = fold_steps(KIND);
-    const uint16_t* w = reinterpret_cast<const uint16_t*>(p.w);
+    const int lane = threadIdx.x & 63;
+    const float rs[4] = {row.x, row.y, row.z, row.w};
     float a[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 1
-    for (int k = 0; k < p.S * 16; ++k) {
-      const float x = p.fx[(int64_t)mm * p.ldfx + k];
+    for (int c = lane; c < p.S * 2; c += 64) {
+      const float4 x0 = *reinterpret_cast<const float4*>(p.fx + (int64_t)mm * p.ldfx + 8 * c);
+      const float4 x1 = *reinterpret_cast<const float4*>(p.fx + (int64_t)mm * p.ldfx + 8 * c + 4);
+      const float x[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
+        __builtin_amdgcn_sched_barrier(0);   // one output's weights at a time: the tile's registers are few
         const int r = nn + e;
-        const int64_t at = (((int64_t)(r >> 5) * p.S + (k >> 4)) * 64 + (r & 31) + 32 * ((k >> 3) & 1)) * 8 + (k & 7);
-        float v = 0.f;   // lo + mid + hi: exact in this order
+        const int64_t at = ((int64_t)(r >> 5) * p.S + (c >> 1)) * 64 + (r & 31) + 32 * (c & 1);
+        uint4 f[NPW];
 #pragma unroll
-        for (int pl = NPW - 1; pl >= 0; --pl) v += __uint_as_float((uint32_t)w[at + pl * p.wpl * 8] << 16);
-        if constexpr (KIND == W_ROW) v *= e == 0 ? row.x : e == 1 ? row.y : e == 2 ? row.z : row.w;
-        if constexpr (FOLD > 0) v *= p.scales[(int64_t)(k / (16 * FOLD)) * p.nbw * 32 + r];
-        a[e] = fmaf(x, v, a[e]);
+        for (int pl = 0; pl < NPW; ++pl) f[pl] = p.w[at + pl * p.wpl];
+        float scale = 1.f;
+        if constexpr (KIND == W_ROW) scale = rs[e];
+        if constexpr (FOLD > 0) scale = p.scales[(int64_t)((c >> 1) / FOLD) * p.nbw * 32 + r];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          float w = 0.f;   // lo + mid + hi: exact in this order
+#pragma unroll
+          for (int pl = NPW - 1; pl >= 0; --pl) {
+            const uint32_t two = j < 2 ? f[pl].x : j < 4 ? f[pl].y : j < 6 ? f[pl].z : f[pl].w;
+            w += __uint_as_float(j & 1 ? two & 0xffff0000u : two << 16);
+          }
+          if constexpr (KIND != W_F32) w *= scale;
+          a[e] = fmaf(x[j], w, a[e]);
+        }
       }
     }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) a[e] = wave_sum(a[e]);
     return make_float4(a[0], a[1], a[2], a[3]);
+  }
+
+  // Whether row mm of fx holds a NaN (by the whole wave): its outputs are NaN as they stand.
+  __device__ __forceinline__ bool row_is_nan(const PlaneParams& p, int mm) const {
+    bool nan = false;
+#pragma unroll 1
+    for (int k = 4 * (threadIdx.x & 63); k < p.S * 16; k += 256) {
+      const float4 x = *reinterpret_cast<const float4*>(p.fx + (int64_t)mm * p.ldfx + k);
+      nan |= x.x != x.x || x.y != x.y || x.z != x.z || x.w != x.w;
+    }
+    return __any(nan);
+  }
+
+  // Forms the groups that are out of the planes' range again.  Float32 [3000, 1024] x 3072, 0.12 ms: with one NaN
+  // row as long, nothing but such rows 0.22 ms, nothing but rows of 1e-30 8.8 ms (each lane alone: 3.0, 8.2, 8.2).
+  __device__ __forceinline__ void mend(const PlaneParams& p, float4 (&v)[G]) const {
+    const int lane = threadIdx.x & 63;
+    enum { UNREAD, NUMBERS, LOST };
+    int mine = UNREAD;   // what the lane's row is
+#pragma unroll
+    for (int q = 0; q < G; ++q) {
+      const bool bad = !in_range(v[q]) && m[q] < p.m && n[q] < p.n;
+      if (q == 0 || __builtin_amdgcn_readfirstlane(m[q]) != __builtin_amdgcn_readfirstlane(m[q - (q > 0)])) mine = UNREAD;
+      uint64_t todo = __ballot(bad && mine != LOST);
+      while (todo) {
+        const int src = __builtin_ctzll(todo);
+        const int mm = __builtin_amdgcn_readlane(m[q], src), nn = __builtin_amdgcn_readlane(n[q], src);
+        if (__builtin_amdgcn_readlane(mine, src) == UNREAD) {
+          const bool nan = row_is_nan(p, mm);
+          if (m[q] == mm) mine = nan ? LOST : NUMBERS;
+          if (nan) {
+            todo &= ~__ballot(m[q] == mm);
+            continue;
+          }
+        }
+        todo &= todo - 1;
+        float4 row = make_float4(1.f, 1.f, 1.f, 1.f);
+        if constexpr (KIND == W_ROW) {
+          auto at = [&](float f) { return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(f), src)); };
+          row = make_float4(at(scale[q].x), at(scale[q].y), at(scale[q].z), at(scale[q].w));
+        }
+        const float4 again4 = again(p, mm, nn, row);
+        if (lane == src) v[q] = again4;
+      }
+    }
   }
 
   __device__ __forceinline__ void store_swiglu(const PlaneParams& p, const float4 (&v)[G]) const {
@@ -278,15 +342,11 @@ struct PlaneEpilogue {
       if constexpr (KIND == W_ROW)
         v[q] = make_float4(v[q].x * scale[q].x, v[q].y * scale[q].y, v[q].z * scale[q].z, v[q].w * scale[q].w);
     }
-    if (p.fx) {  // a row's four outputs are small together: its rows' fault (a weight's such rows have no planes)
+    if constexpr (AGAIN) {  // a row's four outputs are small together: its rows' fault (a weight's such rows have no planes)
       bool fine = true;
 #pragma unroll
       for (int q = 0; q < G; ++q) fine &= in_range(v[q]);
-      if (!fine) {
-#pragma unroll
-        for (int q = 0; q < G; ++q)
-          if (!in_range(v[q]) && m[q] < p.m && n[q] < p.n) v[q] = again(p, m[q], n[q], scale[q]);
-      }
+      if (__any(!fine)) mend(p, v);
     }
 #pragma unroll
     for (int q = 0; q < G; ++q) {
@@ -336,7 +396,7 @@ struct PlaneEpilogue {
 
 // ---- fragments straight into registers, K split over the workgroup's waves ----
 // PF register stages (PF - 1 steps in flight); a block-scaled weight's ranges are whole 64-k blocks.
-template <int KIND, int ACT, bool GATED, int RM, int RN, int WK, int PF>
+template <int KIND, int ACT, bool GATED, bool AGAIN, int RM, int RN, int WK, int PF>
 __global__ __launch_bounds__(64 * WK) void k_pg_reg(PlaneParams p) {
   constexpr int NPW = planes_of(KIND), FOLD = fold_steps(KIND), UNIT = FOLD ? FOLD : 1, LOADS = RM * 3 + RN * NPW;
   static_assert(UNIT == 1 || PF % 4 == 0, "a turn of the register ring is whole blocks");
@@ -418,7 +478,7 @@ __global__ __launch_bounds__(64 * WK) void k_pg_reg(PlaneParams p) {
 #undef CV3_STEP
   // the waves' partial sums meet in LDS, in wave order; each wave finishes its share of the groups
   constexpr int GROUPS = RM * RN * 4, G = GROUPS > WK ? GROUPS / WK : 1;
-  PlaneEpilogue<ACT, KIND, GATED, G> ep;
+  PlaneEpilogue<ACT, KIND, GATED, AGAIN, G> ep;
 #pragma unroll
   for (int q = 0; q < G; ++q) {
     const int id = min(wave * G + q, GROUPS - 1), blk = id >> 2, g = id & 3;
@@ -456,7 +516,7 @@ __global__ __launch_bounds__(64 * WK) void k_pg_reg(PlaneParams p) {
 //   landed and every wave has read this one (vmcnt counts this wave's DMAs, which land in order);
 //   refill this slot NST stages ahead and read the next stage's first fragments under the second
 //   step's MFMAs.
-template <int KIND, int ACT, bool GATED, int WM, int WN, int RM, int RN, int NST>
+template <int KIND, int ACT, bool GATED, bool AGAIN, int WM, int WN, int RM, int RN, int NST>
 __global__ __launch_bounds__(64 * WM * WN) void k_pg_lds(PlaneParams p) {
   constexpr int NPW = planes_of(KIND), NW = WM * WN, TM = WM * RM, TN = WN * RN;
   constexpr int F = (TM * 3 + TN * NPW) * 2, FP = (F + NW - 1) / NW;  // fragments per stage, per wave
@@ -598,7 +658,7 @@ __global__ __launch_bounds__(64 * WM * WN) void k_pg_lds(PlaneParams p) {
 #undef CV3_STAGE
   __builtin_amdgcn_s_waitcnt(CV3_VM(0));  // no DMA outlives the workgroup's LDS
   constexpr int G = RM * RN * 4;
-  PlaneEpilogue<ACT, KIND, GATED, G> ep;
+  PlaneEpilogue<ACT, KIND, GATED, AGAIN, G> ep;
   float4 v[G];
 #pragma unroll
   for (int i = 0; i < RM; ++i)
@@ -723,7 +783,7 @@ int plane_variant(int kind, int nbm, int nbn, int S) {
   return best;
 }
 
-template <int KIND, int ACT, bool GATED>
+template <int KIND, int ACT, bool GATED, bool AGAIN = false>
 void launch(int variant, const PlaneParams& p, hipStream_t st) {
   const dim3 grid((unsigned)(p.tiles_m * p.tiles_n));
   // the waves a tile's K is split over and the register ring, as measured per weight kind: float32
@@ -731,9 +791,9 @@ void launch(int variant, const PlaneParams& p, hipStream_t st) {
   constexpr bool F = KIND == W_F32, B = fold_steps(KIND) > 0;
   constexpr int NST = F ? 3 : 4;
 #define CV3_REG(RM, RN, WK, PF) \
-  hipLaunchKernelGGL((k_pg_reg<KIND, ACT, GATED, RM, RN, WK, PF>), grid, dim3(64 * (WK)), 0, st, p)
+  hipLaunchKernelGGL((k_pg_reg<KIND, ACT, GATED, AGAIN, RM, RN, WK, PF>), grid, dim3(64 * (WK)), 0, st, p)
 #define CV3_LDS(WM, WN, RM, RN) \
-  hipLaunchKernelGGL((k_pg_lds<KIND, ACT, GATED, WM, WN, RM, RN, NST>), grid, dim3(64 * (WM) * (WN)), 0, st, p)
+  hipLaunchKernelGGL((k_pg_lds<KIND, ACT, GATED, AGAIN, WM, WN, RM, RN, NST>), grid, dim3(64 * (WM) * (WN)), 0, st, p)
   switch (variant) {
     case V_R11: CV3_REG(1, 1, (F ? 4 : 8), 4); break;
     case V_R12: CV3_REG(1, 2, (F ? 4 : 8), (F ? 3 : 4)); break;
@@ -751,16 +811,24 @@ int launch_act(int act, int variant, const PlaneParams& p, hipStream_t st) {
   const bool gated = p.epi.gate || p.epi.residual;
   CV3_REQUIRE(!gated || act == CV3_ACT_NONE, CV3_EUNSUPPORTED,
               "plane linear: a gate or residual comes without an activation here");
+  const bool again = p.fx != nullptr;
   if (act == CV3_ACT_NONE) {
-    if (gated)
+    if (gated && again)
+      launch<KIND, CV3_ACT_NONE, true, true>(variant, p, st);
+    else if (gated)
       launch<KIND, CV3_ACT_NONE, true>(variant, p, st);
+    else if (again)
+      launch<KIND, CV3_ACT_NONE, false, true>(variant, p, st);
     else
       launch<KIND, CV3_ACT_NONE, false>(variant, p, st);
     return CV3_OK;
   }
   if constexpr (KIND != W_B32) {
     if (act == CV3_ACT_GELU_TANH) {
-      launch<KIND, CV3_ACT_GELU_TANH, false>(variant, p, st);
+      if (again)
+        launch<KIND, CV3_ACT_GELU_TANH, false, true>(variant, p, st);
+      else
+        launch<KIND, CV3_ACT_GELU_TANH, false>(variant, p, st);
       return CV3_OK;
     }
   }
