@@ -625,7 +625,7 @@ __global__ __launch_bounds__(512) void k_flash64x(AttnParams p, int nq) {
   for (int db = 0; db < 4; ++db) oacc[db] = ob[db] + os[db];
   // merge the key groups through LDS, as k_flash64
   __syncthreads();
-  {
+  if (p.mask_kind != 0) {
     // thread -> dims 4 dq .. + 3 of every 32nd row; rows past the end clamp to the last one
     const int rows0 = (int)(st0 * STAGE), at1 = (int)(nstages * STAGE), rows1 = max((int)p.m - at1, 0);
     float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -675,11 +675,13 @@ __global__ __launch_bounds__(512) void k_flash64x(AttnParams p, int nq) {
   }
   float l_tot = l_run + __shfl_xor(l_run, 16, 64);
   l_tot += __shfl_xor(l_tot, 32, 64);
-  const uint32_t lost[2] = {skipped[0], skipped[1]};
-  auto value = [&](int db, int i) {
-    const bool nan = lost[db >> 1] >> (16 * (db & 1) + 4 * g + i) & 1;
-    return nan ? __builtin_nanf("") : oacc[db][i] / l_tot;
-  };
+  if (p.mask_kind != 0 && (skipped[0] | skipped[1])) {
+#pragma unroll
+    for (int db = 0; db < 4; ++db)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (skipped[db >> 1] >> (16 * (db & 1) + 4 * g + i) & 1) oacc[db][i] = __builtin_nanf("");
+  }
   if (p.op && qvalid) {
     // row b n + qi of [batch n, 64 h] rows as the fragments a plane linear reads: four neighbouring
     // columns are half of a lane's 16 bytes
@@ -690,31 +692,38 @@ __global__ __launch_bounds__(512) void k_flash64x(AttnParams p, int nq) {
       const int64_t at = (((row >> 5) * (4 * p.h) + (col >> 4)) * 64 + (row & 31) + 32 * ((col >> 3) & 1)) * 2 +
                          ((col >> 2) & 1);
       uint2 hi, mid, lo;
-      split_x3(value(db, 0), value(db, 1), hi.x, mid.x, lo.x);
-      split_x3(value(db, 2), value(db, 3), hi.y, mid.y, lo.y);
+      split_x3(oacc[db][0] / l_tot, oacc[db][1] / l_tot, hi.x, mid.x, lo.x);
+      split_x3(oacc[db][2] / l_tot, oacc[db][3] / l_tot, hi.y, mid.y, lo.y);
       p.op[at] = hi;
       p.op[at + p.opl] = mid;
       p.op[at + 2 * p.opl] = lo;
     }
   }
   if (p.op) return;
-  [[maybe_unused]] uint32_t bad = 0;   // bit 4 db + i
+  [[maybe_unused]] float y[4][4];
+  [[maybe_unused]] uint32_t most = 0, least = 0xffffffffu;   // least: of the magnitudes but zero, less one
   if (qvalid) {
     float* orow = p.o + b * p.o_sb + hq * p.o_sh + qi * p.o_sn;
 #pragma unroll
     for (int db = 0; db < 4; ++db)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const float y = value(db, i);
-        orow[db * 16 + 4 * g + i] = y;
-        bad |= (uint32_t)!in_range(magnitude(y)) << (4 * db + i);
+        y[db][i] = oacc[db][i] / l_tot;
+        orow[db * 16 + 4 * g + i] = y[db][i];
+        most = max(most, magnitude(y[db][i]));
+        least = min(least, magnitude(y[db][i]) - 1u);
       }
   }
   if constexpr (AGAIN) {
     // infinities and the largest floats have no planes here (inf - inf), values below 2^-110 not all their bits: the
     // whole wave does those queries again, but for dims with a NaN among the values and queries with one, which are
     // NaN as they stand
-    if (__any(bad)) {
+    uint32_t bad = 0;   // bit 4 db + i
+    if (__any(!in_range(most) || !in_range(least + 1u))) {
+#pragma unroll
+      for (int db = 0; db < 4; ++db)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) bad |= (uint32_t)(qvalid && !in_range(magnitude(y[db][i]))) << (4 * db + i);
       const int sub = lane >> 4;
       uint32_t nan = 0;
       for (int r = sub; r < (int)p.m; r += 4) {

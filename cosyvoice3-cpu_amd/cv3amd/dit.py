@@ -392,13 +392,20 @@ class DeviceDiT:
         self.mods = DeviceArray((S, self.ld_mod))
         self._graph = None
 
-    def _row_planes(self):
-        """Planes for a batch row of its own, while the two rows run apart (fragments hold 32 rows, so the second
-        cannot start inside one)."""
+    def _row_buffers(self):
+        """Where a launch over both batch rows, and one over the second alone, finds its rows: (h, n, attention,
+        qkv, feed-forward) floats and (norm, attention, feed-forward) planes.  The second row has planes of its own
+        while the two run apart (fragments hold 32 rows, so it cannot start inside one)."""
+        planes = ((self.np, self.dim), (self.attp, self.dim), (self.ffp, self.ff_dim))
         if self.halves:
-            for held, k in ((self.np, self.dim), (self.attp, self.dim), (self.ffp, self.ff_dim)):
+            for held, k in planes:
                 if len(held) == 1:
                     held.append(self._planes(self._T, k))
+        D, floats = self.dim, (self.h, self.n, self.att, self.qkvb, self.ffb)
+        self._at = [[a.ptr + 4 * r0 * w if a is not None else None
+                     for a, w in zip(floats, (D, D, D, 3 * D, self.ff_dim))] +
+                    [held[i].ptr if len(held) > i else None for held, _ in planes]
+                    for i, r0 in enumerate((0, self._T))]
 
     @staticmethod
     def _planes(rows: int, k: int) -> DeviceArray:
@@ -432,17 +439,13 @@ class DeviceDiT:
         T, D, H, dh, f4 = self._T, self.dim, self.heads, self.dim_head, 4
         S3 = ctypes.c_int64 * 3
         rows = nb * T
-        h, n, att, qkvb, ffb = (a.ptr + f4 * r0 * w if a is not None else None
-                                for a, w in ((self.h, D), (self.n, D), (self.att, D), (self.qkvb, 3 * D),
-                                             (self.ffb, self.ff_dim)))
+        h, n, att, qkvb, ffb, np_, attp, ffp = self._at[1 if r0 else 0]
         qs = S3(T * 3 * D, dh, 3 * D)
         os_ = S3(T * D, dh, D)
         scale = float(np.float32(1.0 / math.sqrt(dh)))
         base = mrow + i * 6 * D * f4
         sh_a, sc_a, g_a, sh_m, sc_m, g_m = (base + j * D * f4 for j in range(6))
-        slot = 1 if r0 else 0
         plan = dict(st=st, plan_rows=2 * T)
-        np_, attp, ffp = (held[slot].ptr if held else None for held in (self.np, self.attp, self.ffp))
         # partial rotary on q and k, channels 0..dh-1 (dit.py:119-120), in the GEMM epilogue
         rope_epi = _lib.epilogue(rope=(self.cos.ptr, self.sin.ptr, T, D, dh, 2 * D))
         if self.qkv_frag:
@@ -534,7 +537,7 @@ class DeviceDiT:
         """Euler solve from x0 (1, 80, T) (already scaled by the temperature); returns the
         resident (80, T) result.  ``graph=True`` replays one captured HIP graph."""
         self.x.copy_from(np.asarray(x0, np.float32).reshape(self.mel, self._T))
-        self._row_planes()
+        self._row_buffers()
         if not graph:
             self._enqueue_solve()
             return self.x
@@ -550,7 +553,7 @@ class DeviceDiT:
         """One estimator evaluation at the s-th Euler time on the CFG pair built from x0 (1, 80, T);
         returns the (2, 80, T) velocity, i.e. ``DiT.forward`` (dit.py:144-180) without the update."""
         self.x.copy_from(np.asarray(x0, np.float32).reshape(self.mel, self._T))
-        self._row_planes()
+        self._row_buffers()
         self._time_and_mod()
         self._step(s, 0.0, update=False)
         return self.outT.numpy()
