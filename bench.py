@@ -52,9 +52,9 @@ HBM_PEAK = 8.0e12          # bytes/s, MI355X HBM3E
 # KV 512: 400.9 MB read + 9.2 MB written).  Counters cannot be read inside this process, so these
 # are the measured figures for exactly these kernels and shapes.
 TRAFFIC_DECODE_STEP = 410.1e6
-# the same passes over the 10 s solve's fused QKV GEMM on bfloat16 planes in fragment order
-# (k_gemm_x3f, [1000, 1024] x [3072, 1024]^T): 53.4 MB read + 12.3 MB written
-TRAFFIC_QKV_GEMM_X3 = 65.7e6
+# the same passes over the 10 s solve's fused QKV linear with both operands as bfloat16 planes in fragment
+# order (k_pg_lds, [1000, 1024] x [3072, 1024]^T): 68.8 MB read + 12.3 MB written
+TRAFFIC_QKV_PLANES = 81.1e6
 FP32_MFMA_PEAK = 157.3e12  # flop/s, MI355X dense fp32 matrix
 # float32 products on the bfloat16 matrix cores: six bfloat16 plane products each (cv3_linear_x3),
 # so the dense bfloat16 peak (2.5 PFLOP/s) over six
@@ -381,12 +381,16 @@ def bench_flow(args, tensors, meta):
     kflops = 2.0 * M * N * K
     log(f"flow: QKV GEMM {kms * 1e3:.1f} us/launch, {kflops / (kms / 1e3) / 1e12:.1f} TFLOP/s")
     planes = d.qkv[0].planes is not None if d.depth else False
-    name = ("plane linear (float32 GEMM as six bfloat16 plane products, both operands as planes in fragment order, "
-            "fused QKV 1000x3072x1024)" if planes
-            else "k_gemm<0> (fp32 MFMA GEMM, fused QKV 1000x3072x1024)")
+    if planes and d.qkv_frag:
+        t = [ctypes.c_int() for _ in range(5)]   # the tile the library picks for this shape
+        _lib.call("plane_linear_tile", _lib.KIND_F32, 1, M, K, N, *(ctypes.addressof(v) for v in t))
+        name = (f"k_pg_{'lds' if t[4].value else 'reg'} {32 * t[2].value}x{32 * t[3].value} (float32 linear as six "
+                "bfloat16 plane products, both operands as planes in fragment order, fused QKV 1000x3072x1024)")
+    else:
+        name = "k_gemm<0> (fp32 MFMA GEMM, fused QKV 1000x3072x1024)"
     return {"ms": ms, "flops": flops, "by_unit": by_unit, "T": T, "depth": d.depth,
             "kernel": {"name": name, "flops_per_launch": kflops, "peak": SPLIT_BF16_PEAK if planes else FP32_MFMA_PEAK,
-                       "traffic": TRAFFIC_QKV_GEMM_X3 if planes else None,
+                       "traffic": TRAFFIC_QKV_PLANES if planes and d.qkv_frag else None,
                        "us_per_launch": kms * 1e3, "achieved_flops": kflops / (kms / 1e3)}}
 
 
