@@ -133,8 +133,10 @@ int cv3_x3_rows_fit(const float* w, int64_t n, int64_t k, int64_t ldw, int* fit,
   if (!rc) {
     hipLaunchKernelGGL(k_rows_fit, dim3((unsigned)std::min<int64_t>(ceil_div(n, 4), 65536)), dim3(256), 0, st, w, n, k, ldw,
                        reinterpret_cast<int*>(flag));
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) rc = fail(CV3_EHIP, "kernel launch failed: %s", hipGetErrorString(e));
     int small = 0;
-    rc = cv3_copy_d2h(&small, flag, sizeof(int), reinterpret_cast<cv3_stream_t>(st));
+    if (!rc) rc = cv3_copy_d2h(&small, flag, sizeof(int), reinterpret_cast<cv3_stream_t>(st));
     *fit = !small;
   }
   const int rf = scratch_free(flag, st);
