@@ -359,9 +359,11 @@ int cv3_malloc(void** ptr, size_t bytes) {
       return CV3_OK;
     }
   }
+  // hipMalloc is refused to a thread that captures, and would spoil the capture and the stream with it
+  CV3_REQUIRE(!cap, CV3_EHIP, "no block of %zu bytes is cached, and none can be allocated in a capture", sz);
   void* p = nullptr;
   e = hipMalloc(&p, sz);
-  if (e != hipSuccess && !cap) {
+  if (e != hipSuccess) {
     // Out of memory: release the cache and try once more.
     cv3_empty_cache();
     (void)hipGetLastError();

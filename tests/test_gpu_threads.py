@@ -247,3 +247,22 @@ def test_block_dropped_during_another_streams_capture_belongs_to_its_graph(gpu):
     _lib.call("graph_destroy", x.value)
     assert in_use0 - _lib.mem_stats()[0] == nbytes
     del b
+
+
+def test_refused_allocation_leaves_the_capture_and_the_thread_whole(gpu):
+    """A capture takes memory from the cache only.  An allocation that finds none raises; the thread's stream goes on
+    afterwards, and captures again."""
+    from cv3amd import _lib
+    from cv3amd.device import DeviceArray, Graph, synchronize, to_device
+    a = to_device(np.arange(1024, dtype=np.float32))
+    synchronize()
+    _lib.call("empty_cache")
+    with pytest.raises(_lib.HIPError, match="capture"):
+        with Graph():
+            a.zero_()
+            DeviceArray((91 << 20,), np.uint8)
+    np.testing.assert_array_equal(a.numpy(), np.arange(1024))    # captured, not run
+    with Graph() as g:
+        a.zero_()
+    g.launch()
+    assert not a.numpy().any()
