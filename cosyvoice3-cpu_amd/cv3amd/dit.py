@@ -205,9 +205,10 @@ class DeviceLinear:
         (cv3_layer_norm_rexp); ``st``: a stream handle (None: the calling thread's)."""
         b = self.bias.ptr if self.bias is not None else None
         e = ctypes.byref(epi) if epi is not None else None
-        if self.q8 and self.q is None:
-            raise ValueError("this linear was kept for activations in planes (from_planes)")
-        if self.q8_digits:
+        if self.q8 and self.q is None:   # kept for activations in planes: the rows are split on the way
+            _lib.call("linear_rows_planes", _lib.KIND_Q8, x, m, self.k, ldx, self.codes16.ptr, self.scales_t.ptr,
+                      self.block, self.n, b, y, ldy, e, st)
+        elif self.q8_digits:
             if self.rexp is None or self.rexp.size < rexp_row0 + m:
                 raise ValueError("the digit-plane linear needs an int32 workspace of m entries (rexp)")
             _lib.call("linear_q8_digits", x, m, self.k, ldx, self.q.ptr, self.scales.ptr,

@@ -157,6 +157,16 @@ def test_linears_hold_the_layout_they_are_read_in(gpu, profile, layouts):
     d.halves = True
     np.testing.assert_array_equal(d.solve(x0).numpy(), want)
     assert max(map(len, (d.np, d.attp, d.ffp))) == 2
-    if profile == "balanced":
-        with pytest.raises(ValueError, match="planes"):
-            d.qkv[0](0, 1, d.dim, 0, 3 * d.dim)
+    for lin in (d.qkv[0], d.out[0]):    # float rows go through either layout
+        from cv3amd.device import empty, to_device
+        x = np.random.default_rng(5).standard_normal((37, lin.k), dtype=np.float32)
+        y, xd = empty((37, lin.n)), to_device(x)
+        if lin.q8_digits:
+            lin.rexp = empty((37,), np.int32)
+        lin(xd.ptr, 37, lin.k, y.ptr, lin.n)
+        name = "transformer_blocks.0.attn." + ("to_{}.weight" if lin is d.qkv[0] else "to_out.0.weight")
+        names = [name.format(p) for p in "qkv"] if lin is d.qkv[0] else [name]
+        full = [dev.get("flow.decoder.estimator." + n) for n in names]
+        w = np.concatenate([f.dequant() if hasattr(f, "dequant") else np.asarray(f) for f in full]).astype(np.float64)
+        b = np.concatenate([np.asarray(dev.get("flow.decoder.estimator." + n.replace("weight", "bias"))) for n in names])
+        assert rel_err(y.numpy(), x @ w.T + b) < 1e-5
