@@ -716,8 +716,8 @@ __global__ __launch_bounds__(512) void k_flash64x(AttnParams p, int nq) {
   }
   if constexpr (AGAIN) {
     // infinities and the largest floats have no planes here (inf - inf), values below 2^-110 not all their bits: the
-    // whole wave does those queries again, but for dims with a NaN among the values and queries with one, which are
-    // NaN as they stand
+    // whole wave does those queries again, but for dims with a NaN among the values and queries with one or with no
+    // key to see, which are NaN as they stand
     uint32_t bad = 0;   // bit 4 db + i
     if (__any(!in_range(most) || !in_range(least + 1u))) {
 #pragma unroll
@@ -742,7 +742,9 @@ __global__ __launch_bounds__(512) void k_flash64x(AttnParams p, int nq) {
       const int64_t row = q0 + __builtin_ctzll(todo);
       todo &= todo - 1;
       const float x = p.q[b * p.q_sb + hq * p.q_sh + row * p.q_sn + lane] * p.scale;
-      if (__any(x != x)) continue;
+      int64_t lo, hi;
+      visible_keys(p, row, lo, hi);
+      if (hi <= lo || __any(x != x)) continue;
       qs[lane] = x;
       __builtin_amdgcn_wave_barrier();
       attend_again(p, b, hq, hkv, row, lane, reinterpret_cast<const float4*>(qs));

@@ -58,10 +58,10 @@ struct PlaneParams {
   float *kc, *vc;
   int heads, kv_heads, cap, pos0;
   const float *cos, *sin;  // [cap][64]
-  // the float32 rows x was split from, or null (AGAIN kernels read them).  Outputs that come out not finite are formed again from these:
-  // an infinity times a plane of zero is NaN, and code products may pass the range before their scale.  So are
-  // those below 2^-90: rows below 2^-110 have fewer than 24 bits in their planes, which shows (2^-134 an element)
-  // only in outputs this small, unless an output's weights sum to more than 2^20.
+  // the float32 rows x was split from, or null (AGAIN kernels read them).  Outputs that come out not finite are
+  // formed again from these: an infinity times a plane of zero is NaN, and code products may pass the range before
+  // their scale.  So are those below 2^-90: rows below 2^-110 have fewer than 24 bits in their planes, which shows
+  // (2^-134 an element) only in outputs this small, unless an output's weights sum to more than 2^20.
   const float* fx;
   int64_t ldfx;
   int tiles_m, tiles_n, gm;
@@ -342,7 +342,7 @@ struct PlaneEpilogue {
       if constexpr (KIND == W_ROW)
         v[q] = make_float4(v[q].x * scale[q].x, v[q].y * scale[q].y, v[q].z * scale[q].z, v[q].w * scale[q].w);
     }
-    if constexpr (AGAIN) {  // a row's four outputs are small together: its rows' fault (a weight's such rows have no planes)
+    if constexpr (AGAIN) {  // a row too small makes its outputs small together (weights with such rows have no planes)
       bool fine = true;
 #pragma unroll
       for (int q = 0; q < G; ++q) fine &= in_range(v[q]);
